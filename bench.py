@@ -228,7 +228,7 @@ def layernorm_roofline(n: int, reps: int) -> dict:
     ms = event_time_ms(launch, reps, warm=reps)
     nbytes = 2.0 * n * n * 128 * 2
     gbs = nbytes / (ms * 1e-3) / 1e9
-    return {"kernel": "layer_norm_bf16_128", "bound": "hbm", "achieved": round(gbs, 1),
+    return {"kernel": "layer_norm_vec<bf16, 16, 1>", "bound": "hbm", "achieved": round(gbs, 1),
             "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": round(gbs / PEAK_HBM_GBS, 4),
             "us_per_launch": round(ms * 1e3, 2), "bytes_per_launch": nbytes}
 
