@@ -1,4 +1,5 @@
-"""ctypes binding of ``libfoldforge_amd.so`` (the C-ABI declared in ``include/foldforge_amd.h``).
+"""Bindings of ``libfoldforge_amd.so`` (the C-ABI declared in ``include/foldforge_amd.h``):
+:func:`calls`, the compiled ones that every op goes through, and :func:`lib`, ctypes.
 
 The library is loaded after ``torch`` so that it binds to the HIP runtime torch already
 loaded (both carry the soname ``libamdhip64.so.7``): device pointers and stream handles
@@ -9,8 +10,10 @@ unloadable library raises :class:`NativeUnavailable`.
 from __future__ import annotations
 
 import ctypes
+import importlib
 from ctypes import c_float, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
+from types import ModuleType
 
 LIBRARY = Path(__file__).resolve().with_name("libfoldforge_amd.so")
 
@@ -147,6 +150,25 @@ def lib() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = handle
     return _lib
+
+
+_calls: ModuleType | None = None
+
+
+def calls() -> ModuleType:
+    """The compiled calls of the library (``csrc/bindings.cpp``): the same entry points as
+    :func:`lib`, taking tensors (or None) for pointers; loaded on first use."""
+    global _calls
+    if _calls is None:
+        lib()  # torch's HIP runtime first, then this library
+        try:
+            _calls = importlib.import_module("foldforge_amd._bindings")
+        except ImportError as exc:
+            raise NativeUnavailable(
+                f"cannot load the compiled calls ({exc}); run `python -m foldforge_amd.build` "
+                "(the hip backend has no fallback)"
+            ) from exc
+    return _calls
 
 
 def check(status: int, what: str) -> None:

@@ -35,38 +35,50 @@ def _on_device(t: Tensor) -> bool:
     return t.device.type == DEVICE_TYPE
 
 
-def _ptr(t: Tensor | None) -> int | None:
-    return None if t is None else t.data_ptr()
-
-
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)  # torch.cuda.current_stream's handle
 
 
-def _need(cond: bool, message: str) -> None:
-    if not cond:
-        raise ValueError(message)
+def _refuse(message: str) -> None:
+    raise ValueError(message)
 
 
 def _param(t: Tensor, device: torch.device, name: str, shape: tuple[int, ...] | None = None) -> Tensor:
     """An fp32 parameter on ``device`` of exactly ``shape``: the C-ABI receives no sizes for
     parameters, so a wrong shape must stop here, not as an out-of-bounds device read."""
-    _need(isinstance(t, Tensor), f"{name} is missing")
-    _need(t.device == device, f"{name} is on {t.device}, expected {device}")
-    _need(t.dtype == torch.float32, f"{name} must be fp32 (got {t.dtype})")
+    if not isinstance(t, Tensor):
+        _refuse(f"{name} is missing")
+    if t.device != device:
+        _refuse(f"{name} is on {t.device}, expected {device}")
+    if t.dtype != torch.float32:
+        _refuse(f"{name} must be fp32 (got {t.dtype})")
     if shape is not None:
-        _need(tuple(t.shape) == tuple(shape), f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
+        if tuple(t.shape) != tuple(shape):
+            _refuse(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
     return t.contiguous()
+
+
+def _params(x: Tensor, spec: tuple[tuple[str, Tensor, tuple[int, ...]], ...]) -> tuple[Tensor, ...]:
+    """The parameters ``(name, tensor, shape)`` of a call on ``x``'s device, each checked as
+    :func:`_param` does (in one native pass where nothing is to be said about any of them)."""
+    names, tensors, shapes = zip(*spec)
+    if x.is_cuda and _native.calls().params_ok(x, tensors, shapes):
+        return tensors
+    return tuple(_param(t, x.device, nm, shape) for nm, t, shape in spec)
 
 
 def _output(out: Tensor | None, shape: tuple[int, ...], dtype: torch.dtype, device: torch.device) -> Tensor:
     """The caller's ``out=`` tensor (checked: it is written through a raw pointer) or a new one."""
     if out is None:
         return torch.empty(shape, dtype=dtype, device=device)
-    _need(tuple(out.shape) == tuple(shape), f"out has shape {tuple(out.shape)}, expected {tuple(shape)}")
-    _need(out.dtype == dtype, f"out must be {dtype} (got {out.dtype})")
-    _need(out.device == device, f"out is on {out.device}, expected {device}")
-    _need(out.is_contiguous(), "out must be contiguous")
+    if tuple(out.shape) != tuple(shape):
+        _refuse(f"out has shape {tuple(out.shape)}, expected {tuple(shape)}")
+    if out.dtype != dtype:
+        _refuse(f"out must be {dtype} (got {out.dtype})")
+    if out.device != device:
+        _refuse(f"out is on {out.device}, expected {device}")
+    if not out.is_contiguous():
+        _refuse("out must be contiguous")
     return out
 
 
@@ -93,31 +105,42 @@ def triangle_attention_supported(d_pair: int, n_head: int, d_head: int, transpos
 
 
 def _pair(z: Tensor, mask: Tensor, width: int | None = PAIR_WIDTH) -> tuple[int, int]:
-    _need(_on_device(z), "z must be a device tensor")
-    _need(z.dtype == torch.bfloat16, f"z must be bf16 (got {z.dtype})")
-    _need(z.dim() == 4 and z.shape[1] == z.shape[2], f"z must be [B, N, N, c] (got {tuple(z.shape)})")
+    if not _on_device(z):
+        _refuse("z must be a device tensor")
+    if z.dtype != torch.bfloat16:
+        _refuse(f"z must be bf16 (got {z.dtype})")
+    if not (z.dim() == 4 and z.shape[1] == z.shape[2]):
+        _refuse(f"z must be [B, N, N, c] (got {tuple(z.shape)})")
     if width is not None:
-        _need(z.shape[3] == width, f"pair width {z.shape[3]} (the kernels take {width})")
-    _need(z.is_contiguous(), "z must be contiguous")
-    _need(mask.dtype == torch.bool and mask.shape == z.shape[:2], "mask must be bool [B, N]")
-    _need(mask.device == z.device and mask.is_contiguous(), "mask must be a contiguous device tensor")
+        if z.shape[3] != width:
+            _refuse(f"pair width {z.shape[3]} (the kernels take {width})")
+    if not z.is_contiguous():
+        _refuse("z must be contiguous")
+    if not (mask.dtype == torch.bool and mask.shape == z.shape[:2]):
+        _refuse("mask must be bool [B, N]")
+    if not (mask.device == z.device and mask.is_contiguous()):
+        _refuse("mask must be a contiguous device tensor")
     return z.shape[0], z.shape[1]
 
 
 def layer_norm(x: Tensor, weight: Tensor | None, bias: Tensor | None, eps: float = 1e-5) -> Tensor:
     """LayerNorm over the last axis (fp32 statistics and affine), returned in ``x.dtype``."""
-    _need(_on_device(x) and x.is_contiguous(), "x must be a contiguous device tensor")
-    _need(x.dtype in (torch.bfloat16, torch.float32), f"x must be bf16 or fp32 (got {x.dtype})")
+    if not (_on_device(x) and x.is_contiguous()):
+        _refuse("x must be a contiguous device tensor")
+    if x.dtype not in (torch.bfloat16, torch.float32):
+        _refuse(f"x must be bf16 or fp32 (got {x.dtype})")
     cols = x.shape[-1]
-    for t, name in ((weight, "weight"), (bias, "bias")):
-        if t is not None:
-            _need(t.numel() == cols, f"{name} has {t.numel()} entries for {cols} channels")
-    weight = None if weight is None else _param(weight, x.device, "weight", (cols,))
-    bias = None if bias is None else _param(bias, x.device, "bias", (cols,))
+    if weight is None or bias is None or not (
+            x.is_cuda and _native.calls().params_ok(x, (weight, bias), ((cols,), (cols,)))):
+        for t, name in ((weight, "weight"), (bias, "bias")):
+            if t is not None and t.numel() != cols:
+                _refuse(f"{name} has {t.numel()} entries for {cols} channels")
+        weight = None if weight is None else _param(weight, x.device, "weight", (cols,))
+        bias = None if bias is None else _param(bias, x.device, "bias", (cols,))
     y = torch.empty_like(x)
     dtype = 0 if x.dtype == torch.bfloat16 else 1
-    status = _native.lib().ffk_layer_norm(
-        x.data_ptr(), _ptr(weight), _ptr(bias), y.data_ptr(), x.numel() // cols, cols,
+    status = _native.calls().ffk_layer_norm(
+        x, weight, bias, y, x.numel() // cols, cols,
         float(eps), dtype, _stream(x.device),
     )
     _native.check(status, "layer_norm")
@@ -136,23 +159,28 @@ def layer_norm_linear(x: Tensor, ln_weight: Tensor | None, ln_bias: Tensor | Non
     ``layer_norm_linear``): fp32 statistics, ``weight [d_out, d_in]`` fp32, ``bias [d_out]``,
     output ``[..., d_out]`` in ``out_dtype`` (bf16 or fp32). d_in a multiple of 64 up to 768,
     d_out a multiple of 32."""
-    _need(_on_device(x) and x.is_contiguous(), "x must be a contiguous device tensor")
-    _need(x.dtype == torch.bfloat16, f"x must be bf16 (got {x.dtype})")
-    _need(activation in ACTIVATIONS, f"activation must be one of {sorted(ACTIVATIONS)}")
-    _need(out_dtype in (torch.bfloat16, torch.float32), f"out_dtype must be bf16 or fp32 (got {out_dtype})")
+    if not (_on_device(x) and x.is_contiguous()):
+        _refuse("x must be a contiguous device tensor")
+    if x.dtype != torch.bfloat16:
+        _refuse(f"x must be bf16 (got {x.dtype})")
+    if activation not in ACTIVATIONS:
+        _refuse(f"activation must be one of {sorted(ACTIVATIONS)}")
+    if out_dtype not in (torch.bfloat16, torch.float32):
+        _refuse(f"out_dtype must be bf16 or fp32 (got {out_dtype})")
     d_in = x.shape[-1]
-    _need(weight.dim() == 2, f"weight must be [d_out, d_in] (got {tuple(weight.shape)})")
+    if weight.dim() != 2:
+        _refuse(f"weight must be [d_out, d_in] (got {tuple(weight.shape)})")
     d_out = weight.shape[0]
-    _need(d_in % 64 == 0 and 0 < d_in <= 768 and d_out % 32 == 0 and d_out > 0,
-          f"d_in={d_in} d_out={d_out} (the kernel takes d_in a multiple of 64 up to 768, d_out a multiple of 32)")
+    if not (d_in % 64 == 0 and 0 < d_in <= 768 and d_out % 32 == 0 and d_out > 0):
+        _refuse(f"d_in={d_in} d_out={d_out} (the kernel takes d_in a multiple of 64 up to 768, d_out a multiple of 32)")
     dev = x.device
     w = _param(weight, dev, "weight", (d_out, d_in))
     lw = None if ln_weight is None else _param(ln_weight, dev, "ln_weight", (d_in,))
     lb = None if ln_bias is None else _param(ln_bias, dev, "ln_bias", (d_in,))
     b = None if bias is None else _param(bias, dev, "bias", (d_out,))
     out = _output(out, (*x.shape[:-1], d_out), out_dtype, dev)
-    status = _native.lib().ffk_layer_norm_linear(
-        x.data_ptr(), _ptr(lw), _ptr(lb), w.data_ptr(), _ptr(b), out.data_ptr(), x.numel() // d_in,
+    status = _native.calls().ffk_layer_norm_linear(
+        x, lw, lb, w, b, out, x.numel() // d_in,
         d_in, d_out, ACTIVATIONS[activation], 0 if out_dtype == torch.bfloat16 else 1, float(eps),
         _stream(dev))
     _native.check(status, "layer_norm_linear")
@@ -164,25 +192,28 @@ def swiglu_ffn(x: Tensor, w_a: Tensor, w_b: Tensor, w_out: Tensor, residual: Ten
     """``(silu(x W_a^T) * (x W_b^T)) W_out^T`` (+ ``residual``) over the last axis of
     ``x [..., d]`` bf16 (the engine's ``swiglu_ffn``): ``w_a, w_b [hidden, d]``,
     ``w_out [d, hidden]`` fp32; d a multiple of 64 up to 768, hidden a multiple of 64."""
-    _need(_on_device(x) and x.is_contiguous(), "x must be a contiguous device tensor")
-    _need(x.dtype == torch.bfloat16, f"x must be bf16 (got {x.dtype})")
+    if not (_on_device(x) and x.is_contiguous()):
+        _refuse("x must be a contiguous device tensor")
+    if x.dtype != torch.bfloat16:
+        _refuse(f"x must be bf16 (got {x.dtype})")
     d = x.shape[-1]
     hidden = w_a.shape[0]
-    _need(d % 64 == 0 and 0 < d <= 768 and hidden % 64 == 0 and hidden > 0,
-          f"d={d} hidden={hidden} (the kernel takes d a multiple of 64 up to 768, hidden a multiple of 64)")
+    if not (d % 64 == 0 and 0 < d <= 768 and hidden % 64 == 0 and hidden > 0):
+        _refuse(f"d={d} hidden={hidden} (the kernel takes d a multiple of 64 up to 768, hidden a multiple of 64)")
     dev = x.device
     wa = _param(w_a, dev, "w_a", (hidden, d))
     wb = _param(w_b, dev, "w_b", (hidden, d))
     wo = _param(w_out, dev, "w_out", (d, hidden))
     if residual is not None:
-        _need(residual.dtype == torch.bfloat16 and residual.shape == x.shape and residual.device == dev
-              and residual.is_contiguous(), "residual must be a contiguous bf16 tensor shaped like x")
+        if not (residual.dtype == torch.bfloat16 and residual.shape == x.shape and residual.device == dev
+                and residual.is_contiguous()):
+            _refuse("residual must be a contiguous bf16 tensor shaped like x")
     out = _output(out, tuple(x.shape), torch.bfloat16, dev)
     rows = x.numel() // d
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_swiglu_ffn_workspace(rows, hidden), dev)
-    status = lib.ffk_swiglu_ffn(x.data_ptr(), wa.data_ptr(), wb.data_ptr(), wo.data_ptr(), _ptr(residual),
-                                out.data_ptr(), ws.data_ptr(), ws.numel(), rows, d, hidden, _stream(dev))
+    status = lib.ffk_swiglu_ffn(x, wa, wb, wo, residual,
+                                out, ws, ws.numel(), rows, d, hidden, _stream(dev))
     _native.check(status, "swiglu_ffn")
     return out
 
@@ -216,20 +247,21 @@ def triangle_multiplicative_update(
     c = z.shape[3]
     dev = z.device
     hidden = to_left.shape[0]
-    _need(trimul_supported(c, hidden), f"d_pair={c} d_hidden={hidden} (the kernels take 128 / 128, "
-          "or a pair width a multiple of 64 up to 256 with a hidden width a multiple of 64 up to 768)")
+    if not trimul_supported(c, hidden):
+        _refuse(f"d_pair={c} d_hidden={hidden} (the kernels take 128 / 128, "
+                    "or a pair width a multiple of 64 up to 256 with a hidden width a multiple of 64 up to 768)")
     spec = (("ln_pair_weight", ln_pair_weight, (c,)), ("ln_pair_bias", ln_pair_bias, (c,)),
             ("to_left", to_left, (hidden, c)), ("to_right", to_right, (hidden, c)),
             ("to_left_gate", to_left_gate, (hidden, c)), ("to_right_gate", to_right_gate, (hidden, c)),
             ("ln_out_weight", ln_out_weight, (hidden,)), ("ln_out_bias", ln_out_bias, (hidden,)),
             ("to_out", to_out, (c, hidden)), ("to_gate", to_gate, (c, c)))
-    ps = [_param(t, dev, nm, shape) for nm, t, shape in spec]
+    ps = _params(z, spec)
     out = _output(out, tuple(z.shape), torch.bfloat16, dev)
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_triangle_multiplication_workspace(batch, n, c, hidden), dev)
     status = lib.ffk_triangle_multiplication(
-        z.data_ptr(), mask.data_ptr(), *(p.data_ptr() for p in ps), out.data_ptr(),
-        ws.data_ptr(), ws.numel(), batch, n, c, hidden, int(outgoing), int(residual),
+        z, mask, *ps, out,
+        ws, ws.numel(), batch, n, c, hidden, int(outgoing), int(residual),
         int(length_divided), float(eps), _stream(dev),
     )
     _native.check(status, "triangle_multiplicative_update")
@@ -269,13 +301,15 @@ def triangle_attention(
     c = z.shape[3]
     dev = z.device
     hd = to_query.shape[0]
-    _need(n_head > 0 and hd % n_head == 0, f"hidden {hd} is not a multiple of {n_head} heads")
-    _need(out_t_bias is None or to_out_t is not None, "out_t_bias needs to_out_t")
+    if not (n_head > 0 and hd % n_head == 0):
+        _refuse(f"hidden {hd} is not a multiple of {n_head} heads")
+    if not (out_t_bias is None or to_out_t is not None):
+        _refuse("out_t_bias needs to_out_t")
     spec = (("ln_pair_weight", ln_pair_weight, (c,)), ("ln_pair_bias", ln_pair_bias, (c,)),
             ("to_bias", to_bias, (n_head, c)), ("to_query", to_query, (hd, c)),
             ("to_key", to_key, (hd, c)), ("to_value", to_value, (hd, c)),
             ("to_gate", to_gate, (hd, c)), ("to_out", to_out, (c, hd)))
-    ps = [_param(t, dev, nm, shape) for nm, t, shape in spec]
+    ps = _params(z, spec)
     extra = (("gate_bias", gate_bias, (hd,)), ("out_bias", out_bias, (c,)),
              ("to_out_t", to_out_t, (c, hd)), ("out_t_bias", out_t_bias, (c,)))
     opt = [None if t is None else _param(t, dev, nm, shape) for nm, t, shape in extra]
@@ -283,17 +317,18 @@ def triangle_attention(
     # workspace the staging buffer of form 1
     form = 2 if to_out_t is not None else 1 if untransposed_output and not starting else 0
     d = hd // n_head
-    _need(triangle_attention_supported(c, n_head, d, transposed_bias),
-          f"d_pair={c} heads={n_head} x {d} (the kernels take 128 with 4 x 32, or pair 64 / 128 / "
-          "256 with at most 32 heads of 8 to 64 channels, heads x d_head a multiple of 64)")
+    if not triangle_attention_supported(c, n_head, d, transposed_bias):
+        _refuse(f"d_pair={c} heads={n_head} x {d} (the kernels take 128 with 4 x 32, or pair 64 / 128 / "
+                    "256 with at most 32 heads of 8 to 64 channels, heads x d_head a multiple of 64)")
     if (c, n_head, d) != (128, 4, 32):
-        _need(batch * n <= 65535, f"batch x n = {batch * n} exceeds the launch grid")
+        if batch * n > 65535:
+            _refuse(f"batch x n = {batch * n} exceeds the launch grid")
     out = _output(out, tuple(z.shape), torch.bfloat16, dev)
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_triangle_attention_workspace(batch, n, c, n_head, d, form), dev)
     status = lib.ffk_triangle_attention(
-        z.data_ptr(), mask.data_ptr(), *(p.data_ptr() for p in ps), *(_ptr(t) for t in opt),
-        out.data_ptr(), ws.data_ptr(), ws.numel(), batch, n, c, n_head, d, int(starting),
+        z, mask, *ps, *opt,
+        out, ws, ws.numel(), batch, n, c, n_head, d, int(starting),
         int(transposed_bias), form, int(residual), float(eps), _stream(dev),
     )
     _native.check(status, "triangle_attention")
@@ -314,25 +349,28 @@ def transition(
 ) -> Tensor:
     """SwiGLU transition of ``x [..., d]`` bf16: one fused kernel at d = 128 x 4, token-row
     GEMMs (LayerNorm, expand with SwiGLU epilogue, squeeze + residual) at other widths."""
-    _need(_on_device(x) and x.is_contiguous(), "x must be a contiguous device tensor")
-    _need(x.dtype == torch.bfloat16, f"x must be bf16 (got {x.dtype})")
+    if not (_on_device(x) and x.is_contiguous()):
+        _refuse("x must be a contiguous device tensor")
+    if x.dtype != torch.bfloat16:
+        _refuse(f"x must be bf16 (got {x.dtype})")
     d = x.shape[-1]
     factor = expand_a.shape[0] // d
-    _need(transition_supported(d, factor),
-          f"width {d} x {factor} (the kernels take 128 x 4, or d and factor * d multiples of 64)")
-    _need(expand_a.shape == (factor * d, d) and expand_b.shape == (factor * d, d)
-          and squeeze.shape == (d, factor * d), "expand_a/expand_b [f d, d], squeeze [d, f d]")
+    if not transition_supported(d, factor):
+        _refuse(f"width {d} x {factor} (the kernels take 128 x 4, or d and factor * d multiples of 64)")
+    if not (expand_a.shape == (factor * d, d) and expand_b.shape == (factor * d, d)
+            and squeeze.shape == (d, factor * d)):
+        _refuse("expand_a/expand_b [f d, d], squeeze [d, f d]")
     dev = x.device
     spec = (("ln_weight", ln_weight, (d,)), ("ln_bias", ln_bias, (d,)),
             ("expand_a", expand_a, (factor * d, d)), ("expand_b", expand_b, (factor * d, d)),
             ("squeeze", squeeze, (d, factor * d)))
-    ps = [_param(t, dev, nm, shape) for nm, t, shape in spec]
+    ps = _params(x, spec)
     rows = x.numel() // d
     out = _output(out, tuple(x.shape), torch.bfloat16, dev)
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_transition_workspace(rows, d, factor), dev)
     status = lib.ffk_transition(
-        x.data_ptr(), *(p.data_ptr() for p in ps), out.data_ptr(), ws.data_ptr(), ws.numel(),
+        x, *ps, out, ws, ws.numel(),
         rows, d, factor, int(residual), float(eps), _stream(dev),
     )
     _native.check(status, "transition")
@@ -381,13 +419,13 @@ def triangle_attention_transition(
             ("ln_weight", ln_weight, (c,)), ("ln_bias", ln_bias, (c,)),
             ("expand_a", expand_a, (4 * c, c)), ("expand_b", expand_b, (4 * c, c)),
             ("squeeze", squeeze, (c, 4 * c)))
-    ps = [_param(t, dev, nm, shape) for nm, t, shape in spec]
+    ps = _params(z, spec)
     out = _output(out, tuple(z.shape), torch.bfloat16, dev)
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_triangle_attention_transition_workspace(batch, n), dev)
     status = lib.ffk_triangle_attention_transition(
-        z.data_ptr(), mask.data_ptr(), *(p.data_ptr() for p in ps), out.data_ptr(),
-        ws.data_ptr(), ws.numel(), batch, n, int(starting), int(transposed_bias),
+        z, mask, *ps, out,
+        ws, ws.numel(), batch, n, int(starting), int(transposed_bias),
         float(eps_pair), float(eps), _stream(dev),
     )
     _native.check(status, "triangle_attention_transition")
@@ -436,25 +474,27 @@ def attention_pair_bias(
     ``extra_bias`` (fp32 or bf16, broadcastable to ``[B, H, N, N]``, e.g. an ``[N, N]`` or
     an expanded view) joins every logit; broadcast axes are passed as zero strides."""
     batch, n = _pair(z, mask)
-    _need(_on_device(s) and s.is_contiguous() and s.dtype == torch.bfloat16,
-          "s must be a contiguous bf16 device tensor")
-    _need(s.dim() == 3 and s.shape[:2] == z.shape[:2], f"s {tuple(s.shape)} does not match z")
+    if not (_on_device(s) and s.is_contiguous() and s.dtype == torch.bfloat16):
+        _refuse("s must be a contiguous bf16 device tensor")
+    if not (s.dim() == 3 and s.shape[:2] == z.shape[:2]):
+        _refuse(f"s {tuple(s.shape)} does not match z")
     cs = s.shape[-1]
-    _need(single_attention_heads_supported(cs, n_head),
-          f"single width {cs} with {n_head} heads (the kernels take a multiple of 64 split "
-          "into at most 32 heads of 8, 16, 24 or 32)")
+    if not single_attention_heads_supported(cs, n_head):
+        _refuse(f"single width {cs} with {n_head} heads (the kernels take a multiple of 64 split "
+                    "into at most 32 heads of 8, 16, 24 or 32)")
     dev = s.device
     spec = (("ln_single_weight", ln_single_weight, (cs,)), ("ln_single_bias", ln_single_bias, (cs,)),
             ("to_query", to_query, (cs, cs)), ("query_bias", query_bias, (cs,)),
             ("to_key", to_key, (cs, cs)), ("to_value", to_value, (cs, cs)),
             ("ln_pair_weight", ln_pair_weight, (PAIR_WIDTH,)), ("to_bias", to_bias, (n_head, PAIR_WIDTH)),
             ("to_gate", to_gate, (cs, cs)), ("to_out", to_out, (cs, cs)))
-    ps = [_param(t, dev, nm, shape) for nm, t, shape in spec]
+    ps = _params(s, spec)
     extra, strides, extra_bf16 = None, (0, 0, 0), 0
     if extra_bias is not None:
-        _need(extra_bias.dtype in (torch.float32, torch.bfloat16),
-              f"extra_bias must be fp32 or bf16 (got {extra_bias.dtype})")
-        _need(extra_bias.device == dev, "extra_bias must be on the device of s")
+        if extra_bias.dtype not in (torch.float32, torch.bfloat16):
+            _refuse(f"extra_bias must be fp32 or bf16 (got {extra_bias.dtype})")
+        if extra_bias.device != dev:
+            _refuse("extra_bias must be on the device of s")
         try:
             extra = extra_bias.expand(batch, n_head, n, n)
         except RuntimeError:
@@ -464,11 +504,11 @@ def attention_pair_bias(
             extra = extra.contiguous()
         strides, extra_bf16 = extra.stride()[:3], int(extra.dtype == torch.bfloat16)
     out = _output(out, tuple(s.shape), torch.bfloat16, dev)
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_attention_pair_bias_workspace(batch, n, cs, PAIR_WIDTH, n_head), dev)
     status = lib.ffk_attention_pair_bias(
-        s.data_ptr(), z.data_ptr(), mask.data_ptr(), *(p.data_ptr() for p in ps), _ptr(extra),
-        extra_bf16, *strides, out.data_ptr(), ws.data_ptr(), ws.numel(), batch, n, cs,
+        s, z, mask, *ps, extra,
+        extra_bf16, *strides, out, ws, ws.numel(), batch, n, cs,
         PAIR_WIDTH, n_head, float(gate_bias), int(residual), float(eps_single), float(eps_pair),
         _stream(dev),
     )
@@ -503,29 +543,30 @@ def msa_pair_weighted_averaging(
     """MSA pair-weighted averaging of ``m [B, S, N, c_m]`` bf16 with the weights
     ``softmax_j(LN_pair(z) . to_bias)`` from ``z [B, N, N, 128]`` bf16, under the key mask."""
     batch, n = _pair(z, mask)
-    _need(_on_device(m) and m.is_contiguous() and m.dtype == torch.bfloat16,
-          "m must be a contiguous bf16 device tensor")
-    _need(m.dim() == 4 and m.shape[0] == batch and m.shape[2] == n,
-          f"m {tuple(m.shape)} does not match z {tuple(z.shape)}")
+    if not (_on_device(m) and m.is_contiguous() and m.dtype == torch.bfloat16):
+        _refuse("m must be a contiguous bf16 device tensor")
+    if not (m.dim() == 4 and m.shape[0] == batch and m.shape[2] == n):
+        _refuse(f"m {tuple(m.shape)} does not match z {tuple(z.shape)}")
     depth, cm = m.shape[1], m.shape[3]
     hd = to_value.shape[0]
-    _need(hd % n_head == 0, f"hidden {hd} is not a multiple of {n_head} heads")
+    if hd % n_head != 0:
+        _refuse(f"hidden {hd} is not a multiple of {n_head} heads")
     dh = hd // n_head
-    _need(msa_pair_weighted_averaging_supported(cm, n_head, dh),
-          f"d_msa={cm} heads={n_head} x {dh} (the kernels take d_msa a multiple of 64 up to 768, "
-          "at most 32 heads of a multiple of 4, heads x d_head a multiple of 64)")
+    if not msa_pair_weighted_averaging_supported(cm, n_head, dh):
+        _refuse(f"d_msa={cm} heads={n_head} x {dh} (the kernels take d_msa a multiple of 64 up to 768, "
+                    "at most 32 heads of a multiple of 4, heads x d_head a multiple of 64)")
     dev = m.device
     spec = (("ln_msa_weight", ln_msa_weight, (cm,)), ("ln_msa_bias", ln_msa_bias, (cm,)),
             ("ln_pair_weight", ln_pair_weight, (PAIR_WIDTH,)), ("to_bias", to_bias, (n_head, PAIR_WIDTH)),
             ("to_value", to_value, (hd, cm)), ("to_gate", to_gate, (hd, cm)), ("to_out", to_out, (cm, hd)))
-    ps = [_param(t, dev, nm, shape) for nm, t, shape in spec]
+    ps = _params(m, spec)
     out = _output(out, tuple(m.shape), torch.bfloat16, dev)
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_msa_pair_weighted_averaging_workspace(batch, depth, n, cm, PAIR_WIDTH,
                                                                   n_head, dh), dev)
     status = lib.ffk_msa_pair_weighted_averaging(
-        m.data_ptr(), z.data_ptr(), mask.data_ptr(), *(p.data_ptr() for p in ps), out.data_ptr(),
-        ws.data_ptr(), ws.numel(), batch, depth, n, cm, PAIR_WIDTH, n_head, dh, int(residual),
+        m, z, mask, *ps, out,
+        ws, ws.numel(), batch, depth, n, cm, PAIR_WIDTH, n_head, dh, int(residual),
         float(eps_msa), float(eps_pair), _stream(dev),
     )
     _native.check(status, "msa_pair_weighted_averaging")
@@ -558,38 +599,40 @@ def outer_product_mean(
     """Outer product mean of ``m [B, S, N, c_m]`` bf16 under the MSA row mask
     ``rows_mask [B, S, N]`` bool -> ``[B, N, N, 128]`` bf16 (plus ``residual`` when given).
     ``count_offset`` None divides by ``max(n, 1)``, a number by ``n + count_offset``."""
-    _need(_on_device(m) and m.is_contiguous() and m.dtype == torch.bfloat16,
-          "m must be a contiguous bf16 device tensor")
-    _need(m.dim() == 4, f"m must be [B, S, N, c_m] (got {tuple(m.shape)})")
+    if not (_on_device(m) and m.is_contiguous() and m.dtype == torch.bfloat16):
+        _refuse("m must be a contiguous bf16 device tensor")
+    if m.dim() != 4:
+        _refuse(f"m must be [B, S, N, c_m] (got {tuple(m.shape)})")
     batch, depth, n, cm = m.shape
-    _need(rows_mask.dtype == torch.bool and tuple(rows_mask.shape) == (batch, depth, n)
-          and rows_mask.device == m.device and rows_mask.is_contiguous(),
-          "rows_mask must be a contiguous bool device tensor [B, S, N]")
+    if not (rows_mask.dtype == torch.bool and tuple(rows_mask.shape) == (batch, depth, n)
+            and rows_mask.device == m.device and rows_mask.is_contiguous()):
+        _refuse("rows_mask must be a contiguous bool device tensor [B, S, N]")
     hidden = to_left.shape[0]
     cz = to_out.shape[0]
-    _need(outer_product_mean_supported(cm, hidden, cz),
-          f"d_msa={cm} d_hidden={hidden} d_pair={cz} (the kernels take d_msa a multiple of 64 "
-          "up to 768, d_hidden 32, d_pair 128)")
-    _need(depth > 0 and n > 0 and batch > 0, "empty MSA")
+    if not outer_product_mean_supported(cm, hidden, cz):
+        _refuse(f"d_msa={cm} d_hidden={hidden} d_pair={cz} (the kernels take d_msa a multiple of 64 "
+                    "up to 768, d_hidden 32, d_pair 128)")
+    if not (depth > 0 and n > 0 and batch > 0):
+        _refuse("empty MSA")
     dev = m.device
     spec = (("ln_weight", ln_weight, (cm,)), ("ln_bias", ln_bias, (cm,)),
             ("to_left", to_left, (hidden, cm)), ("to_right", to_right, (hidden, cm)),
             ("to_out", to_out, (cz, hidden * hidden)), ("to_out_bias", to_out_bias, (cz,)))
-    ln_w, ln_b, wl, wr, wo, bo = (_param(t, dev, nm, shape) for nm, t, shape in spec)
+    ln_w, ln_b, wl, wr, wo, bo = _params(m, spec)
     bl = None if left_bias is None else _param(left_bias, dev, "left_bias", (hidden,))
     br = None if right_bias is None else _param(right_bias, dev, "right_bias", (hidden,))
     if residual is not None:
-        _need(residual.dtype == torch.bfloat16 and residual.is_contiguous()
-              and tuple(residual.shape) == (batch, n, n, cz) and residual.device == dev,
-              "residual must be a contiguous bf16 [B, N, N, 128] device tensor")
+        if not (residual.dtype == torch.bfloat16 and residual.is_contiguous()
+                and tuple(residual.shape) == (batch, n, n, cz) and residual.device == dev):
+            _refuse("residual must be a contiguous bf16 [B, N, N, 128] device tensor")
     out = _output(out, (batch, n, n, cz), torch.bfloat16, dev)
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_outer_product_mean_workspace(batch, depth, n, cm, hidden, cz), dev)
     status = lib.ffk_outer_product_mean(
-        m.data_ptr(), rows_mask.data_ptr(), ln_w.data_ptr(), ln_b.data_ptr(), wl.data_ptr(),
-        None if bl is None else bl.data_ptr(), wr.data_ptr(), None if br is None else br.data_ptr(),
-        wo.data_ptr(), bo.data_ptr(), None if residual is None else residual.data_ptr(),
-        out.data_ptr(), ws.data_ptr(), ws.numel(), batch, depth, n, cm, hidden, cz, float(eps),
+        m, rows_mask, ln_w, ln_b, wl,
+        bl, wr, br,
+        wo, bo, residual,
+        out, ws, ws.numel(), batch, depth, n, cm, hidden, cz, float(eps),
         -1.0 if count_offset is None else float(count_offset), int(normalize_before_proj),
         _stream(dev),
     )
@@ -626,42 +669,45 @@ def outer_product_mean_grouped(
     [B, S, N]`` bool -> ``[B, N, N, c_z]`` bf16: products within each of ``groups`` channel
     groups, summed over the MSA rows, the product norm (``norm_weight`` / ``norm_bias``, eps
     ``norm_eps``), then ``to_out`` (plus ``residual`` when given)."""
-    _need(_on_device(m) and m.is_contiguous() and m.dtype == torch.bfloat16,
-          "m must be a contiguous bf16 device tensor")
-    _need(m.dim() == 4, f"m must be [B, S, N, c_m] (got {tuple(m.shape)})")
+    if not (_on_device(m) and m.is_contiguous() and m.dtype == torch.bfloat16):
+        _refuse("m must be a contiguous bf16 device tensor")
+    if m.dim() != 4:
+        _refuse(f"m must be [B, S, N, c_m] (got {tuple(m.shape)})")
     batch, depth, n, cm = m.shape
-    _need(rows_mask.dtype == torch.bool and tuple(rows_mask.shape) == (batch, depth, n)
-          and rows_mask.device == m.device and rows_mask.is_contiguous(),
-          "rows_mask must be a contiguous bool device tensor [B, S, N]")
+    if not (rows_mask.dtype == torch.bool and tuple(rows_mask.shape) == (batch, depth, n)
+            and rows_mask.device == m.device and rows_mask.is_contiguous()):
+        _refuse("rows_mask must be a contiguous bool device tensor [B, S, N]")
     hidden = to_left.shape[0]
     cz = to_out.shape[0]
-    _need(hidden % groups == 0, f"d_hidden={hidden} is not a multiple of groups={groups}")
+    if hidden % groups != 0:
+        _refuse(f"d_hidden={hidden} is not a multiple of groups={groups}")
     dg = hidden // groups
-    _need(outer_product_mean_grouped_supported(cm, groups, dg, cz),
-          f"d_msa={cm} {groups} groups of {dg} d_pair={cz} (the kernels take d_msa a multiple of "
-          "64 up to 768, 8 groups of 8, d_pair 128 or 256)")
-    _need(depth > 0 and n > 0 and batch > 0, "empty MSA")
+    if not outer_product_mean_grouped_supported(cm, groups, dg, cz):
+        _refuse(f"d_msa={cm} {groups} groups of {dg} d_pair={cz} (the kernels take d_msa a multiple of "
+                    "64 up to 768, 8 groups of 8, d_pair 128 or 256)")
+    if not (depth > 0 and n > 0 and batch > 0):
+        _refuse("empty MSA")
     dev = m.device
     k2 = groups * dg * dg
     spec = (("ln_weight", ln_weight, (cm,)), ("ln_bias", ln_bias, (cm,)),
             ("to_left", to_left, (hidden, cm)), ("to_right", to_right, (hidden, cm)),
             ("norm_weight", norm_weight, (k2,)), ("norm_bias", norm_bias, (k2,)),
             ("to_out", to_out, (cz, k2)), ("to_out_bias", to_out_bias, (cz,)))
-    ln_w, ln_b, wl, wr, nw, nb, wo, bo = (_param(t, dev, nm, shape) for nm, t, shape in spec)
+    ln_w, ln_b, wl, wr, nw, nb, wo, bo = _params(m, spec)
     bl = None if left_bias is None else _param(left_bias, dev, "left_bias", (hidden,))
     br = None if right_bias is None else _param(right_bias, dev, "right_bias", (hidden,))
     if residual is not None:
-        _need(residual.dtype == torch.bfloat16 and residual.is_contiguous()
-              and tuple(residual.shape) == (batch, n, n, cz) and residual.device == dev,
-              f"residual must be a contiguous bf16 [B, N, N, {cz}] device tensor")
+        if not (residual.dtype == torch.bfloat16 and residual.is_contiguous()
+                and tuple(residual.shape) == (batch, n, n, cz) and residual.device == dev):
+            _refuse(f"residual must be a contiguous bf16 [B, N, N, {cz}] device tensor")
     out = _output(out, (batch, n, n, cz), torch.bfloat16, dev)
-    lib = _native.lib()
+    lib = _native.calls()
     ws = _workspace(lib.ffk_outer_product_mean_grouped_workspace(batch, depth, n, cm, groups, dg, cz), dev)
     status = lib.ffk_outer_product_mean_grouped(
-        m.data_ptr(), rows_mask.data_ptr(), ln_w.data_ptr(), ln_b.data_ptr(), wl.data_ptr(),
-        None if bl is None else bl.data_ptr(), wr.data_ptr(), None if br is None else br.data_ptr(),
-        nw.data_ptr(), nb.data_ptr(), wo.data_ptr(), bo.data_ptr(),
-        None if residual is None else residual.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(),
+        m, rows_mask, ln_w, ln_b, wl,
+        bl, wr, br,
+        nw, nb, wo, bo,
+        residual, out, ws, ws.numel(),
         batch, depth, n, cm, groups, dg, cz, float(eps), float(norm_eps), _stream(dev),
     )
     _native.check(status, "outer_product_mean_grouped")
@@ -673,7 +719,8 @@ def blocked_bias(bias: Tensor) -> Tensor:
     ``[B * H, Np/32, Np/32, 4, 64, 4]``: entry ``[.., qb, kb, v, lane, e]`` with
     ``lane = 32 g + li`` is query ``32 qb + li``, key ``32 kb + 8 v + 4 g + e``."""
     b, h, n1, n2 = bias.shape
-    _need(n1 == n2 and n1 % 32 == 0, "bias must be [B, H, Np, Np] with Np % 32 == 0")
+    if not (n1 == n2 and n1 % 32 == 0):
+        _refuse("bias must be [B, H, Np, Np] with Np % 32 == 0")
     nb = n1 // 32
     t = bias.float().reshape(b * h, nb, 32, nb, 4, 2, 4)  # [bh, qb, li, kb, v, g, e]
     return t.permute(0, 1, 3, 4, 5, 2, 6).reshape(b * h, nb, nb, 4, 64, 4).contiguous()
@@ -684,12 +731,14 @@ def flash_v_layout(v_t: Tensor) -> Tensor:
     by 32 keys (block ``kb`` holds ``[d][keys 32 kb ..]``), and inside every group of 16 keys
     the keys stored in the order 0-3, 8-11, 4-7, 12-15 (index bits 2 and 3 exchanged)."""
     n = v_t.shape[-1]
-    _need(n % 32 == 0, "the key count must be a multiple of 32")
+    if n % 32 != 0:
+        _refuse("the key count must be a multiple of 32")
     idx = torch.arange(n, device=v_t.device)
     perm = (idx & ~12) | ((idx & 4) << 1) | ((idx & 8) >> 1)
     d = v_t.shape[-2]
     blocked = v_t[..., perm].unflatten(-1, (n // 32, 32)).transpose(-3, -2)  # [..., Np/32, d, 32]
-    _need(blocked.shape[-2] == d, "v_t must be [..., d, Np]")
+    if blocked.shape[-2] != d:
+        _refuse("v_t must be [..., d, Np]")
     return blocked.contiguous()
 
 
@@ -711,20 +760,26 @@ def flash_attention_bias(
     ``out [B, R, n_valid, H * 32]`` bf16 receives ``o`` for rows < rows_valid.
     """
     batch, heads, rows, n_pad, d = q.shape
-    _need(d == TRI_HEAD_DIM, f"head dim {d} (the kernel takes {TRI_HEAD_DIM})")
-    _need(k.shape == q.shape and v_t.shape == (batch, heads, rows, n_pad // 32, d, 32), "q/k/v_t shapes")
-    _need(bias_blk.dtype == torch.float32 and bias_blk.numel() == batch * heads * n_pad * n_pad,
-          "bias_blk must be the blocked fp32 layout of [B, H, Np, Np]")
-    _need(all(t.is_contiguous() for t in (q, k, v_t, bias_blk)), "operands must be contiguous")
-    _need(out.dtype == torch.bfloat16 and out.dim() == 4 and out.shape[-1] == heads * d,
-          "out must be bf16 [B, R, n_valid, H * 32]")
-    _need(out.device == q.device and out.stride(3) == 1, "out must be on q's device with unit channel stride")
-    _need(0 <= rows_valid <= rows and 0 <= n_valid <= n_pad, "valid extents exceed the operands")
-    _need(out.shape[0] >= batch and out.shape[1] >= rows_valid and out.shape[2] >= n_valid,
-          f"out {tuple(out.shape)} does not cover [{batch}, {rows_valid}, {n_valid}, {heads * d}]")
-    _need(all(t.device == q.device for t in (k, v_t, bias_blk)), "operands must share q's device")
-    status = _native.lib().ffk_flash_attention_bias(
-        q.data_ptr(), k.data_ptr(), v_t.data_ptr(), bias_blk.data_ptr(), out.data_ptr(),
+    if d != TRI_HEAD_DIM:
+        _refuse(f"head dim {d} (the kernel takes {TRI_HEAD_DIM})")
+    if not (k.shape == q.shape and v_t.shape == (batch, heads, rows, n_pad // 32, d, 32)):
+        _refuse("q/k/v_t shapes")
+    if not (bias_blk.dtype == torch.float32 and bias_blk.numel() == batch * heads * n_pad * n_pad):
+        _refuse("bias_blk must be the blocked fp32 layout of [B, H, Np, Np]")
+    if not (all(t.is_contiguous() for t in (q, k, v_t, bias_blk))):
+        _refuse("operands must be contiguous")
+    if not (out.dtype == torch.bfloat16 and out.dim() == 4 and out.shape[-1] == heads * d):
+        _refuse("out must be bf16 [B, R, n_valid, H * 32]")
+    if not (out.device == q.device and out.stride(3) == 1):
+        _refuse("out must be on q's device with unit channel stride")
+    if not (0 <= rows_valid <= rows and 0 <= n_valid <= n_pad):
+        _refuse("valid extents exceed the operands")
+    if not (out.shape[0] >= batch and out.shape[1] >= rows_valid and out.shape[2] >= n_valid):
+        _refuse(f"out {tuple(out.shape)} does not cover [{batch}, {rows_valid}, {n_valid}, {heads * d}]")
+    if not (all(t.device == q.device for t in (k, v_t, bias_blk))):
+        _refuse("operands must share q's device")
+    status = _native.calls().ffk_flash_attention_bias(
+        q, k, v_t, bias_blk, out,
         batch, heads, rows, n_pad, rows_valid, n_valid,
         out.stride(0), out.stride(1), out.stride(2), _stream(q.device),
     )

@@ -30,11 +30,16 @@ from typing import Any
 import torch
 from torch import nn
 
-from foldforge_amd import dispatch, torch_ops
+from foldforge_amd import dispatch, kernels, torch_ops
 
 Tensor = torch.Tensor
 
 HIP_ARCH = "gfx950"
+
+
+#: device index -> architecture, as :func:`device_arch` found it (asked for every tensor of every
+#: call; a device's architecture does not change)
+_ARCH: dict[int, str] = {}
 
 
 class BackendUnsupported(RuntimeError):
@@ -45,14 +50,17 @@ def device_arch(device: torch.device) -> str | None:
     """gfx architecture of a ROCm device (``"gfx950"`` on an MI355X), None elsewhere."""
     if device.type != "cuda" or not torch.cuda.is_available():
         return None
-    name = torch.cuda.get_device_properties(device).gcnArchName
-    return name.split(":")[0]
+    index = torch.cuda._utils._get_device_index(device, optional=True)
+    name = _ARCH.get(index)
+    if name is None:
+        name = _ARCH[index] = torch.cuda.get_device_properties(device).gcnArchName.split(":")[0]
+    return name
 
 
 def hip_reason(*tensors: Tensor) -> str | None:
     """Why the hip backend cannot take tensors on these devices (None: it can)."""
     for t in tensors:
-        if t is None:
+        if t is None or (t.is_cuda and _ARCH.get(t.get_device()) == HIP_ARCH):
             continue
         if t.device.type != "cuda":
             return f"a {t.device.type} tensor (the hip backend needs a gfx950 device)"
@@ -141,6 +149,49 @@ class EngineOp:
         return getattr(self, f"_forward_{self._route(args, kwargs)}")(*args, residual=False, **kwargs)
 
 
+def _spec(**paths: str) -> tuple[tuple[str, str, str], ...]:
+    """``name="child.kind"`` -> ``(name, child, kind)`` for :func:`_read`."""
+    return tuple((name, *path.split(".")) for name, path in paths.items())  # type: ignore[misc]
+
+
+def _read(module: nn.Module, spec: tuple[tuple[str, str, str], ...]) -> dict[str, Any]:
+    """``{name: module.<child>.<kind>}``, straight from the parameter tables where it is a plain
+    parameter (a call reads a dozen, and ``nn.Module``'s attribute lookup is two Python calls
+    each), else by attribute (parametrised and replicated ones)."""
+    children = module._modules
+    try:
+        return {name: children[child]._parameters[kind] for name, child, kind in spec}  # type: ignore[union-attr]
+    except (KeyError, AttributeError):
+        return {name: getattr(getattr(module, child), kind) for name, child, kind in spec}
+
+
+# kernel arguments -> the parameters the ops pass for them
+_TRIMUL = _spec(
+    ln_pair_weight="ln_pair.weight", ln_pair_bias="ln_pair.bias", to_left="to_left.weight",
+    to_right="to_right.weight", to_left_gate="to_left_gate.weight", to_right_gate="to_right_gate.weight",
+    ln_out_weight="ln_out.weight", ln_out_bias="ln_out.bias", to_out="to_out.weight", to_gate="to_gate.weight")
+_TRIATTN_PLAIN = _spec(
+    ln_pair_weight="ln_pair.weight", ln_pair_bias="ln_pair.bias", to_bias="to_bias.weight",
+    to_query="to_query.weight", to_key="to_key.weight", to_value="to_value.weight",
+    to_gate="to_gate.weight", to_out="to_out.weight")
+_TRIATTN = _TRIATTN_PLAIN + _spec(gate_bias="to_gate.bias", out_bias="to_out.bias")
+_TRIATTN_DUAL = _TRIATTN + _spec(to_out_t="to_out_t.weight", out_t_bias="to_out_t.bias")
+_TRANSITION = _spec(
+    ln_weight="ln_in.weight", ln_bias="ln_in.bias", expand_a="expand_a.weight",
+    expand_b="expand_b.weight", squeeze="squeeze.weight")
+_APB = _spec(
+    ln_single_weight="ln_single.weight", ln_single_bias="ln_single.bias", to_query="to_query.weight",
+    query_bias="to_query.bias", to_key="to_key.weight", to_value="to_value.weight",
+    ln_pair_weight="ln_pair.weight", to_bias="to_bias.weight", to_gate="to_gate.weight", to_out="to_out.weight")
+_PWA = _spec(
+    ln_msa_weight="ln_msa.weight", ln_msa_bias="ln_msa.bias", ln_pair_weight="ln_pair.weight",
+    to_bias="to_bias.weight", to_value="to_value.weight", to_gate="to_gate.weight", to_out="to_out.weight")
+_OPM = _spec(
+    ln_weight="ln_msa.weight", ln_bias="ln_msa.bias", to_left="to_left.weight", to_right="to_right.weight",
+    to_out="to_out.weight", to_out_bias="to_out.bias", left_bias="to_left.bias", right_bias="to_right.bias")
+_OPM_GROUPED = _OPM + _spec(norm_weight="product_norm.weight", norm_bias="product_norm.bias")
+
+
 def _linear(d_in: int, d_out: int, bias: bool = False) -> nn.Linear:
     return nn.Linear(d_in, d_out, bias=bias)
 
@@ -179,8 +230,6 @@ class LayerNorm(EngineOp, nn.LayerNorm):
         return torch_ops.layer_norm(self, x)
 
     def _forward_hip(self, x: Tensor) -> Tensor:
-        from foldforge_amd import kernels
-
         return kernels.layer_norm(x.contiguous(), self.weight, self.bias, self.eps)
 
 
@@ -230,9 +279,7 @@ class TriangleMultiplication(EngineOp, MasterWeights, nn.Module):
         reason = _pair_reason(x, mask)
         if reason is not None:
             return reason
-        from foldforge_amd.kernels import trimul_supported
-
-        if x.shape[-1] != self.d_pair or not trimul_supported(self.d_pair, self.d_hidden):
+        if x.shape[-1] != self.d_pair or not kernels.trimul_supported(self.d_pair, self.d_hidden):
             return (f"d_pair={x.shape[-1]} d_hidden={self.d_hidden} (the kernels take 128 / 128, or a "
                     "pair width a multiple of 64 up to 256 with a hidden width a multiple of 64 up to 768)")
         return None
@@ -245,18 +292,9 @@ class TriangleMultiplication(EngineOp, MasterWeights, nn.Module):
     def _forward_hip(self, x: Tensor, mask: Tensor, *, residual: bool = True) -> Tensor:
         if self.dead:
             return x if residual else torch.zeros_like(x)
-        from foldforge_amd import kernels
-
         return kernels.triangle_multiplicative_update(
-            x.contiguous(), mask.contiguous(),
-            ln_pair_weight=self.ln_pair.weight, ln_pair_bias=self.ln_pair.bias,
-            to_left=self.to_left.weight, to_right=self.to_right.weight,
-            to_left_gate=self.to_left_gate.weight, to_right_gate=self.to_right_gate.weight,
-            ln_out_weight=self.ln_out.weight, ln_out_bias=self.ln_out.bias,
-            to_out=self.to_out.weight, to_gate=self.to_gate.weight,
-            outgoing=self.outgoing, residual=residual, length_divided=self.divide_by_length,
-            eps=self.ln_pair.eps,
-        )
+            x.contiguous(), mask.contiguous(), outgoing=self.outgoing, residual=residual,
+            length_divided=self.divide_by_length, eps=self.ln_pair.eps, **_read(self, _TRIMUL))
 
 
 class TriangleMultiplicationRF3(TriangleMultiplication):
@@ -334,11 +372,9 @@ class TriangleAttention(EngineOp, MasterWeights, nn.Module):
         reason = _pair_reason(x, mask)
         if reason is not None:
             return reason
-        from foldforge_amd.kernels import triangle_attention_supported
-
         d = self.d_hidden // self.n_head
         if (x.shape[-1] != self.d_pair or self.d_hidden % self.n_head
-                or not triangle_attention_supported(self.d_pair, self.n_head, d, self.transposed_bias)):
+                or not kernels.triangle_attention_supported(self.d_pair, self.n_head, d, self.transposed_bias)):
             return (f"d_pair={x.shape[-1]} heads={self.n_head} hidden={self.d_hidden} (the kernels "
                     "take 128 with 4 x 32, or pair 64 / 128 / 256 with at most 32 heads of 8 to 64 "
                     "channels, heads x d_head a multiple of 64)")
@@ -354,20 +390,11 @@ class TriangleAttention(EngineOp, MasterWeights, nn.Module):
     def _forward_hip(self, x: Tensor, mask: Tensor, *, residual: bool = True) -> Tensor:
         if self.dead:
             return x if residual else torch.zeros_like(x)
-        from foldforge_amd import kernels
-
         return kernels.triangle_attention(
-            x.contiguous(), mask.contiguous(),
-            ln_pair_weight=self.ln_pair.weight, ln_pair_bias=self.ln_pair.bias,
-            to_bias=self.to_bias.weight, to_query=self.to_query.weight,
-            to_key=self.to_key.weight, to_value=self.to_value.weight,
-            to_gate=self.to_gate.weight, to_out=self.to_out.weight, n_head=self.n_head,
-            gate_bias=self.to_gate.bias, out_bias=self.to_out.bias,
-            to_out_t=self.to_out_t.weight if self.dual_output else None,
-            out_t_bias=self.to_out_t.bias if self.dual_output else None,
-            starting=self.starting, transposed_bias=self.transposed_bias,
-            untransposed_output=self.untransposed_output, residual=residual, eps=self.ln_pair.eps,
-        )
+            x.contiguous(), mask.contiguous(), n_head=self.n_head, starting=self.starting,
+            transposed_bias=self.transposed_bias, untransposed_output=self.untransposed_output,
+            residual=residual, eps=self.ln_pair.eps,
+            **_read(self, _TRIATTN_DUAL if self.dual_output else _TRIATTN))
 
 
 class TriangleAttentionAF3(TriangleAttention):
@@ -423,9 +450,7 @@ class Transition(EngineOp, MasterWeights, nn.Module):
             return reason
         if x.dtype != torch.bfloat16:
             return f"{x.dtype} activations (the kernel takes bf16)"
-        from foldforge_amd.kernels import transition_supported
-
-        if not transition_supported(self.d, self.n):
+        if not kernels.transition_supported(self.d, self.n):
             return (f"width {self.d} x {self.n} (the kernels take 128 x 4, or d and "
                     "n * d multiples of 64)")
         return None
@@ -438,13 +463,8 @@ class Transition(EngineOp, MasterWeights, nn.Module):
     def _forward_hip(self, x: Tensor, *, residual: bool = True) -> Tensor:
         if self.dead:
             return x if residual else torch.zeros_like(x)
-        from foldforge_amd import kernels
-
         return kernels.transition(
-            x.contiguous(), ln_weight=self.ln_in.weight, ln_bias=self.ln_in.bias,
-            expand_a=self.expand_a.weight, expand_b=self.expand_b.weight,
-            squeeze=self.squeeze.weight, residual=residual, eps=self.ln_in.eps,
-        )
+            x.contiguous(), residual=residual, eps=self.ln_in.eps, **_read(self, _TRANSITION))
 
 
 class AttentionPairBias(EngineOp, MasterWeights, nn.Module):
@@ -477,9 +497,7 @@ class AttentionPairBias(EngineOp, MasterWeights, nn.Module):
             return f"single shape {tuple(s.shape)} for pair {tuple(z.shape)}"
         if z.shape[-1] != 128 or self.d_pair != 128:
             return f"d_pair={z.shape[-1]} (the kernels take 128)"
-        from foldforge_amd.kernels import single_attention_heads_supported
-
-        if not single_attention_heads_supported(self.d_single, self.n_head):
+        if not kernels.single_attention_heads_supported(self.d_single, self.n_head):
             return (f"d_single={self.d_single} heads={self.n_head} (the kernels take a multiple "
                     "of 64 split into at most 32 heads of 8, 16, 24 or 32)")
         if extra_bias is not None:
@@ -504,18 +522,10 @@ class AttentionPairBias(EngineOp, MasterWeights, nn.Module):
                      *, residual: bool = True) -> Tensor:
         if self.dead:
             return s if residual else torch.zeros_like(s)
-        from foldforge_amd import kernels
-
         return kernels.attention_pair_bias(
-            s.contiguous(), z.contiguous(), mask.contiguous(),
-            ln_single_weight=self.ln_single.weight, ln_single_bias=self.ln_single.bias,
-            to_query=self.to_query.weight, query_bias=self.to_query.bias,
-            to_key=self.to_key.weight, to_value=self.to_value.weight,
-            ln_pair_weight=self.ln_pair.weight, to_bias=self.to_bias.weight,
-            to_gate=self.to_gate.weight, to_out=self.to_out.weight, n_head=self.n_head,
-            gate_bias=self.gate_bias, extra_bias=extra_bias, residual=residual,
-            eps_single=self.ln_single.eps, eps_pair=self.ln_pair.eps,
-        )
+            s.contiguous(), z.contiguous(), mask.contiguous(), n_head=self.n_head, gate_bias=self.gate_bias,
+            extra_bias=extra_bias, residual=residual, eps_single=self.ln_single.eps, eps_pair=self.ln_pair.eps,
+            **_read(self, _APB))
 
 
 # ------------------------------------------------------------------------------------ MSA stack
@@ -549,9 +559,7 @@ class MSAPairWeightedAveraging(EngineOp, MasterWeights, nn.Module):
             return f"MSA shape {tuple(m.shape)} for pair {tuple(z.shape)}"
         if z.shape[-1] != 128 or self.d_pair != 128:
             return f"d_pair={z.shape[-1]} (the kernels take 128)"
-        from foldforge_amd.kernels import msa_pair_weighted_averaging_supported
-
-        if not msa_pair_weighted_averaging_supported(self.d_msa, self.n_head, self.d_hidden):
+        if not kernels.msa_pair_weighted_averaging_supported(self.d_msa, self.n_head, self.d_hidden):
             return (f"d_msa={self.d_msa} heads={self.n_head} x {self.d_hidden} (the kernels take "
                     "d_msa a multiple of 64 up to 768, at most 32 heads of a multiple of 4, "
                     "heads x d_head a multiple of 64 up to 768)")
@@ -565,16 +573,9 @@ class MSAPairWeightedAveraging(EngineOp, MasterWeights, nn.Module):
     def _forward_hip(self, m: Tensor, z: Tensor, mask: Tensor, *, residual: bool = True) -> Tensor:
         if self.dead:
             return m if residual else torch.zeros_like(m)
-        from foldforge_amd import kernels
-
         return kernels.msa_pair_weighted_averaging(
-            m.contiguous(), z.contiguous(), mask.contiguous(),
-            ln_msa_weight=self.ln_msa.weight, ln_msa_bias=self.ln_msa.bias,
-            ln_pair_weight=self.ln_pair.weight, to_bias=self.to_bias.weight,
-            to_value=self.to_value.weight, to_gate=self.to_gate.weight, to_out=self.to_out.weight,
-            n_head=self.n_head, residual=residual, eps_msa=self.ln_msa.eps,
-            eps_pair=self.ln_pair.eps,
-        )
+            m.contiguous(), z.contiguous(), mask.contiguous(), n_head=self.n_head, residual=residual,
+            eps_msa=self.ln_msa.eps, eps_pair=self.ln_pair.eps, **_read(self, _PWA))
 
 
 class OuterProductMean(EngineOp, MasterWeights, nn.Module):
@@ -627,16 +628,14 @@ class OuterProductMean(EngineOp, MasterWeights, nn.Module):
         if residual is not None and (residual.dtype != torch.bfloat16
                                      or tuple(residual.shape) != (m.shape[0], m.shape[2], m.shape[2], self.d_pair)):
             return f"residual {tuple(residual.shape)} {residual.dtype}"
-        from foldforge_amd.kernels import outer_product_mean_grouped_supported, outer_product_mean_supported
-
         if self.groups != 1:
             dg = self.d_hidden // self.groups
-            if not outer_product_mean_grouped_supported(self.d_msa, self.groups, dg, self.d_pair):
+            if not kernels.outer_product_mean_grouped_supported(self.d_msa, self.groups, dg, self.d_pair):
                 return (f"d_msa={self.d_msa} {self.groups} groups of {dg} d_pair={self.d_pair} (the "
                         "grouped kernels take d_msa a multiple of 64 up to 768, 8 groups of 8, "
                         "d_pair 128 or 256)")
             return None
-        if not outer_product_mean_supported(self.d_msa, self.d_hidden, self.d_pair):
+        if not kernels.outer_product_mean_supported(self.d_msa, self.d_hidden, self.d_pair):
             return (f"d_msa={self.d_msa} d_hidden={self.d_hidden} d_pair={self.d_pair} (the kernels "
                     "take d_msa a multiple of 64 up to 768, d_hidden 32, d_pair 128)")
         return None
@@ -650,27 +649,15 @@ class OuterProductMean(EngineOp, MasterWeights, nn.Module):
     def _forward_hip(self, m: Tensor, mask: Tensor, residual: Tensor | None = None) -> Tensor:
         if self.dead:
             return self._forward_pytorch(m, mask, residual)
-        from foldforge_amd import kernels
-
         if self.groups != 1:
             return kernels.outer_product_mean_grouped(
-                m.contiguous(), mask.contiguous(), groups=self.groups, ln_weight=self.ln_msa.weight,
-                ln_bias=self.ln_msa.bias, to_left=self.to_left.weight, to_right=self.to_right.weight,
-                norm_weight=self.product_norm.weight, norm_bias=self.product_norm.bias,
-                to_out=self.to_out.weight, to_out_bias=self.to_out.bias, left_bias=self.to_left.bias,
-                right_bias=self.to_right.bias,
-                residual=None if residual is None else residual.contiguous(),
-                eps=self.ln_msa.eps, norm_eps=self.product_norm.eps,
-            )
+                m.contiguous(), mask.contiguous(), groups=self.groups,
+                residual=None if residual is None else residual.contiguous(), eps=self.ln_msa.eps,
+                norm_eps=self.product_norm.eps, **_read(self, _OPM_GROUPED))
         return kernels.outer_product_mean(
-            m.contiguous(), mask.contiguous(), ln_weight=self.ln_msa.weight,
-            ln_bias=self.ln_msa.bias, to_left=self.to_left.weight, to_right=self.to_right.weight,
-            to_out=self.to_out.weight, to_out_bias=self.to_out.bias, left_bias=self.to_left.bias,
-            right_bias=self.to_right.bias,
-            residual=None if residual is None else residual.contiguous(),
+            m.contiguous(), mask.contiguous(), residual=None if residual is None else residual.contiguous(),
             count_offset=self.count_offset, normalize_before_proj=self.normalize_before_proj,
-            eps=self.ln_msa.eps,
-        )
+            eps=self.ln_msa.eps, **_read(self, _OPM))
 
     def delta(self, m: Tensor, mask: Tensor, residual: Tensor | None = None) -> Tensor:
         """The update alone (what the forward returns without ``residual``)."""
@@ -700,18 +687,10 @@ def attention_then_transition(att: "TriangleAttention", tr: "Transition", z: Ten
         # attention's output, which has z's shape, dtype and device
         b_tr = tr._route((z,), {})
         if b_tr == "hip":
-            from foldforge_amd import kernels
-
             return kernels.triangle_attention_transition(
-                z.contiguous(), mask.contiguous(),
-                ln_pair_weight=att.ln_pair.weight, ln_pair_bias=att.ln_pair.bias,
-                to_bias=att.to_bias.weight, to_query=att.to_query.weight,
-                to_key=att.to_key.weight, to_value=att.to_value.weight,
-                to_gate=att.to_gate.weight, to_out=att.to_out.weight,
-                ln_weight=tr.ln_in.weight, ln_bias=tr.ln_in.bias, expand_a=tr.expand_a.weight,
-                expand_b=tr.expand_b.weight, squeeze=tr.squeeze.weight, starting=att.starting,
+                z.contiguous(), mask.contiguous(), starting=att.starting,
                 transposed_bias=att.transposed_bias, eps_pair=att.ln_pair.eps, eps=tr.ln_in.eps,
-            )
+                **_read(att, _TRIATTN_PLAIN), **_read(tr, _TRANSITION))
         return getattr(tr, f"_forward_{b_tr}")(att._forward_hip(z, mask))
     z = getattr(att, f"_forward_{b_att}")(z, mask)
     return tr(z)

@@ -107,3 +107,40 @@ def test_build_recipe_targets_gfx950_without_packed_fp32():
         assert "--offload-arch=gfx950" in cmd
         assert "-packed-fp32-ops" in cmd
     assert "--offload-arch=gfx950" in build.link_command([s.with_suffix(".o") for s in srcs])
+
+
+def test_compiled_calls_refuse_what_the_checks_refuse(lib):
+    import torch
+
+    calls = _native.calls()
+    x, w = torch.zeros(2, 4), torch.zeros(3, 4)
+    assert calls.params_ok(x, (w, torch.zeros(4)), ((3, 4), (4,)))
+    for bad in (torch.zeros(4, 3), torch.zeros(4, 3).t(), w.double(), w.to("meta"), torch.zeros(3, 4, 1), None):
+        assert not calls.params_ok(x, (w, bad), ((3, 4), (3, 4)))
+    # the workspace queries read their arguments as ctypes does, and reject a wrong count or type
+    args = (2, 300, 128, 128)
+    assert calls.ffk_triangle_multiplication_workspace(*args) == lib.ffk_triangle_multiplication_workspace(*args)
+    with pytest.raises(TypeError):
+        calls.ffk_triangle_multiplication_workspace(*args[:3])
+    with pytest.raises(TypeError):
+        calls.ffk_triangle_multiplication_workspace(2, "300", 128, 128)
+    with pytest.raises(OverflowError):
+        calls.ffk_triangle_multiplication_workspace(2, 300, 1 << 40, 128)
+
+
+def test_parameters_are_read_by_attribute_where_they_are_not_plain():
+    import torch
+    from torch.nn.utils import parametrize
+
+    from foldforge_amd import factories, modules
+
+    m = factories.transition(64, 2)
+    assert modules._read(m, modules._TRANSITION)["squeeze"] is m.squeeze.weight
+
+    class Twice(torch.nn.Module):
+        def forward(self, w):
+            return 2 * w
+
+    plain = m.squeeze.weight.detach().clone()
+    parametrize.register_parametrization(m.squeeze, "weight", Twice())
+    assert torch.equal(modules._read(m, modules._TRANSITION)["squeeze"], 2 * plain)
