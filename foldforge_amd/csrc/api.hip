@@ -374,6 +374,23 @@ int32_t transition_check(const void* x, const float* ln_w, const float* ln_b, co
 int32_t transition_run(const TransitionWs& w, const void* x, const float* ln_w, const float* ln_b,
                        const float* wa, const float* wb, const float* wsq, void* out, int64_t rows,
                        int d, int factor, int residual, float eps, hipStream_t st) {
+  if (d == 64 && (factor == 2 || factor == 4)) {
+    // the widths whose three weights fit in LDS (the hidden rows of the workspace stay unused)
+    TransitionRowsArgs a;
+    a.x = static_cast<const bf16*>(x);
+    a.ln_w = ln_w;
+    a.ln_b = ln_b;
+    a.w_a = wa;
+    a.w_b = wb;
+    a.w_s = wsq;
+    a.out = static_cast<bf16*>(out);
+    a.rows = rows;
+    a.factor = factor;
+    a.residual = residual ? 1 : 0;
+    a.eps = eps;
+    launch_transition_rows(a, st);
+    return check_launch("transition");
+  }
   if (!transition_fused(d, factor)) {
     RowGemmArgs g{};
     g.w_split = 1;  // fp32-accurate weights (see row_gemm)

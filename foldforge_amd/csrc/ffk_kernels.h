@@ -275,6 +275,18 @@ struct TriattnRowsArgs {
 };
 void launch_triattn_out_rows(const TriattnRowsArgs& a, hipStream_t stream);
 
+// SwiGLU transition of 64-channel rows, hidden width 64 factor (factor 2 or 4); out may alias x.
+struct TransitionRowsArgs {
+  const bf16* x;                     // [rows][64]
+  const float *ln_w, *ln_b;          // [64]
+  const float *w_a, *w_b, *w_s;      // [64 factor][64] twice, [64][64 factor]
+  bf16* out;                         // [rows][64]
+  int64_t rows;                      // > 0
+  int factor, residual;
+  float eps;
+};
+void launch_transition_rows(const TransitionRowsArgs& a, hipStream_t stream);
+
 // Channel planes P [batch][hid][np][np] -> token rows Pt [batch][n][n][hid] (bf16).
 void launch_planes_to_rows(const bf16* planes, bf16* rows, int batch, int hid, int n, int np,
                            hipStream_t stream);

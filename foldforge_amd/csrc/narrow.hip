@@ -468,6 +468,179 @@ __global__ __launch_bounds__(64 * kTmoWaves) void triattn_out_rows(TriattnRowsAr
   }
 }
 
+// Transition of 64-channel rows, hidden width 64 F (F = 2: the AF3 and Protenix-1 template
+// stacks; F = 4: the Boltz-2 and RoseTTAFold3 ones and the MSA track):
+//   out = x + (silu(LN(x) W_a^T) * (LN(x) W_b^T)) W_s^T
+// as one streaming kernel, so the hidden rows never reach memory (two row GEMMs wrote and read
+// 128 F bytes of them per 128-byte row: 131072 rows, F = 4: 66 -> 31 us; 589824
+// rows, F = 2: 145 -> 71 us). All three weights sit in LDS
+// as bf16 (F = 4: 108 KiB, one workgroup of 8 waves per CU; F = 2: 54 KiB, two of 4: a
+// wave needs 190 VGPRs, and three waves per SIMD spilled: 96 instead of 73 us for F = 2). Every
+// wave walks tiles of 32 rows on its own, the next tile's rows loaded while it works: lane
+// (li, g) holds channels 32 g .. 32 g + 31 of row li, normalised to bf16 hi + lo as in the row
+// GEMMs. Per 32 hidden channels the two expand products leave the lane with 16 of its row's
+// hidden values, which in accumulator order are the squeeze's operand as they stand (its
+// weight columns are stored in that order); the squeeze rows are permuted so that a lane's
+// accumulators hold its own channels of x. expand_a is held times -log2(e) and the squeeze times
+// -ln(2), so that the accumulator is the exponent of the sigmoid (as in transition.hip). Bound
+// by instruction issue: per tile 160 / 80 MFMAs (5.1 / 2.6 k cycles) and about as long again of
+// SwiGLU, normalisation and rounding.
+template <int F>
+struct __attribute__((aligned(16))) TransitionRowsLds {
+  bf16 wa[64 * F * kTmoWs];        // expand_a rows, k = 64
+  bf16 wb[64 * F * kTmoWs];        // expand_b rows
+  bf16 ws[64 * (64 * F + 8)];      // squeeze rows (permuted), hidden in accumulator order
+  float lnw[64], lnb[64];
+};
+constexpr int transition_rows_waves(int F) { return F == 4 ? 8 : 4; }
+
+template <int F>
+__global__ __launch_bounds__(64 * transition_rows_waves(F), 2) void transition_rows(TransitionRowsArgs a) {
+  constexpr int W = transition_rows_waves(F), H = 64 * F, HS = H + 8;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  TransitionRowsLds<F>& lds = *reinterpret_cast<TransitionRowsLds<F>*>(smem);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, g = lane >> 5, li = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int idx = tid; idx < H * 8; idx += 64 * W) {
+    const int row = idx >> 3, ch = 8 * (idx & 7);
+    bf16x8 w;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = (bf16)(-kLog2e * a.w_a[row * 64 + ch + e]);
+    *reinterpret_cast<bf16x8*>(lds.wa + row * kTmoWs + ch) = w;
+    *reinterpret_cast<bf16x8*>(lds.wb + row * kTmoWs + ch) = cvt8(a.w_b + row * 64 + ch);
+  }
+  for (int idx = tid; idx < 64 * (H / 8); idx += 64 * W) {
+    // piece q of a 16-block: hidden 4 q .. 4 q + 3 and 8 + 4 q .. 8 + 4 q + 3
+    const int row = idx / (H / 8), p = idx % (H / 8);
+    const float* src = a.w_s + tmo_perm(row) * H + 16 * (p >> 1) + 4 * (p & 1);
+    bf16x8 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      w[e] = (bf16)((-1.f / kLog2e) * src[e]);
+      w[4 + e] = (bf16)((-1.f / kLog2e) * src[8 + e]);
+    }
+    *reinterpret_cast<bf16x8*>(lds.ws + row * HS + 8 * p) = w;
+  }
+  if (tid < 64) {
+    lds.lnw[tid] = a.ln_w[tid];
+    lds.lnb[tid] = a.ln_b[tid];
+  }
+  __syncthreads();
+
+  const int64_t tiles = (a.rows + 31) / 32;
+  const int64_t stride = (int64_t)gridDim.x * W;
+  int64_t t = (int64_t)wave * gridDim.x + blockIdx.x;  // few tiles spread over the workgroups
+  if (t >= tiles) return;
+
+  auto fetch = [&](int64_t tile, bf16x8* x) __attribute__((always_inline)) {
+    // the last real row past the end
+    const int64_t m = min(min(tile, tiles - 1) * 32 + li, a.rows - 1);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = ld8(a.x + m * 64 + 32 * g + 8 * s);
+  };
+  auto process = [&](int64_t tile, const bf16x8* x) __attribute__((always_inline)) {
+    float s1 = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s1 += (float)x[s][e];
+    const float mean = pair_sum(s1) * (1.f / 64);
+    float s2 = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float d = (float)x[s][e] - mean;
+        s2 += d * d;
+      }
+    const float rstd = __builtin_amdgcn_rsqf(pair_sum(s2) * (1.f / 64) + a.eps);
+    int cb = 32 * g;  // the affine is read per tile (held, it would take 64 registers)
+    asm volatile("" : "+v"(cb));
+    bf16x8 xh[4], xl[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const f32x4 w0 = *reinterpret_cast<const f32x4*>(&lds.lnw[cb + 8 * s]);
+      const f32x4 w1 = *reinterpret_cast<const f32x4*>(&lds.lnw[cb + 8 * s + 4]);
+      const f32x4 b0 = *reinterpret_cast<const f32x4*>(&lds.lnb[cb + 8 * s]);
+      const f32x4 b1 = *reinterpret_cast<const f32x4*>(&lds.lnb[cb + 8 * s + 4]);
+      f32x4 y0, y1;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        y0[e] = ((float)x[s][e] - mean) * rstd * w0[e] + b0[e];
+        y1[e] = ((float)x[s][4 + e] - mean) * rstd * w1[e] + b1[e];
+      }
+      split8(y0, y1, xh[s], xl[s]);
+    }
+    f32x16 oy[2] = {zero16(), zero16()};
+#pragma unroll 1
+    for (int hb = 0; hb < 2 * F; ++hb) {
+      const bf16* wa = lds.wa + (32 * hb + li) * kTmoWs + 32 * g;
+      const bf16* wb = lds.wb + (32 * hb + li) * kTmoWs + 32 * g;
+      f32x16 av = zero16(), bv = zero16();
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bf16x8 a8 = ld8(wa + 8 * s), b8 = ld8(wb + 8 * s);
+        av = mfma32(a8, xl[s], av);
+        bv = mfma32(b8, xl[s], bv);
+        av = mfma32(a8, xh[s], av);
+        bv = mfma32(b8, xh[s], bv);
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        bf16x8 h;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float v = av[8 * k + e];
+          h[e] = (bf16)(v * sigmoid_scaled(v) * bv[8 * k + e]);
+        }
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2)
+          oy[t2] = mfma32(ld8(lds.ws + (32 * t2 + li) * HS + 32 * hb + 16 * k + 8 * g), h, oy[t2]);
+      }
+    }
+    const int64_t m = tile * 32 + li;
+    if (m >= a.rows) return;
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      bf16x8 y[2];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int c = 16 * t2 + i;  // channel within the lane's half
+        const float r = a.residual ? (float)x[c >> 3][c & 7] : 0.f;
+        y[i >> 3][i & 7] = (bf16)(oy[t2][i] + r);
+      }
+      bf16* dst = a.out + m * 64 + 32 * g + 16 * t2;
+      *reinterpret_cast<bf16x8*>(dst) = y[0];
+      *reinterpret_cast<bf16x8*>(dst + 8) = y[1];
+    }
+  };
+
+  bf16x8 x0[4], x1[4];
+  fetch(t, x0);
+  while (true) {
+    fetch(t + stride, x1);
+    process(t, x0);
+    t += stride;
+    if (t >= tiles) break;
+    fetch(t + stride, x0);
+    process(t, x1);
+    t += stride;
+    if (t >= tiles) break;
+  }
+}
+
+template <int F>
+void launch_transition_rows_t(const TransitionRowsArgs& a, hipStream_t stream) {
+  constexpr int W = transition_rows_waves(F);
+  const size_t lds = sizeof(TransitionRowsLds<F>);
+  if (lds > 65536)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(transition_rows<F>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const int64_t blocks = std::min<int64_t>((a.rows + 31) / 32, (int64_t)cu_count() * (F == 4 ? 1 : 2));
+  transition_rows<F><<<dim3((unsigned)blocks), 64 * W, lds, stream>>>(a);
+}
+
 }  // namespace
 
 // out[b][i][j][:] = (base ? base[b][i][j][:] : 0) + t[b][j][i][:]: one thread per 8 channels
@@ -527,6 +700,13 @@ void launch_triattn_out_rows(const TriattnRowsArgs& a, hipStream_t stream) {
     triattn_out_rows<128><<<grid, 64 * kTmoWaves, 0, stream>>>(a);
   else
     triattn_out_rows<64><<<grid, 64 * kTmoWaves, 0, stream>>>(a);
+}
+
+void launch_transition_rows(const TransitionRowsArgs& a, hipStream_t stream) {
+  if (a.factor == 4)
+    launch_transition_rows_t<4>(a, stream);
+  else
+    launch_transition_rows_t<2>(a, stream);
 }
 
 void launch_pair_add_transposed(const bf16* base, const bf16* t, bf16* out, int64_t batch, int n,

@@ -12,7 +12,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from foldforge_amd import dispatch, factories
+from foldforge_amd import dispatch, factories, kernels
 from foldforge_amd.trunk import randomise
 from oracle import pairstack as ps
 from tests.hip_calls import hip_delta, hip_forward
@@ -206,3 +206,23 @@ def test_pair_256_block_runs_on_the_kernels():
     rr = ps.rel_rms(got - z, want - z.double(), where)
     print(f"pair-256 block: update rel_rms={rr:.2e}", flush=True)
     assert rr <= 3e-2
+
+
+@pytest.mark.parametrize("factor", [2, 4])
+@pytest.mark.parametrize("rows", [1, 31, 33, 2561, 32 * 256 * 12 + 5, 2 * 32 * 256 * 12 + 33])
+def test_transition_of_64_channels(rows, factor):
+    """The fused 64-channel transition at the ends of its tiles (32 rows), of its workgroups and
+    of one pass of the grid, in place too. Tolerance: the bf16 rounding of the output (2^-8 of
+    the value) and of the hidden rows and weights (2^-9 each, averaged over 64 F products)."""
+    g = torch.Generator().manual_seed(rows)
+    m = randomise(factories.transition(64, factor), seed=factor).cuda()
+    m.set_backend("hip")
+    x = torch.randn(rows, 64, generator=g).bfloat16()
+    want = ps.transition(x, m.state_dict(), dtype=torch.float64)
+    got = m(x.cuda())
+    _check(hip_delta(m, x.cuda()).cpu(), want - x.double(), None, f"transition rows={rows} x{factor}")
+    assert ((got.cpu().double() - want).norm() / want.norm()).item() <= 4e-3
+    inplace = x.cuda()
+    kernels.transition(inplace, ln_weight=m.ln_in.weight, ln_bias=m.ln_in.bias, expand_a=m.expand_a.weight,
+                       expand_b=m.expand_b.weight, squeeze=m.squeeze.weight, out=inplace)
+    assert torch.equal(inplace, got)
