@@ -1439,9 +1439,7 @@ int32_t ffk_outer_product_mean(
   c.batch = (int)batch;
   c.n = (int)n;
   c.sp = (int)sp;
-  launch_opm_count(c, st);
-
-  launch_opm_pack(w_out, w.wp, d_pair, st);
+  launch_opm_prepare(c, w_out, w.wp, st);
 
   OpmContractArgs o;
   o.lt = w.lt;
@@ -1454,7 +1452,6 @@ int32_t ffk_outer_product_mean(
   o.batch = (int)batch;
   o.n = (int)n;
   o.sp = (int)sp;
-  o.cz = d_pair;
   o.count_offset = count_offset;
   o.normalize_before_proj = normalize_before_proj ? 1 : 0;
   launch_opm_contract(o, st);

@@ -363,6 +363,10 @@ __device__ __forceinline__ void dma4(const void* sbase, uint32_t voff, uint32_t 
   asm volatile(FFK_DMA_HAZARD "global_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m0)
                : "memory");
 }
+// Same with a whole 64-bit address per lane.
+__device__ __forceinline__ void dma16_at(const void* src, uint32_t m0) {
+  asm volatile(FFK_DMA_HAZARD "global_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(m0) : "memory");
+}
 // Wait until at most N vector-memory operations of this wave are in flight and its LDS
 // operations are done.
 template <int N>

@@ -320,17 +320,17 @@ struct OpmCountArgs {
   float* count;    // [batch][n][n]
   int batch, n, sp;
 };
-void launch_opm_count(const OpmCountArgs& a, hipStream_t stream);
-// to_out.weight [c_z][32 * 32] fp32 (column c * 32 + e) -> the contraction's bf16 order.
-void launch_opm_pack(const float* w, bf16* wp, int cz, hipStream_t stream);
+// The counts, and w = to_out.weight [128][32 * 32] fp32 (column c * 32 + e) -> wp in the
+// contraction's bf16 order.
+void launch_opm_prepare(const OpmCountArgs& a, const float* w, bf16* wp, hipStream_t stream);
 struct OpmContractArgs {
   const bf16 *lt, *rt;   // [batch][n][32][sp]
-  const bf16* wp;        // [c_z][1024] from launch_opm_pack
-  const float* bias;     // [c_z]
+  const bf16* wp;        // [128 * 1024] from launch_opm_prepare
+  const float* bias;     // [128]
   const float* count;    // [batch][n][n]
-  const bf16* res;       // [batch][n][n][c_z] or NULL
-  bf16* out;             // [batch][n][n][c_z]
-  int batch, n, sp, cz;
+  const bf16* res;       // [batch][n][n][128] or NULL
+  bf16* out;             // [batch][n][n][128]
+  int batch, n, sp;
   float count_offset;
   int normalize_before_proj;
 };

@@ -79,6 +79,18 @@ def test_outer_product_mean_matches_oracle(form, batch, depth, n, cm):
     _check(full, want + pair.double(), f"opm {form} residual")
 
 
+@pytest.mark.parametrize("batch,depth,n", [(1, 64, 8), (1, 65, 7), (2, 128, 17), (1, 129, 64), (1, 1, 1)])
+def test_outer_product_mean_at_stage_and_tile_edges(batch, depth, n):
+    """Whole and broken 64-row stages, whole and broken 8-token tiles, one token and one row."""
+    m, rows = _inputs(batch, depth, n, 64, seed=depth * n)
+    mod = _opm(64, seed=n, count_offset=1e-3, normalize_before_proj=False)
+    pair = torch.randn(batch, n, n, 128, generator=torch.Generator().manual_seed(n)).bfloat16()
+    got = hip_forward(mod, m.cuda(), rows.cuda(), residual=pair.cuda()).cpu()
+    want = ps.outer_product_mean(m, rows, mod.state_dict(), count_offset=1e-3, normalize_before_proj=False,
+                                 dtype=torch.float64)
+    _check(got, want + pair.double(), f"opm edges B={batch} S={depth} n={n}")
+
+
 def test_outer_product_mean_masked_entries_do_not_leak_and_empty_tokens_use_the_clamp():
     batch, depth, n, cm = 1, 40, 70, 64
     m, rows = _inputs(batch, depth, n, cm, seed=5, keep=0.6)
