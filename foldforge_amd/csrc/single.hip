@@ -113,12 +113,14 @@ __device__ __forceinline__ int apb_width(const RowGemmArgs& a) { return a.O / (a
 // The weight row (fp32, K values) multiplied by row li of output tile ot, and the tile's
 // segment and first channel as the epilogue reads them (packed tiles: see kEpiTrimul and
 // kEpiSwiglu below).
+// (row_stream's kEpiApb with flash_rows > 0: an epilogue of its own.)
+constexpr int kEpiApbFlash = 100;
 template <int EPI>
 __device__ inline const float* tile_weight_row(const RowGemmArgs& a, int ot, int li, int& seg, int& cbase) {
   const float* wr;
   seg = 0;
   cbase = 0;
-  if (EPI == kEpiApb) {
+  if (EPI == kEpiApb || EPI == kEpiApbFlash) {
     const int cs = apb_width(a);
     seg = (ot * 32) / cs;
     cbase = ot * 32 - seg * cs;
@@ -146,32 +148,6 @@ __device__ inline const float* tile_weight_row(const RowGemmArgs& a, int ot, int
   return wr;
 }
 
-__device__ __forceinline__ int stage_row(int r) { return r ^ ((r >> 2) & 1); }
-
-// A 32-row tile inside one run of an epilogue's row decomposition m = q L + rem (kEpiApb's flash
-// layout: L = np, q = b n + r, rem = the key j; kEpiTrimul: L = npm^2, q = b), computed once per
-// tile from its first row (uniform across the wave) instead of per lane and output tile.
-struct TileRun {
-  int64_t m0, q, rem0, b;
-  int r;
-};
-template <int EPI>
-__device__ __forceinline__ TileRun tile_run(const RowGemmArgs& a, int64_t m0) {
-  TileRun t{};
-  t.m0 = m0;
-  const int64_t len = EPI == kEpiTrimul ? (int64_t)a.npm * a.npm
-                      : EPI == kEpiOpm   ? (int64_t)a.sp
-                      : EPI == kEpiPwa   ? (int64_t)a.n
-                                         : (int64_t)a.np;
-  t.q = m0 / len;
-  t.rem0 = m0 - t.q * len;
-  if (EPI == kEpiApb) {
-    t.b = t.q / a.n;
-    t.r = (int)(t.q - t.b * a.n);
-  }
-  return t;
-}
-
 // The per-row value an epilogue reads from memory, once per row rather than per output tile:
 // kEpiTrimul's pair mask factor m_i m_k (symmetric, so the same for the transposed read).
 template <int EPI>
@@ -188,106 +164,18 @@ __device__ __forceinline__ float row_pre(const RowGemmArgs& a, const int64_t m) 
 // Epilogue of output tile ot for logical row m (< M): lane half g holds outputs
 // 32 ot + 8 v + 4 g + e in acc[4 v + e]. lb: the per-output biases (q_bias / gate_b of kEpiApb,
 // bias_out of kEpiResid) staged in LDS by output index, or NULL to read them from the arguments.
-// The loads an epilogue needs are all issued before its first store.
-// stage: a wave-private LDS tile of 32 x 32 bf16 (NULL: none), through which the
-// position-contiguous outputs (kEpiApb's flash-layout v^T, kEpiTrimul's channel planes) are
-// transposed and written as 16-byte pieces of 64-byte runs; tr: the tile's run (tile_run),
-// required with stage, whose 32 rows must then be consecutive positions of one run
-// (np % 32 == 0), so those epilogues take both only from the streaming kernel. ypre: the yin
-// values of kEpiGateResid, loaded by the caller (NULL: loaded here). rpre: the
-// residual values of kEpiResid and kEpiGateResid, loaded by the caller (NULL: loaded here); both
-// as the two 16-byte pieces (acc_pieces) of the lane. Channel row r of the tile sits at LDS row
-// stage_row(r), which puts the rows the two lane halves write at once (r, r + 4) on different
-// banks.
+// The loads an epilogue needs are all issued before its first store. ypre: the yin values of
+// kEpiGateResid, loaded by the caller (NULL: loaded here). rpre: the residual values of kEpiResid
+// and kEpiGateResid, loaded by the caller (NULL: loaded here); both as the two 16-byte pieces
+// (acc_pieces) of the lane.
 template <int EPI>
 __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16& acc, const int64_t m, const int ot,
                                     const int seg, const int cbase, const int g, const float* lb,
-                                    const float pre, bf16* stage = nullptr,
-                                    const TileRun* tr = nullptr, const bf16x8* rpre = nullptr,
+                                    const float pre, const bf16x8* rpre = nullptr,
                                     const bf16x8* ypre = nullptr) {
   // the bias of output o (global index gi of src when not staged)
   auto obias = [&](int o, const float* src, int gi) { return lb ? lb[o] : (src ? src[gi] : 0.f); };
-  if (EPI == kEpiApb && a.flash_rows > 0) {
-    const int cs = apb_width(a);
-    int64_t bn, b;
-    int j, r;
-    if (tr) {
-      bn = tr->q;
-      j = (int)(tr->rem0 + (m - tr->m0));
-      b = tr->b;
-      r = tr->r;
-    } else {
-      bn = m / a.np;
-      j = (int)(m - bn * a.np);
-      b = bn / a.n;
-      r = (int)(bn - b * a.n);
-    }
-    if (seg != 2) {
-      // q, k (the flash layouts) and the gate (token rows) as 16-byte pieces of 8 channels of
-      // one head (dh % 8 == 0)
-      float y[2][8];
-      acc_pieces(acc, g, y);
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int c = cbase + 8 * (2 * k + g);
-        const int o0 = 32 * ot + 8 * (2 * k + g);
-        const int hh = c / a.dh, d0 = c - hh * a.dh;
-        const int64_t blk = (b * a.heads + hh) * a.flash_rows + r;  // the (b, h, r) block
-        bf16x8 o;
-        if (seg == 0) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] = (bf16)((y[k][e] + obias(o0 + e, a.q_bias, c + e)) * a.q_scale);
-          *reinterpret_cast<bf16x8*>(a.q + (blk * a.np + j) * a.dh + d0) = o;
-        } else if (seg == 1) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] = (bf16)y[k][e];
-          *reinterpret_cast<bf16x8*>(a.k + (blk * a.np + j) * a.dh + d0) = o;
-        } else if (j < a.n) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            o[e] = (bf16)sigmoid_scaled((y[k][e] + obias(o0 + e, a.gate_b, c + e) + a.gate_bias) * -kLog2e);
-          *reinterpret_cast<bf16x8*>(a.gate + (bn * a.n + j) * cs + c) = o;
-        }
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int c = cbase + 8 * v + 4 * g;  // 4 channels of one head (dh % 4 == 0)
-      const int hh = c / a.dh, d0 = c - hh * a.dh;
-      const int64_t blk = (b * a.heads + hh) * a.flash_rows + r;  // the (b, h, r) block
-      float y[4] = {acc[4 * v], acc[4 * v + 1], acc[4 * v + 2], acc[4 * v + 3]};
-      if (seg == 2) {
-        const int pos = vkey_pos(j);
-        if (stage) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) stage[stage_row(8 * v + 4 * g + e) * 32 + (pos & 31)] = (bf16)y[e];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            a.vt[blk * a.dh * a.np + (pos >> 5) * 32 * a.dh + (d0 + e) * 32 + (pos & 31)] = (bf16)y[e];
-        }
-      }
-    }
-    if (seg == 2 && stage) {
-      // the tile's 32 v^T rows (tile-local channel r) of this run of 32 positions: lane L
-      // writes pieces L and L + 64 (row piece / 4, 8 positions each)
-      __builtin_amdgcn_wave_barrier();
-      const int lane = 32 * g + (int)(m - tr->m0);
-      const int jt = (int)tr->rem0;
-      const int64_t bt = tr->b;
-      const int rt = tr->r;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int piece = lane + 64 * u, r = piece >> 2, part = piece & 3;
-        const int c = cbase + r, hh = c / a.dh, d = c - hh * a.dh;
-        const int64_t blk = (bt * a.heads + hh) * a.flash_rows + rt;
-        // (v^T blocked by 32 keys; jt is a multiple of 32)
-        *reinterpret_cast<bf16x8*>(a.vt + blk * a.dh * a.np + jt * a.dh + d * 32 + 8 * part) =
-            *reinterpret_cast<const bf16x8*>(stage + stage_row(r) * 32 + 8 * part);
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-  } else if (EPI == kEpiApb) {
+  if (EPI == kEpiApb) {
     const int cs = apb_width(a);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -331,30 +219,9 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
     }
   } else if (EPI == kEpiPwa) {
     const int hd = a.O / 2;
-    const int64_t bs = m / a.n;  // b S + s
-    const int j = (int)(m - bs * a.n);
+    const int64_t bs = m / a.np;  // b S + s
+    const int j = (int)(m - bs * a.np);
     const int64_t b = bs / a.depth, srow = bs - b * a.depth;
-    if (seg == 0 && stage) {
-      // v^T: the tile's 32 channel rows of this run of 32 tokens (n % 32 == 0), transposed
-      // through the wave's LDS tile and written as 16-byte pieces of 64-byte runs
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) stage[stage_row(8 * v + 4 * g + e) * 32 + (j & 31)] = (bf16)acc[4 * v + e];
-      __builtin_amdgcn_wave_barrier();
-      const int lane = 32 * g + (int)(m - tr->m0);
-      const int64_t bt = tr->q / a.depth, st = tr->q - bt * a.depth;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int piece = lane + 64 * u, r = piece >> 2, part = piece & 3;
-        const int c = cbase + r, hh = c / a.dh, d = c - hh * a.dh;
-        *reinterpret_cast<bf16x8*>(a.vt + (((bt * a.heads + hh) * a.depth + st) * a.dh + d) * a.np +
-                                   tr->rem0 + 8 * part) =
-            *reinterpret_cast<const bf16x8*>(stage + stage_row(r) * 32 + 8 * part);
-      }
-      __builtin_amdgcn_wave_barrier();
-      return;
-    }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int c = cbase + 8 * v + 4 * g;  // 4 channels of one head (dh % 4 == 0)
@@ -364,10 +231,10 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
         bf16* dst = a.vt + (((b * a.heads + hh) * a.depth + srow) * a.dh + d0) * a.np + j;
 #pragma unroll
         for (int e = 0; e < 4; ++e) dst[(int64_t)e * a.np] = (bf16)y[e];
-      } else {
+      } else if (j < a.n) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = sigmoid_scaled(-kLog2e * y[e]);
-        store4(a.gate + m * hd + c, y[0], y[1], y[2], y[3]);
+        store4(a.gate + (bs * a.n + j) * hd + c, y[0], y[1], y[2], y[3]);
       }
     }
   } else if (EPI == kEpiOpm) {
@@ -379,42 +246,18 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
     const float* bias = seg == 0 ? a.bias0 : a.bias1;
     const int hd = a.O / 2;  // channels a side (32; Chai-1's grouped form 64)
     bf16* dst = (seg == 0 ? a.lt : a.rt) + bj * hd * a.sp + s;
-    if (stage) {
-      // the tile's 32 channel rows of this run of 32 MSA rows, transposed through the wave's
-      // LDS tile and written as 16-byte pieces of 64-byte runs (lane L: pieces L and L + 64)
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
+    for (int v = 0; v < 4; ++v)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int c = cbase + 8 * v + 4 * g + e;
-          stage[stage_row(8 * v + 4 * g + e) * 32 + (s & 31)] =
-              (bf16)((acc[4 * v + e] + (bias ? bias[c] : 0.f)) * keep);
-        }
-      __builtin_amdgcn_wave_barrier();
-      const int lane = 32 * g + (int)(m - tr->m0);
-      bf16* run = (seg == 0 ? a.lt : a.rt) + tr->q * hd * a.sp + tr->rem0;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int piece = lane + 64 * u, r = piece >> 2, part = piece & 3;
-        *reinterpret_cast<bf16x8*>(run + (int64_t)(cbase + r) * a.sp + 8 * part) =
-            *reinterpret_cast<const bf16x8*>(stage + stage_row(r) * 32 + 8 * part);
+      for (int e = 0; e < 4; ++e) {
+        const int c = cbase + 8 * v + 4 * g + e;
+        dst[(int64_t)c * a.sp] = (bf16)((acc[4 * v + e] + (bias ? bias[c] : 0.f)) * keep);
       }
-      __builtin_amdgcn_wave_barrier();
-    } else {
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int c = cbase + 8 * v + 4 * g + e;
-          dst[(int64_t)c * a.sp] = (bf16)((acc[4 * v + e] + (bias ? bias[c] : 0.f)) * keep);
-        }
-    }
     if (seg == 0 && cbase == 0 && g == 0) a.mt[bj * a.sp + s] = (bf16)keep;
   } else if (EPI == kEpiTrimul) {
     const int hid = a.O / 4;
     const int64_t gg = (int64_t)a.npm * a.npm;
-    const int64_t b = tr ? tr->q : m / gg;
-    const int64_t rem = tr ? tr->rem0 + (m - tr->m0) : m - b * gg;
+    const int64_t b = m / gg, rem = m - b * gg;
     const float keep = pre;  // the pair mask factor (row_pre)
     bf16* plane = (seg == 0 ? a.pa : a.pb) + b * hid * gg + rem;
 #pragma unroll
@@ -424,24 +267,11 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
         const int c = cbase + 8 * v + 4 * g + e;
         const float proj = acc[4 * v + e] * keep;  // masked before the gate, as the reference
         const bf16 y = (bf16)(proj * sigmoid_scaled(-kLog2e * acc[8 + 4 * v + e]));
-        if (stage)
-          stage[stage_row(8 * v + 4 * g + e) * 32 + (int)(m - tr->m0)] = y;
-        else
-          plane[(int64_t)c * gg] = y;
+        plane[(int64_t)c * gg] = y;
       }
-    if (stage) {
-      // the tile's 16 channel rows of 32 positions: lane L writes piece L (row L / 4)
-      __builtin_amdgcn_wave_barrier();
-      const int lane = 32 * g + (int)(m - tr->m0);
-      const int r = lane >> 2, part = lane & 3;
-      const int64_t bt = tr->q, remt = tr->rem0;
-      *reinterpret_cast<bf16x8*>((seg == 0 ? a.pa : a.pb) + bt * hid * gg + (int64_t)(cbase + r) * gg + remt +
-                                 8 * part) = *reinterpret_cast<const bf16x8*>(stage + stage_row(r) * 32 + 8 * part);
-      __builtin_amdgcn_wave_barrier();
-    }
   } else if (EPI == kEpiStoreY) {
     float y[2][8];
-    acc_pieces(acc, g, y);
+    acc_pieces(acc, y);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       bf16x8 o;
@@ -458,7 +288,7 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
       if (a.residual) rv[k] = rpre ? rpre[k] : *reinterpret_cast<const bf16x8*>(a.res + m * a.O + c);
     }
     float y[2][8];
-    acc_pieces(acc, g, y);
+    acc_pieces(acc, y);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       bf16x8 o;
@@ -508,11 +338,10 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
       bf16x8 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint32_t send = __float_as_uint(g ? y[0][e] : y[1][e]);
-        const auto sw = __builtin_amdgcn_permlane32_swap(send, send, false, false);
-        const float recv = __uint_as_float(g ? sw[0] : sw[1]);
-        o[e] = (bf16)(g ? recv : y[0][e]);
-        o[4 + e] = (bf16)(g ? y[1][e] : recv);
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[0][e]), __float_as_uint(y[1][e]),
+                                                         false, false);
+        o[e] = (bf16)__uint_as_float(sw[0]);
+        o[4 + e] = (bf16)__uint_as_float(sw[1]);
       }
       *reinterpret_cast<bf16x8*>(a.h16 + m * hid + ot * 16 + 8 * g) = o;
     } else {
@@ -528,7 +357,7 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
         rv[k] = rpre ? rpre[k] : *reinterpret_cast<const bf16x8*>(a.res + m * a.O + ot * 32 + 8 * (2 * k + g));
     }
     float y[2][8];
-    acc_pieces(acc, g, y);
+    acc_pieces(acc, y);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int c = ot * 32 + 8 * (2 * k + g);
@@ -688,6 +517,13 @@ __global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
 // bf16 hi + lo (as row_gemm); LayerNorm-fed rows of 256 as the rounded bf16 normalisation (as
 // the reference's bf16 LayerNorm output), and 512-channel (plain bf16) rows are held in one
 // register buffer, loaded after the last product of the previous tile.
+// What the generic path writes key- or row-contiguous (v^T, the contraction's channel planes, the
+// outer product's sides) is multiplied turned, D[row][output], so a lane holds one channel's
+// consecutive rows and stores 16-byte pieces without a transpose. Bound by the vector ALU
+// (LayerNorm, hi / lo split, epilogue) and the stores together; index arithmetic is kept in
+// scalar registers (TileRun), which was most of the vector work: pair 256 x 384 tokens, q / k /
+// v / gate 183 -> 158 us and trimul planes 147 -> 126; pair 64 x 4 templates 105 -> 88 and
+// 84 -> 75 us; MSA 512 x 256 value / gate 22 -> 19 us.
 // Lane (li, g) holds row li's channels (K / 2) g .. (K / 2) g + K / 2 - 1; MFMA step s takes
 // channels (K / 2) g + 8 s .. + 7 of both operands.
 // Waves per workgroup: 4, and 8 (two per SIMD, sharing a weight image of up to 154 KiB, one
@@ -696,8 +532,98 @@ __host__ __device__ constexpr int stream_waves(int K) { return K >= 256 ? 8 : 4;
 
 // LDS of one workgroup holding the weight rows of Op of the O outputs.
 size_t row_stream_lds(int K, int O, int Op) {
-  return (size_t)Op * (K + 8) * sizeof(bf16) + (size_t)(2 * K + O) * sizeof(float) +
-         (size_t)stream_waves(K) * 32 * 32 * sizeof(bf16);
+  return (size_t)Op * (K + 8) * sizeof(bf16) + (size_t)(2 * K + O) * sizeof(float);
+}
+
+// Output tiles that must stay in one part: kEpiTrimul's projection and gate tiles.
+__host__ __device__ constexpr int stream_unit(int epi) { return epi == kEpiTrimul ? 2 : 1; }
+
+// Where a 32-row tile starts: logical row (b R + r) L + rem. A wave's walk advances the digits by
+// the grid stride with adds and carries (an integer division by a runtime value is 20 to 100
+// vector instructions, and a tile has few enough products for that to be most of its time).
+struct TileRun {
+  uint32_t rem, r, b;
+};
+template <int EPI>
+__device__ __forceinline__ void run_radix(const RowGemmArgs& a, uint32_t& L, uint32_t& R) {
+  L = EPI == kEpiTrimul ? a.npm
+      : EPI == kEpiOpm  ? a.sp
+      : EPI == kEpiPwa || EPI == kEpiApbFlash ? a.np
+                                              : a.n;
+  R = EPI == kEpiTrimul ? a.npm : EPI == kEpiPwa ? a.depth : a.n;
+  L = L ? L : 1;  // (the epilogues without a row map leave n unset)
+  R = R ? R : 1;
+}
+__device__ __forceinline__ TileRun run_at(int64_t m, uint32_t L, uint32_t R) {
+  TileRun t;
+  if ((m >> 32) == 0) {
+    const uint32_t x = (uint32_t)m, q = x / L;
+    t.rem = x - q * L;
+    t.b = q / R;
+    t.r = q - t.b * R;
+  } else {
+    const int64_t q = m / L;
+    t.rem = (uint32_t)(m - q * L);
+    t.b = (uint32_t)(q / R);
+    t.r = (uint32_t)(q - (int64_t)t.b * R);
+  }
+  return t;
+}
+__device__ __forceinline__ TileRun run_add(TileRun t, const TileRun& step, uint32_t L, uint32_t R) {
+  t.rem += step.rem;
+  uint32_t carry = t.rem >= L ? 1u : 0u;
+  t.rem -= carry ? L : 0u;
+  t.r += step.r + carry;
+  carry = t.r >= R ? 1u : 0u;
+  t.r -= carry ? R : 0u;
+  t.b += step.b + carry;
+  return t;
+}
+
+// The input row of the tile's row li (rows past M, n or the depth read the last one).
+template <int EPI>
+__device__ __forceinline__ int64_t run_row(const RowGemmArgs& a, const TileRun& t, int64_t m0, int li) {
+  const int n = a.n;
+  if (EPI == kEpiOpm) {
+    const int s = min((int)t.rem + li, a.depth - 1);
+    return (int64_t)t.b * a.depth * n + t.r + (int64_t)s * n;
+  }
+  if (EPI == kEpiTrimul) {
+    const int i = min((int)t.r, n - 1), k = min((int)t.rem + li, n - 1);
+    return a.tmap == kMapGridOut ? ((int64_t)t.b * n + i) * n + k
+                                 : (int64_t)t.b * n * n + i + (int64_t)k * n;
+  }
+  if (EPI == kEpiPwa || EPI == kEpiApbFlash) {
+    const int j = min((int)t.rem + li, n - 1);
+    if (EPI == kEpiPwa || a.tmap == kMapPadKeys)
+      return ((int64_t)t.b * (EPI == kEpiPwa ? a.depth : n) + t.r) * n + j;
+    return (int64_t)t.b * n * n + t.r + (int64_t)j * n;
+  }
+  const int64_t left = a.M - 1 - m0;
+  const int l = left < li ? (int)left : li;
+  if ((EPI == kEpiApb || EPI == kEpiResid) && a.tmap == kMapPairT) {
+    uint32_t j = t.rem + l, r = t.r, b = t.b;
+    if (n >= 32) {  // at most one row of the pair ends inside the tile
+      const bool c = j >= (uint32_t)n;
+      j -= c ? (uint32_t)n : 0u;
+      r += c ? 1u : 0u;
+      const bool c2 = r >= (uint32_t)n;
+      r = c2 ? 0u : r;
+      b += c2 ? 1u : 0u;
+    } else {
+      r += j / n;
+      j %= n;
+      b += r / n;
+      r %= n;
+    }
+    return ((int64_t)b * n + j) * n + r;
+  }
+  return m0 + l;
+}
+
+// Mask bits of a tile's 32 rows at row 8 v + 4 g + e: bit set -> x, clear -> 0.
+__device__ __forceinline__ float keep_bit(float x, uint32_t bits_g, int v, int e) {
+  return __uint_as_float(__float_as_uint(x) & (uint32_t)((int32_t)(bits_g << (31 - 8 * v - e)) >> 31));
 }
 
 template <int EPI, int XSRC, int K>
@@ -713,6 +639,8 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
   // VGPRs) at the start of a row tile instead of a second input buffer
   constexpr bool GR = EPI == kEpiGateResid && K >= 256;
   constexpr bool DB = NX <= 16 && !GR;              // two input buffers (64 VGPRs each at most)
+  constexpr bool kRuns = EPI == kEpiApb || EPI == kEpiApbFlash || EPI == kEpiTrimul || EPI == kEpiOpm || EPI == kEpiPwa ||
+                         EPI == kEpiResid;
   using XT = typename std::conditional<BF, bf16x8, f32x4>::type;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int nt = a.O / 32 / (int)gridDim.y;  // output tiles of this workgroup's part
@@ -720,27 +648,40 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
   bf16* wl = reinterpret_cast<bf16*>(smem);  // [nt][32][WS]: output tiles ot0 ..
   float* lnp = reinterpret_cast<float*>(smem + (size_t)nt * 32 * WS * sizeof(bf16));  // weight, offset
   float* lb = lnp + 2 * K;  // per-output biases (row_epilogue)
-  // this wave's transpose tile (row_epilogue), for the epilogues that write position runs
-  bf16* stage = reinterpret_cast<bf16*>(lb + a.O) + (threadIdx.x >> 6) * 32 * 32;
-  const bool staged = (EPI == kEpiTrimul || EPI == kEpiOpm || (EPI == kEpiApb && a.flash_rows > 0) ||
-                       (EPI == kEpiPwa && a.n % 32 == 0)) &&
-                      a.M % 32 == 0;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // kEpiTrimul: tiles 2 p and 2 p + 1 are 32 projection rows of one side and their gate rows
+  auto trimul_pair = [&](int p, int& side, int& c0) {
+    const int pps = a.O / 128;
+    side = p >= pps ? 1 : 0;
+    c0 = (p - side * pps) * 32;
+  };
   for (int idx = tid; idx < nt * 32 * (K / 8); idx += 64 * kStreamWaves) {
     const int row = idx / (K / 8), ch = 8 * (idx % (K / 8));
-    int seg, cbase;
-    const float* wr = tile_weight_row<EPI>(a, ot0 + (row >> 5), row & 31, seg, cbase);
+    const int ot = ot0 + (row >> 5);
+    const float* wr;
+    if (EPI == kEpiTrimul) {
+      int side, c0;
+      trimul_pair(ot >> 1, side, c0);
+      wr = ((ot & 1) ? (side ? a.w3 : a.w2) : (side ? a.w1 : a.w0)) + (int64_t)(c0 + (row & 31)) * K;
+    } else {
+      int seg, cbase;
+      wr = tile_weight_row<EPI>(a, ot, row & 31, seg, cbase);
+    }
     *reinterpret_cast<bf16x8*>(wl + row * WS + ch) = cvt8(wr + ch);
   }
   for (int o = tid; o < a.O; o += 64 * kStreamWaves) {
     float v = 0.f;
-    if (EPI == kEpiApb) {
+    if (EPI == kEpiApb || EPI == kEpiApbFlash) {
       const int cs = apb_width(a), seg = o / cs, c = o - seg * cs;
       if (seg == 0 && a.q_bias) v = a.q_bias[c];
       if (seg == 3 && a.gate_b) v = a.gate_b[c];
     } else if (EPI == kEpiResid && a.bias_out) {
       v = a.bias_out[o];
+    } else if (EPI == kEpiOpm) {
+      const int hd = a.O / 2;
+      const float* bias = o < hd ? a.bias0 : a.bias1;
+      if (bias) v = bias[o < hd ? o : o - hd];
     }
     lb[o] = v;
   }
@@ -758,12 +699,20 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
   int64_t t = (int64_t)blockIdx.x * kStreamWaves + wave;
   if (t >= tiles) return;
   const float eps = XSRC == kXLn && a.eps_dev ? *a.eps_dev : a.eps;
+  uint32_t L = 1, R = 1;
+  TileRun cur{}, step{};
+  if constexpr (kRuns) {
+    run_radix<EPI>(a, L, R);
+    cur = run_at(t * 32, L, R);
+    step = run_at(stride * 32, L, R);
+  }
+  const int apb_cs = EPI == kEpiApbFlash ? apb_width(a) : 1;
+  const int dsh = EPI == kEpiApbFlash ? __builtin_ctz(a.dh) : 0;  // head widths 16, 32 or 64
 
-  // the input rows of a tile (a tile past the end re-reads the last one, so every load stays
-  // inside the input)
-  auto fetch = [&](XT* x, int64_t tile) __attribute__((always_inline)) {
-    const int64_t tt = tile < tiles ? tile : tiles - 1;
-    const int64_t row = EPI == kEpiOpm ? opm_msa_row(a, tt * 32 + li) : mapped_row(a, tt * 32 + li);
+  // the input rows of a tile, and the mask bytes of its rows (kEpiTrimul: of positions k and i;
+  // kEpiOpm: of the MSA entry), which the epilogue needs a tile later
+  auto fetch = [&](XT* x, uint32_t& keep, const TileRun& tr, int64_t m0) __attribute__((always_inline)) {
+    const int64_t row = run_row<EPI>(a, tr, m0, li);
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       if (BF)
@@ -771,15 +720,50 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
       else
         x[i] = *reinterpret_cast<const XT*>(a.x32 + row * K + KH * g + 4 * i);
     }
+    keep = 0;
+    if (EPI == kEpiTrimul) {
+      const uint8_t* mb = a.mask + (int64_t)tr.b * a.n;
+      const int i = min((int)tr.r, a.n - 1), k = min((int)tr.rem + li, a.n - 1);
+      keep = (uint32_t)mb[k] | ((uint32_t)mb[i] << 8);
+    } else if (EPI == kEpiOpm) {
+      keep = a.rows_mask[row];
+    }
   };
-  auto process = [&](XT* x, int64_t tile) __attribute__((always_inline)) {
+  auto process = [&](XT* x, uint32_t keep, const TileRun& tr, int64_t tile) __attribute__((always_inline)) {
+    const int64_t m = tile * 32 + li;
+    // rows kept by the mask, bit = row of the tile
+    uint32_t bits = ~0u;
+    if constexpr (EPI == kEpiTrimul) {
+      const bool on = (int)tr.r < a.n && (int)tr.rem + li < a.n && (keep & 0xff) && (keep >> 8);
+      bits = (uint32_t)__ballot(on);
+      if (bits == 0) {
+        // every pair of the tile is masked or padding: zeros, without the products
+        const int64_t gg = (int64_t)a.npm * a.npm;
+        const int64_t base = ((int64_t)tr.b * (a.O / 4) * a.npm + tr.r) * a.npm + tr.rem;
+        const bf16x8 o = zero8();
+        for (int u = ot0 / 2; u < (ot0 + nt) / 2; ++u) {
+          int side, c0;
+          trimul_pair(u, side, c0);
+          bf16* dst = (side ? a.pb : a.pa) + base + (int64_t)(c0 + (lane >> 2)) * gg + 8 * (lane & 3);
+          *reinterpret_cast<bf16x8*>(dst) = o;
+          *reinterpret_cast<bf16x8*>(dst + 16 * gg) = o;
+        }
+        return;
+      }
+    }
+    if constexpr (EPI == kEpiOpm) {
+      bits = (uint32_t)__ballot((int)tr.rem + li < a.depth && keep);
+      if (ot0 == 0 && g == 0)
+        a.mt[((int64_t)tr.b * a.n + tr.r) * a.sp + tr.rem + li] = (bf16)((bits >> li) & 1 ? 1.f : 0.f);
+    }
+    const uint32_t bits_g = bits >> (4 * g);
     // GR: the epilogue operands of the first GRS output tiles, loaded first: their wait then
     // comes after the normalisation and the first products, not right behind the previous
     // tile's stores (vmcnt counts stores too). Tiles GRS .. 7 reuse the slots of tiles 0, 1,
     // loaded once those are consumed (all 8 at once would exceed the register file).
     constexpr int GRS = 6;
     bf16x8 gy[GR ? GRS : 1][2], gr[GR ? GRS : 1][2];
-    const int64_t mg = tile * 32 + li < a.M ? tile * 32 + li : a.M - 1;
+    const int64_t mg = m < a.M ? m : a.M - 1;
     auto gr_load = [&](int u, bf16x8 (&yv)[2], bf16x8 (&rv)[2]) __attribute__((always_inline)) {
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
@@ -869,29 +853,158 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
 #pragma unroll
       for (int s = 0; s < KS; ++s) split8(x[2 * s], x[2 * s + 1], xh[s], xl[s]);
     }
-    const int64_t m = tile * 32 + li;
-    const float pre = m < a.M ? row_pre<EPI>(a, m) : 0.f;
-    const TileRun tr = staged ? tile_run<EPI>(a, tile * 32) : TileRun{};
-    auto out_tile = [&](int ot, const bf16x8* rpre, const bf16x8* ypre = nullptr) __attribute__((always_inline)) {
-      const bf16* wt = wl + ((ot - ot0) * 32 + li) * WS + KH * g;
+    // one output tile: D[output][row], or turned, D[row][output]
+    auto product = [&](int u, bool turned) __attribute__((always_inline)) {
+      const bf16* wt = wl + (u * 32 + li) * WS + KH * g;
       f32x16 acc = zero16();
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         const bf16x8 w = *reinterpret_cast<const bf16x8*>(wt + 8 * s);
         if constexpr (LO) {
-          acc = mfma32(w, xl[s], acc);
-          acc = mfma32(w, xh[s], acc);
-        } else {
-          acc = mfma32(w, x[s], acc);
+          acc = turned ? mfma32(xl[s], w, acc) : mfma32(w, xl[s], acc);
+          acc = turned ? mfma32(xh[s], w, acc) : mfma32(w, xh[s], acc);
+        } else if constexpr (BF) {
+          acc = turned ? mfma32(x[s], w, acc) : mfma32(w, x[s], acc);
         }
       }
-      int seg, cbase;
-      (void)tile_weight_row<EPI>(a, ot, li, seg, cbase);
-      if (m < a.M)
-        row_epilogue<EPI>(a, acc, m, ot, seg, cbase, g, lb, pre, staged ? stage : nullptr,
-                          staged ? &tr : nullptr, rpre, ypre);
+      return acc;
     };
-    if (EPI == kEpiResid && a.residual && nt <= 4) {
+    // 16 rows of 32 channels as 16-byte pieces of 8 rows: channel li's pieces 2 k + g
+    auto store_rows = [&](bf16* dst, const f32x16& y) __attribute__((always_inline)) {
+      float p[2][8];
+      acc_pieces(y, p);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (bf16)p[k][e];
+        *reinterpret_cast<bf16x8*>(dst + 16 * k + 8 * g) = o;
+      }
+    };
+    auto out_tile = [&](int ot, const bf16x8* rpre, const bf16x8* ypre = nullptr) __attribute__((always_inline)) {
+      const f32x16 acc = product(ot - ot0, false);
+      int seg = 0, cbase = 0;
+      if (EPI == kEpiApb) (void)tile_weight_row<EPI>(a, ot, li, seg, cbase);
+      if (m < a.M) row_epilogue<EPI>(a, acc, m, ot, seg, cbase, g, lb, 0.f, rpre, ypre);
+    };
+    if constexpr (EPI == kEpiTrimul) {
+      // channel planes: lane li holds channel c0 + li, its registers the tile's positions
+      const int64_t gg = (int64_t)a.npm * a.npm;
+      const int64_t at = ((int64_t)tr.b * (a.O / 4) * a.npm + tr.r) * a.npm + tr.rem + li * gg;
+#pragma unroll 1
+      for (int u = 0; u < nt; u += 2) {
+        f32x16 y = product(u, true);
+        const f32x16 gate = product(u + 1, true);
+        if (bits != ~0u) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[4 * v + e] = keep_bit(y[4 * v + e], bits_g, v, e);
+        }
+        // (masked before the gate, as the reference)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) y[r] *= sigmoid_scaled(-kLog2e * gate[r]);
+        int side, c0;
+        trimul_pair((ot0 + u) >> 1, side, c0);
+        store_rows((side ? a.pb : a.pa) + c0 * gg + at, y);
+      }
+    } else if constexpr (EPI == kEpiOpm) {
+      // MSA rows contiguous per channel: lane li holds channel c0 + li
+      const int hd = a.O / 2;  // channels a side (32; Chai-1's grouped form 64)
+      const int64_t at = (((int64_t)tr.b * a.n + tr.r) * hd + li) * a.sp + tr.rem;
+#pragma unroll 1
+      for (int ot = ot0; ot < ot0 + nt; ++ot) {
+        f32x16 y = product(ot - ot0, true);
+        const float bias = lb[ot * 32 + li];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[4 * v + e] = keep_bit(y[4 * v + e] + bias, bits_g, v, e);
+        const int side = ot * 32 >= hd ? 1 : 0;
+        store_rows((side ? a.rt : a.lt) + at + (int64_t)(ot * 32 - side * hd) * a.sp, y);
+      }
+    } else if constexpr (EPI == kEpiPwa) {
+      // value tiles: v^T keys contiguous per channel; gate tiles: token rows
+      const int hd = a.O / 2;
+      const int64_t bs = (int64_t)tr.b * a.depth + tr.r;
+      const uint32_t inv = ((1u << 24) + a.dh - 1) / a.dh;  // c / dh = (c inv) >> 24 for c, dh <= 768
+      const int j = (int)tr.rem + li;
+#pragma unroll 1
+      for (int ot = ot0; ot < ot0 + nt; ++ot) {
+        if (ot * 32 < hd) {
+          const f32x16 y = product(ot - ot0, true);
+          const int c = ot * 32 + li, hh = (int)(((uint32_t)c * inv) >> 24), d = c - hh * a.dh;
+          store_rows(a.vt + ((((int64_t)tr.b * a.heads + hh) * a.depth + tr.r) * a.dh + d) * a.np + tr.rem, y);
+        } else {
+          const f32x16 acc = product(ot - ot0, false);
+          float y[2][8];
+          acc_pieces(acc, y);
+          if (j < a.n) {
+            bf16* dst = a.gate + (bs * a.n + tr.rem) * hd + li * hd + (ot * 32 - hd);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              bf16x8 o;
+#pragma unroll
+              for (int e = 0; e < 8; ++e) o[e] = (bf16)sigmoid_scaled(-kLog2e * y[k][e]);
+              *reinterpret_cast<bf16x8*>(dst + 16 * k + 8 * g) = o;
+            }
+          }
+        }
+      }
+    } else if constexpr (EPI == kEpiApbFlash) {
+      // the flash core's layouts: everything but the lane's row and piece is uniform
+      const int j = (int)tr.rem + li;
+#pragma unroll 1
+      for (int ot = ot0; ot < ot0 + nt; ++ot) {
+        const int o0 = ot * 32;
+        const int seg = (o0 >= apb_cs ? 1 : 0) + (o0 >= 2 * apb_cs ? 1 : 0) + (o0 >= 3 * apb_cs ? 1 : 0);
+        const int cbase = o0 - seg * apb_cs;
+        const int64_t head = (int64_t)a.flash_rows * a.np * a.dh;  // elements of one (b, h)
+        if (seg == 2) {
+          // v^T, turned: lane li is channel cbase + li and its registers 8 h .. 8 h + 7 are 8
+          // consecutive key slots of the core's order, 16 h + 8 g ..
+          const f32x16 acc = product(ot - ot0, true);
+          const int hh = cbase >> dsh, c = (cbase & (a.dh - 1)) + li;
+          bf16* dst = a.vt + ((int64_t)tr.b * a.heads + hh) * head + ((int64_t)tr.r * a.np + tr.rem) * a.dh +
+                      (c >> dsh) * head + (c & (a.dh - 1)) * 32 + 8 * g;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            bf16x8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = (bf16)acc[8 * h + e];
+            *reinterpret_cast<bf16x8*>(dst + 16 * h) = o;
+          }
+          continue;
+        }
+        const f32x16 acc = product(ot - ot0, false);
+        float y[2][8];
+        acc_pieces(acc, y);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int c = cbase + 16 * k;  // this lane: channels c + 8 g ..
+          bf16x8 o;
+          if (seg == 3) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              o[e] = (bf16)sigmoid_scaled((y[k][e] + lb[o0 + 16 * k + 8 * g + e] + a.gate_bias) * -kLog2e);
+            if (j < a.n)
+              *reinterpret_cast<bf16x8*>(a.gate + (((int64_t)tr.b * a.n + tr.r) * a.n + tr.rem) * apb_cs + c +
+                                         li * apb_cs + 8 * g) = o;
+            continue;
+          }
+          if (seg == 0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = (bf16)((y[k][e] + lb[o0 + 16 * k + 8 * g + e]) * a.q_scale);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = (bf16)y[k][e];
+          }
+          *reinterpret_cast<bf16x8*>((seg == 0 ? a.q : a.k) + ((int64_t)tr.b * a.heads + (c >> dsh)) * head +
+                                     ((int64_t)tr.r * a.np + tr.rem) * a.dh + (c & (a.dh - 1)) + li * a.dh +
+                                     8 * g) = o;
+        }
+      }
+    } else if (EPI == kEpiResid && a.residual && nt <= 4) {
       // the residual of every output tile is loaded before the tile's first store: a wait
       // for a load issued after stores would wait for those stores too (vmcnt counts both)
       bf16x8 rv[4][2];
@@ -943,29 +1056,41 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
     }
   };
 
+  // the tile after t, or t again past the last one (its rows are loaded and dropped)
+  auto next = [&](const TileRun& tr) __attribute__((always_inline)) {
+    return kRuns && t + stride < tiles ? run_add(tr, step, L, R) : tr;
+  };
+  auto next_m = [&]() __attribute__((always_inline)) { return (t + stride < tiles ? t + stride : t) * 32; };
+  uint32_t k0, k1;
   if constexpr (DB) {
     // two register buffers used in turn: the next tile's rows load while the current one is
     // processed
     XT x0[NX], x1[NX];
-    fetch(x0, t);
+    fetch(x0, k0, cur, t * 32);
     while (true) {
-      fetch(x1, t + stride);
-      process(x0, t);
+      TileRun nx = next(cur);
+      fetch(x1, k1, nx, next_m());
+      process(x0, k0, cur, t);
       t += stride;
       if (t >= tiles) break;
-      fetch(x0, t + stride);
-      process(x1, t);
+      cur = nx;
+      nx = next(cur);
+      fetch(x0, k0, nx, next_m());
+      process(x1, k1, cur, t);
       t += stride;
       if (t >= tiles) break;
+      cur = nx;
     }
   } else {
     XT x0[NX];
-    fetch(x0, t);
+    fetch(x0, k0, cur, t * 32);
     while (true) {
-      process(x0, t);
+      process(x0, k0, cur, t);
+      const TileRun nx = next(cur);
       t += stride;
       if (t >= tiles) break;
-      fetch(x0, t);
+      cur = nx;
+      fetch(x0, k0, cur, t * 32);
     }
   }
 }
@@ -1382,23 +1507,24 @@ void launch_row_gemm_t(const RowGemmArgs& a, hipStream_t stream) {
 // Tile shapes: the LayerNorm-fed GEMMs give each workgroup several output tiles (the tile is
 // normalised once per workgroup); the fp32-fed ones split k 8 ways when k is long, and give the
 // waves separate output tiles when k has fewer groups than waves.
-// Output parts: halve the weight rows per workgroup until a workgroup's LDS is at most 72 KiB
-// (two workgroups of 4 waves per CU), as long as the parts stay whole tiles. Measured on the
+// Output parts: the fewest equal parts of whole tiles whose weight rows keep a workgroup's LDS at
+// or below 72 KiB (two workgroups of 4 waves per CU). Measured on the
 // template stacks: splitting at 56 KiB instead (three workgroups per CU, the input read twice
 // for 384 outputs) was 2.5% slower per block. Rows of 256 channels or more: at most 160 KiB
 // (one workgroup of 8 waves per CU), so that each part re-reads and re-normalises the input
 // rows as few times as possible.
 size_t row_stream_lds_cap(int K) { return (K >= 256 ? 160 : 72) * 1024; }
-int row_stream_parts(int K, int O) {
+int row_stream_parts(int K, int O, int unit) {
+  const int units = O / 32 / unit;
   int parts = 1;
-  while (row_stream_lds(K, O, O / parts) > row_stream_lds_cap(K) && (O / 32) % (2 * parts) == 0) parts *= 2;
+  while (parts < units && (units % parts != 0 || row_stream_lds(K, O, O / parts) > row_stream_lds_cap(K))) ++parts;
   return parts;
 }
 
 template <int EPI, int XSRC, int K>
 void launch_row_stream_t(const RowGemmArgs& a, hipStream_t stream) {
   constexpr int kStreamWaves = stream_waves(K);
-  const int parts = row_stream_parts(K, a.O);
+  const int parts = row_stream_parts(K, a.O, stream_unit(EPI));
   const size_t lds = row_stream_lds(K, a.O, a.O / parts);
   auto kernel = row_stream<EPI, XSRC, K>;
   if (lds > 65536)
@@ -1418,7 +1544,7 @@ bool launch_row_stream(const RowGemmArgs& a, hipStream_t stream) {
   if (a.K != 64 && a.K != 128 && !(XSRC != kXF32 && a.K == 256) && !(XSRC == kXBf16 && a.K == 512))
     return false;
   const size_t cap = a.K >= 256 ? 160 * 1024 : 80 * 1024;
-  if (row_stream_lds(a.K, a.O, a.O / row_stream_parts(a.K, a.O)) > cap) return false;
+  if (row_stream_lds(a.K, a.O, a.O / row_stream_parts(a.K, a.O, stream_unit(EPI))) > cap) return false;
   if (a.K == 64) {
     launch_row_stream_t<EPI, XSRC, 64>(a, stream);
   } else if (a.K == 128) {
@@ -1435,6 +1561,10 @@ bool launch_row_stream(const RowGemmArgs& a, hipStream_t stream) {
 void launch_row_gemm(const RowGemmArgs& a, int epi, int xsrc, hipStream_t stream) {
   // short rows of the pair path: the streaming kernel (false: not a case it takes)
   if (xsrc == kXLn) {
+    if (epi == kEpiApb && a.flash_rows > 0) {  // (pair widths 64, 128, 256: always a case)
+      (void)launch_row_stream<kEpiApbFlash, kXLn>(a, stream);
+      return;
+    }
     if (epi == kEpiApb && launch_row_stream<kEpiApb, kXLn>(a, stream)) return;
     if (epi == kEpiTrimul && launch_row_stream<kEpiTrimul, kXLn>(a, stream)) return;
     if (epi == kEpiStoreY && launch_row_stream<kEpiStoreY, kXLn>(a, stream)) return;

@@ -286,18 +286,13 @@ __device__ __forceinline__ void transition_tile(bf16* XR, const TransitionChunk*
           own[t][d] = __builtin_bit_cast(uint32_t, p);
         }
       }
-      uint32_t recv[2];
+      uint32_t v[4];
 #pragma unroll
       for (int d = 0; d < 2; ++d) {
-        const uint32_t send = g ? own[0][d] : own[1][d];
-        const auto sw = __builtin_amdgcn_permlane32_swap(send, send, false, false);
-        recv[d] = g ? sw[0] : sw[1];
+        const auto sw = __builtin_amdgcn_permlane32_swap(own[0][d], own[1][d], false, false);
+        v[d] = sw[0];
+        v[2 + d] = sw[1];
       }
-      uint32_t v[4];
-      v[0] = g ? recv[0] : own[0][0];
-      v[1] = g ? recv[1] : own[0][1];
-      v[2] = g ? own[1][0] : recv[0];
-      v[3] = g ? own[1][1] : recv[1];
       // (regular stores: L2 merges the eight 32-byte pieces of a row into full lines)
       if (r < rows)
         *reinterpret_cast<u32x4*>(out + r * C + 32 * ot + 8 * (2 * mp + g)) =

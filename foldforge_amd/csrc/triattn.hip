@@ -645,7 +645,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_bias(FlashArgs a) {
       // 16-byte pieces of 8 head channels (half the store instructions of 8-byte ones): half g
       // ends with pieces g and 2 + g of the tile's 32 rows
       float y[2][8];
-      acc_pieces(O[rr][hh], g, y);
+      acc_pieces(O[rr][hh], y);
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int d0 = 32 * hh + 8 * (2 * k + g);

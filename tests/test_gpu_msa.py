@@ -74,6 +74,18 @@ def test_msa_pair_weighted_averaging_matches_oracle(cm, heads, dh, depth, n, len
     _check(full, want + msa.double(), "msa_pwa residual")
 
 
+@pytest.mark.parametrize("heads,dh", [(1, 256), (3, 64)])
+@pytest.mark.parametrize("n", [1, 31, 65])
+def test_msa_pair_weighted_averaging_wide_heads_and_broken_key_runs(heads, dh, n):
+    """Heads of 64 channels and more, and tokens that end inside a 32-key run of the values."""
+    msa, z, mask = _inputs(3, n, 64, [n], seed=n + dh)
+    mod = _pwa(64, heads, dh, seed=dh)
+    got = hip_delta(mod, msa.cuda(), z.cuda(), mask.cuda()).cpu()
+    want = ps.msa_pair_weighted_averaging(msa, z, mask, mod.state_dict(), n_head=heads,
+                                          dtype=torch.float64) - msa.double()
+    _check(got, want, f"msa_pwa {heads}x{dh} n={n}")
+
+
 def test_msa_pair_weighted_averaging_masking_is_exact_and_empty_rows_are_zero():
     depth, n, length = 4, 96, 61
     msa, z, mask = _inputs(depth, n, 64, [length, 0], seed=11)

@@ -226,3 +226,21 @@ def test_transition_of_64_channels(rows, factor):
     kernels.transition(inplace, ln_weight=m.ln_in.weight, ln_bias=m.ln_in.bias, expand_a=m.expand_a.weight,
                        expand_b=m.expand_b.weight, squeeze=m.squeeze.weight, out=inplace)
     assert torch.equal(inplace, got)
+
+
+@pytest.mark.parametrize("c,h", [(64, 64), (256, 256)])
+@pytest.mark.parametrize("n,lengths", [(1, [1]), (31, [31, 7]), (97, [97, 20])])
+def test_streaming_projections_at_row_and_mask_edges(c, h, n, lengths):
+    """The projections' tile walk where it can go wrong: rows shorter than a 32-row tile, rows that
+    end inside one, and a batch element whose mask leaves whole tiles without a pair."""
+    z, mask = _pair(n, c, lengths, seed=n + c)
+    for outgoing in (True, False):
+        m = randomise(factories.triangle_multiplication(c, outgoing=outgoing, d_hidden=h), seed=n + h).cuda()
+        m.set_backend("hip")
+        want = ps.triangle_multiplication(z, mask, m.state_dict(), outgoing=outgoing, dtype=torch.float64) - z.double()
+        _check(hip_delta(m, z.cuda(), mask.cuda()).cpu(), want, _pairs(mask), f"trimul c={c} n={n} outgoing={outgoing}")
+    for starting in (True, False):
+        m = randomise(factories.triangle_attention(c, 4, starting=starting, model="af3", d_hidden=c), seed=n).cuda()
+        m.set_backend("hip")
+        want = ps.triangle_attention(z, mask, m.state_dict(), n_head=4, starting=starting, dtype=torch.float64) - z.double()
+        _check(hip_delta(m, z.cuda(), mask.cuda()).cpu(), want, _pairs(mask), f"triattn c={c} n={n} starting={starting}")
