@@ -102,50 +102,16 @@ struct Carver {
   }
 };
 
-// Workgroup row y converts segment y (the row past the last segment converts the mask), so
-// the segments' loads are in flight together rather than one segment after another.
-__global__ __launch_bounds__(256) void pack_bf16(PackJob job) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if ((int)blockIdx.y < job.nseg) {
-    const PackSeg sg = job.seg[blockIdx.y];
-    for (int64_t i = first; i < sg.n; i += stride) {
-      const int64_t j = sg.swap23 ? (i & ~int64_t(12)) | ((i & 4) << 1) | ((i & 8) >> 1) : i;
-      sg.dst[i] = (bf16)(sg.src ? sg.src[j] * sg.scale : 0.f);
-    }
-  } else if (job.mask) {
-    // one workgroup per batch element: its mask row, and the number of key stages up to the
-    // last real key
-    __shared__ int last;
-    for (int b = blockIdx.x; b < job.batch; b += gridDim.x) {
-      if (threadIdx.x == 0) last = -1;
-      __syncthreads();
-      int mine = -1;
-      for (int s = threadIdx.x; s < job.np; s += blockDim.x) {
-        const bool real = s < job.n && job.mask[(int64_t)b * job.n + s] != 0;
-        job.maskf[(int64_t)b * job.np + s] = real ? 1.f : 0.f;
-        if (real) mine = s;
-      }
-      if (mine >= 0) atomicMax(&last, mine);
-      __syncthreads();
-      if (threadIdx.x == 0 && job.kstages) job.kstages[b] = (last + 32) / 32;
-      __syncthreads();
-    }
-  }
+__global__ __launch_bounds__(256) void pack_bf16(const float* __restrict__ src, bf16* __restrict__ dst,
+                                                 int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[i] = (bf16)src[i];
 }
 
 }  // namespace
 
-// Grid: one row of workgroups per segment (plus one for the mask), each row as wide as the
-// largest segment needs (at most 1024 workgroups); the weights of one op are a few hundred
-// thousand values, a latency-bound pass either way.
-void launch_pack(const PackJob& job, hipStream_t stream) {
-  int64_t most = job.mask ? (int64_t)job.batch * 256 : 0;  // the mask row: a workgroup per batch
-  for (int s = 0; s < job.nseg; ++s) most = job.seg[s].n > most ? job.seg[s].n : most;
-  int64_t blocks = (most + 255) / 256;
-  blocks = blocks < 1 ? 1 : blocks > 1024 ? 1024 : blocks;
-  const unsigned rows = (unsigned)job.nseg + (job.mask ? 1u : 0u);
-  pack_bf16<<<dim3((unsigned)blocks, rows < 1 ? 1u : rows), 256, 0, stream>>>(job);
+void launch_pack(const float* src, bf16* dst, int64_t n, hipStream_t stream) {
+  pack_bf16<<<dim3((unsigned)((n + 255) / 256)), 256, 0, stream>>>(src, dst, n);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -157,9 +123,9 @@ bool trimul_fused(int c, int h) { return c == 128 && h == 128; }
 bool triattn_fused(int c, int heads, int d) { return c == 128 && heads == 4 && d == 32; }
 
 struct TrimulWs {
-  bf16 *wp, *wg, *wo, *A, *B, *P, *Pt;
+  bf16 *wgo, *A, *B, *P, *Pt;
   bf16* y;  // the update before the gate (generic path, bf16)
-  float *maskf, *eps_out;
+  float* eps_out;
   int* kst;
   size_t bytes;
 };
@@ -188,23 +154,24 @@ TrimulWs trimul_ws(void* ws, int64_t batch, int64_t n, int c, int h) {
     w.bytes = cv.used;
     return w;
   }
-  w.wp = cv.take<bf16>((size_t)4 * h * c);
-  w.wg = cv.take<bf16>((size_t)c * c);
-  w.wo = cv.take<bf16>((size_t)c * h);
+  w.wgo = cv.take<bf16>((size_t)2 * 128 * 128);
+  // (callers size workspaces once: the sizes stay those of the form with every weight packed
+  // and the key mask widened, whose pieces nothing uses any more)
+  cv.used += 4 * 128 * 128 * sizeof(bf16) + up256((size_t)batch * np * sizeof(float));
   w.A = cv.take<bf16>(plane);
   w.B = cv.take<bf16>(plane);
   w.P = cv.take<bf16>(plane);
-  w.maskf = cv.take<float>((size_t)batch * np);
   w.kst = cv.take<int>((size_t)batch);
   w.bytes = cv.used;
   return w;
 }
 
 int64_t pad32(int64_t n);
+int64_t pad64(int64_t n);
 
 struct TriattnWs {
-  bf16 *wqkv, *wb, *wg, *wo, *wo_t, *q, *k, *vt, *o, *gate, *tbuf, *ogb;
-  float *bias, *og, *maskf;
+  bf16 *wgo, *q, *k, *vt, *o, *gate, *tbuf, *ogb;
+  float *bias, *og;
   int* kst;
   size_t bytes;
 };
@@ -249,17 +216,14 @@ TriattnWs triattn_ws(void* ws, int64_t batch, int64_t n, int c, int heads, int d
     w.bytes = cv.used;
     return w;
   }
-  w.wqkv = cv.take<bf16>((size_t)3 * hd * c);
-  w.wb = cv.take<bf16>((size_t)32 * c);
-  w.wg = cv.take<bf16>((size_t)hd * c);
-  w.wo = cv.take<bf16>((size_t)c * hd);
-  if (form == kTriattnDual) w.wo_t = cv.take<bf16>((size_t)c * hd);
+  w.wgo = cv.take<bf16>((size_t)(form == kTriattnDual ? 3 : 2) * 128 * 128);
+  // (the size of the form with every weight packed and the mask widened: see trimul_ws)
+  cv.used += (3 * 128 + 32) * 128 * sizeof(bf16) + up256((size_t)batch * np * sizeof(float));
   w.q = cv.take<bf16>((size_t)batch * heads * np * np * d);
   w.k = cv.take<bf16>((size_t)batch * heads * np * np * d);
   w.vt = cv.take<bf16>((size_t)batch * heads * np * np * d);
   w.bias = cv.take<float>((size_t)batch * heads * np * np);
   w.o = cv.take<bf16>((size_t)batch * n * n * hd);
-  w.maskf = cv.take<float>((size_t)batch * np);
   w.kst = cv.take<int>((size_t)batch);
   w.bytes = cv.used;
   return w;
@@ -546,7 +510,8 @@ int32_t ffk_triangle_multiplication(
     p.w1 = w_right;
     p.w2 = w_left_gate;
     p.w3 = w_right_gate;
-    p.M = batch * np * np;
+    p.gk = (int)pad64(n);
+    p.M = batch * n * p.gk;
     p.K = d_pair;
     p.O = 4 * d_hidden;
     p.n = (int)n;
@@ -556,7 +521,7 @@ int32_t ffk_triangle_multiplication(
     p.pa = w.A;
     p.pb = w.B;
     launch_row_gemm(p, kEpiTrimul, kXLn, st);
-    launch_trimul_contract(w.A, w.B, w.P, batch * d_hidden, (int)np, st);
+    launch_trimul_contract(w.A, w.B, w.P, batch * d_hidden, (int)n, (int)np, st);
     if (trimul_planes(batch, n, d_pair, d_hidden)) {
       TrimulPlanesArgs r{};
       r.planes = w.P;
@@ -607,23 +572,6 @@ int32_t ffk_triangle_multiplication(
     launch_row_gemm(f, kEpiGateResid, kXLn, st);
     return check_launch("triangle_multiplication");
   }
-  const int64_t hc = (int64_t)d_hidden * d_pair;
-  PackJob job{};
-  // gate projections pre-multiplied by -log2(e): the kernels' sigmoid is 1 / (1 + 2^y)
-  job.seg[0] = {w_left, w.wp, hc, 1.f};
-  job.seg[1] = {w_left_gate, w.wp + hc, hc, -kLog2e};
-  job.seg[2] = {w_right, w.wp + 2 * hc, hc, 1.f};
-  job.seg[3] = {w_right_gate, w.wp + 3 * hc, hc, -kLog2e};
-  job.seg[4] = {w_gate, w.wg, (int64_t)d_pair * d_pair, -kLog2e};
-  job.seg[5] = {w_out, w.wo, (int64_t)d_pair * d_hidden, 1.f};
-  job.nseg = 6;
-  job.mask = key_mask;
-  job.maskf = w.maskf;
-  job.kstages = w.kst;
-  job.batch = (int)batch;
-  job.n = (int)n;
-  job.np = (int)pad128(n);
-  launch_pack(job, st);
   TrimulArgs a;
   a.z = static_cast<const bf16*>(z);
   a.mask = key_mask;
@@ -631,13 +579,16 @@ int32_t ffk_triangle_multiplication(
   a.ln_b = ln_pair_b;
   a.lno_w = ln_out_w;
   a.lno_b = ln_out_b;
-  a.wp = w.wp;
-  a.wg = w.wg;
-  a.wo = w.wo;
+  a.w_left = w_left;
+  a.w_right = w_right;
+  a.w_left_gate = w_left_gate;
+  a.w_right_gate = w_right_gate;
+  a.w_gate = w_gate;
+  a.w_out = w_out;
+  a.wgo = w.wgo;
   a.A = w.A;
   a.B = w.B;
   a.P = w.P;
-  a.maskf = w.maskf;
   a.kstages = w.kst;
   a.out = static_cast<bf16*>(out);
   a.batch = (int)batch;
@@ -651,7 +602,7 @@ int32_t ffk_triangle_multiplication(
   return check_launch("triangle_multiplication");
 }
 
-// The pack and the launches of the fused-width triangle attention (d_pair 128, 4 x 32) on a
+// The launches of the fused-width triangle attention (d_pair 128, 4 x 32) on a
 // carved workspace; project_only: the projection and the flash core only (w.o holds the
 // attention output in z frame, nothing is written to out).
 static void triattn_fused_launch(const TriattnWs& w, const void* z, const uint8_t* key_mask,
@@ -662,39 +613,19 @@ static void triattn_fused_launch(const TriattnWs& w, const void* z, const uint8_
                           void* out, int64_t batch, int64_t n, int n_head, int d_head,
                           int starting, int transposed_bias, int form, int residual, float eps,
                           bool project_only, hipStream_t st) {
-  const int d_pair = 128;
-  const int hd = n_head * d_head;
-  const int64_t m = (int64_t)hd * d_pair;
-  const float qscale = kLog2e / sqrtf((float)d_head);
-  PackJob job{};
-  job.seg[0] = {w_query, w.wqkv, m, qscale};
-  job.seg[1] = {w_key, w.wqkv + m, m, 1.f};
-  job.seg[2] = {w_value, w.wqkv + 2 * m, m, 1.f};
-  job.seg[3] = {w_bias, w.wb, (int64_t)n_head * d_pair, kLog2e};
-  job.seg[4] = {nullptr, w.wb + (int64_t)n_head * d_pair, (int64_t)(32 - n_head) * d_pair, 0.f};
-  // (the fused output-transition kernel packs the gate and output weights itself)
-  job.seg[5] = {w_gate, w.wg, project_only ? 0 : m, -kLog2e};  // sigmoid(x) = 1 / (1 + 2^(-log2(e) x))
-  job.seg[6] = {w_out, w.wo, project_only ? 0 : m, 1.f};
-  job.seg[7] = {w_out_t, w.wo_t, form == kTriattnDual ? m : 0, 1.f};
-  job.nseg = 8;
-  job.mask = key_mask;
-  job.maskf = w.maskf;
-  job.kstages = w.kst;
-  job.batch = (int)batch;
-  job.n = (int)n;
-  job.np = (int)pad128(n);
-  launch_pack(job, st);
   TriattnArgs a{};
   a.z = static_cast<const bf16*>(z);
   a.mask = key_mask;
-  a.maskf = w.maskf;
   a.kstages = w.kst;
   a.ln_w = ln_pair_w;
   a.ln_b = ln_pair_b;
-  a.wqkv = w.wqkv;
-  a.wb = w.wb;
-  a.wg = w.wg;
-  a.wo = w.wo;
+  a.w_query = w_query;
+  a.w_key = w_key;
+  a.w_value = w_value;
+  a.q_scale = kLog2e / sqrtf((float)d_head);
+  a.w_bias = w_bias;
+  a.w_gate = w_gate;
+  a.w_out = w_out;
   a.q = w.q;
   a.k = w.k;
   a.vt = w.vt;
@@ -703,7 +634,8 @@ static void triattn_fused_launch(const TriattnWs& w, const void* z, const uint8_
   a.bg = b_gate;
   a.bo = b_out;
   a.form = form;
-  a.wo_t = w.wo_t;
+  a.w_out_t = w_out_t;
+  a.wgo = w.wgo;
   a.bo_t = b_out_t;
   a.tbuf = w.tbuf;
   a.out = static_cast<bf16*>(out);
@@ -1518,10 +1450,7 @@ int32_t ffk_outer_product_mean_grouped(
   p.mt = w.mt;
   launch_row_gemm(p, kEpiOpm, kXLn, st);
 
-  PackJob job{};
-  job.seg[0] = {w_out, w.wp, (int64_t)d_pair * 512, 1.f};
-  job.nseg = 1;
-  launch_pack(job, st);
+  launch_pack(w_out, w.wp, (int64_t)d_pair * 512, st);
 
   OpmGroupedArgs o;
   o.lt = w.lt;

@@ -197,11 +197,32 @@ struct WFrag {
   bf16x8 k[8];
 };
 
-__device__ __forceinline__ void load_wfrag(WFrag& w, const bf16* __restrict__ W, int first_row,
-                                           int li, int g) {
-  const bf16* row = W + (int64_t)(first_row + li) * 128 + 8 * g;
+// From weights packed in fragment order (pack_wfrag): block b = 32 rows.
+__device__ __forceinline__ void load_wfrag(WFrag& w, const bf16* __restrict__ W, int b, int lane) {
 #pragma unroll
-  for (int kk = 0; kk < 8; ++kk) w.k[kk] = ld8(row + 16 * kk);
+  for (int kk = 0; kk < 8; ++kk) w.k[kk] = ld8(W + ((b * 8 + kk) * 64 + lane) * 8);
+}
+
+// kstages[b] of the batch elements b = first, first + step, ...: the 32-key stages up to the
+// last real key of mask [batch][n] (0 when there is none). One wave.
+__device__ __forceinline__ void count_stages(const uint8_t* __restrict__ mask, int n, int batch, int first,
+                                             int step, int lane, int* __restrict__ kstages) {
+  for (int b = first; b < batch; b += step) {
+    int last = -1;
+#pragma unroll 4
+    for (int s0 = 0; s0 < n; s0 += 64) {
+      const int s = s0 + lane;
+      const uint64_t real = __ballot(s < n && mask[(int64_t)b * n + (s < n ? s : n - 1)] != 0);
+      if (real) last = s0 + 63 - __builtin_clzll(real);
+    }
+    if (lane == 0) kstages[b] = (last + 32) / 32;
+  }
+}
+
+// Mask bits of a tile's 32 rows at row 8 v + 4 g + e (bits_g: the 32 bits shifted right by 4 g):
+// bit set -> x, clear -> 0.
+__device__ __forceinline__ float keep_bit(float x, uint32_t bits_g, int v, int e) {
+  return __uint_as_float(__float_as_uint(x) & (uint32_t)((int32_t)(bits_g << (31 - 8 * v - e)) >> 31));
 }
 
 // Force the loads of a fragment to complete here. Weight fragments are loaded once before a
@@ -336,6 +357,45 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // operand fetch) or the sixteen pieces of one row hit distinct banks.
 __device__ __forceinline__ int off128(int r, int k8) { return r * 128 + 8 * (k8 ^ (r & 15)); }
 
+// The same slice from the fp32 parameter [.][128], in two steps. Fetched row by row (1 KB per load
+// instruction: in fragment order a load touches 64 cache lines, and a workgroup's weights took 4 us
+// instead of 2), then rounded to bf16 times scale and turned in a wave-private 8 KB LDS tile.
+typedef float f32x4_a4 __attribute__((__vector_size__(16), aligned(4)));  // parameters: any slice
+struct WRows {
+  f32x4 v[16];
+};
+__device__ __forceinline__ void fetch_wrows(WRows& w, const float* __restrict__ W, int first_row, int lane) {
+  const float* p = W + (int64_t)(first_row + (lane >> 5)) * 128 + 4 * (lane & 31);
+#pragma unroll
+  for (int u = 0; u < 16; ++u) w.v[u] = *reinterpret_cast<const f32x4_a4*>(p + 256 * u);
+}
+__device__ __forceinline__ void turn_wrows(WFrag& w, const WRows& rows, float scale, bf16* tile, int lane) {
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    bf16x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (bf16)(rows.v[u][e] * scale);
+    *reinterpret_cast<bf16x4*>(&tile[off128(2 * u + (lane >> 5), (lane & 31) >> 1) + 4 * (lane & 1)]) = v;
+  }
+  __builtin_amdgcn_wave_barrier();  // the tile is the wave's own: LDS operations complete in order
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) w.k[kk] = ld8(&tile[off128(lane & 31, 2 * kk + (lane >> 5))]);
+  __builtin_amdgcn_wave_barrier();
+}
+
+// A [128][128] parameter for a later kernel's load_wfrag: bf16 times scale in fragment order,
+// piece idx (16 bytes) of its 2048.
+__device__ __forceinline__ void pack_wfrag(const float* __restrict__ src, float scale, bf16* __restrict__ dst,
+                                           int idx) {
+  const int lane = idx & 63, kk = (idx >> 6) & 7, cb = (idx >> 9) & 3;
+  const float* row = src + (32 * cb + (lane & 31)) * 128 + 16 * kk + 8 * (lane >> 5);
+  bf16x8 v;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = (bf16)(row[e] * scale);
+  *reinterpret_cast<bf16x8*>(dst + (int64_t)idx * 8) = v;
+}
+
+
 // One wave-wide LDS DMA: lane L copies 16 bytes from sbase + voff (bytes) to LDS byte address
 // m0 + 16 L; sbase and m0 are wave-uniform. Issued as inline assembly so that the compiler's
 // wait insertion does not treat every later LDS read as dependent on it: each use is paired
@@ -358,9 +418,10 @@ __device__ __forceinline__ void dma16_stream(const void* sbase, uint32_t voff, u
                "{m0}"(m0)
                : "memory");
 }
-// Same for 4 bytes per lane: lane L copies sbase + voff to LDS byte address m0 + 4 L.
-__device__ __forceinline__ void dma4(const void* sbase, uint32_t voff, uint32_t m0) {
-  asm volatile(FFK_DMA_HAZARD "global_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m0)
+// Same for one byte per lane: lane L writes the byte at sbase + voff, zero-extended, to the four
+// LDS bytes at m0 + 4 L.
+__device__ __forceinline__ void dma1(const void* sbase, uint32_t voff, uint32_t m0) {
+  asm volatile(FFK_DMA_HAZARD "global_load_lds_ubyte %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m0)
                : "memory");
 }
 // Same with a whole 64-bit address per lane.

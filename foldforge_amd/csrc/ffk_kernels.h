@@ -13,12 +13,12 @@ struct TrimulArgs {
   const bf16* z;
   const uint8_t* mask;
   const float *ln_w, *ln_b, *lno_w, *lno_b;
-  const bf16* wp;  // [4h][c]: left, left_gate, right, right_gate
-  const bf16* wg;  // [c][c]
-  const bf16* wo;  // [c][h]
-  bf16 *A, *B, *P;  // [batch][h][np][np]
-  float* maskf;     // [batch][np] scratch: the key mask as 1 / 0, zero past n
-  const int* kstages;  // [batch] 32-wide k stages up to the last real key (NULL: all)
+  const float *w_left, *w_right, *w_left_gate, *w_right_gate;  // [h][c]
+  const float* w_gate;  // [c][c]
+  const float* w_out;   // [c][h]
+  bf16 *A, *B, *P;  // [batch][h][np][np]; A, B: rows < n, columns < n padded to 64
+  bf16* wgo;        // [2][128 * 128] scratch: w_gate and w_out packed for the output kernel
+  int* kstages;     // [batch] scratch: 32-wide k stages up to the last real key
   bf16* out;
   int batch, n, np, outgoing, residual;
   float eps;
@@ -29,29 +29,30 @@ void launch_trimul(const TrimulArgs& a, hipStream_t stream);
 // any batch element (at least 1), from the key mask [batch][n].
 void launch_length_eps(const uint8_t* mask, int batch, int n, float eps, float* eps_out,
                        hipStream_t stream);
-// P[p] = X[p] Y[p]^T for `planes` planes of [np][np] bf16 (np % 128 == 0). With kstages, plane
-// p runs only the first kstages[p / planes_per_batch] k stages of 32 (the operands are zero past
-// them, so the product is unchanged).
-void launch_trimul_contract(const bf16* A, const bf16* B, bf16* P, int64_t planes, int np,
+// P[p] = X[p] Y[p]^T for `planes` planes of [np][np] bf16 (np % 128 == 0): rows and columns
+// i, j < n over k < n padded to 64 (all that X and Y have to hold). With kstages, plane p runs
+// only the first kstages[p / planes_per_batch] k stages of 32 (the operands are zero past them,
+// so the product is unchanged).
+void launch_trimul_contract(const bf16* A, const bf16* B, bf16* P, int64_t planes, int n, int np,
                             hipStream_t stream, const int* kstages = nullptr,
                             int planes_per_batch = 1);
 
 struct TriattnArgs {
   const bf16* z;
   const uint8_t* mask;
-  const float* maskf;  // [batch][np] key mask as 1 / 0, zero past n
   const float *ln_w, *ln_b;
-  const bf16* wqkv;  // [3 * 128][128], query rows carry d^-1/2 * log2(e)
-  const bf16* wb;    // [32][128], rows < heads carry log2(e) * to_bias, others zero
-  const bf16* wg;    // [128][128] to_gate
-  const bf16* wo;    // [128][128] to_out
+  const float *w_query, *w_key, *w_value;  // [128][128]
+  float q_scale;        // d^-1/2 log2(e), folded into the query rows
+  const float* w_bias;  // [heads][128]
+  const float *w_gate, *w_out;  // [128][128]
   bf16 *q, *k, *vt;  // [batch * heads][np][np][32], vt: [batch * heads][np][np / 32][32][32]
   float* bias;       // [batch * heads][np / 32][np / 32][2][32][16] blocked, see triattn.hip
-  const int* kstages;  // [batch] key stages holding a real key (written by the weight packing)
+  bf16* wgo;         // [2 or (dual) 3][128 * 128] scratch: w_gate, w_out, w_out_t packed
+  int* kstages;      // [batch] scratch: key stages up to the last real key
   bf16* o;           // [batch][n][n][128] z-frame attention output
   const float *bg, *bo;  // gate / output projection biases [128] (NULL: none)
   int form;          // kTriattn*: how the update reaches out
-  const bf16* wo_t;  // kTriattnDual: the second output projection [128][128] and its bias
+  const float* w_out_t;  // kTriattnDual: the second output projection [128][128] and its bias
   const float* bo_t;
   bf16* tbuf;        // kTriattnUntransposed / kTriattnDual: [batch][n][n][128] update scratch
   bf16* out;
@@ -141,8 +142,8 @@ enum {
 enum { kActNone = 0, kActSigmoid = 1, kActSilu = 2, kActRelu = 3 };
 // Row maps (RowGemmArgs.tmap): the input row read for logical row m, and the rows the epilogue
 // of kEpiResid writes. kMapPairT: m = (b n + r) n + j reads row (b n + j) n + r (the
-// transposed pair); kMapGridOut / kMapGridIn: m = (b npm + i) npm + k over the padded grid
-// reads pair row (b n + i) n + k / (b n + k) n + i (clamped past n); kMapPadKeys /
+// transposed pair); kMapGridOut / kMapGridIn: m = (b n + i) gk + k (gk = n padded) reads pair
+// row (b n + i) n + k / (b n + k) n + i (k clamped past n); kMapPadKeys /
 // kMapPadKeysT: m = (b n + r) np + j over keys padded to np reads pair row (b n + r) n + j' /
 // (b n + j') n + r with j' = min(j, n - 1).
 enum { kMapIdentity = 0, kMapPairT = 1, kMapGridOut = 2, kMapGridIn = 3, kMapPadKeys = 4, kMapPadKeysT = 5 };
@@ -192,11 +193,11 @@ struct RowGemmArgs {
   bf16 *lt, *rt, *mt;
   int sp;
   // kEpiTrimul: w0..w3 = to_left, to_right, to_left_gate, to_right_gate ([hid][K], O = 4 hid),
-  // tiles packed as 16 projection rows + their 16 gate rows; rows on the padded grid (kMapGrid*);
-  // pa / pb [batch][hid][npm][npm] = proj * mask_i mask_k * sigmoid(gate), 0 past n.
+  // rows on the padded grid (kMapGrid*); pa / pb [batch][hid][npm][npm] =
+  // proj * mask_i mask_k * sigmoid(gate) at rows i < n, columns k < gk (0 past n).
   const uint8_t* mask;
   bf16 *pa, *pb;
-  int tmap, npm;
+  int tmap, npm, gk;
   const bf16* yin;   // kEpiGateResid: [M][O]
   float* h32;  // kEpiSwiglu: [M][hid] = silu(a) * b
   bf16* hy;    // kEpiStoreY: [M][O] = y
@@ -347,26 +348,8 @@ struct OpmGroupedArgs {
 };
 void launch_opm_contract_grouped(const OpmGroupedArgs& a, hipStream_t stream);
 
-struct PackSeg {
-  const float* src;  // NULL: write zeros
-  bf16* dst;
-  int64_t n;
-  float scale;
-  int swap23;        // 1: dst[i] = src[i with index bits 2 and 3 exchanged]
-};
-struct PackJob {
-  PackSeg seg[8];
-  int nseg;
-  // optional: the key mask as fp32 rows maskf[b][s] = mask[b][s] ? 1 : 0 (s < n), 0 for
-  // n <= s < np (mask NULL: none)
-  const uint8_t* mask;
-  float* maskf;
-  // optional with the mask: kstages[b] = the number of 32-key stages up to the last real key
-  // of batch element b (0 when it has none)
-  int* kstages;
-  int batch, n, np;
-};
-void launch_pack(const PackJob& job, hipStream_t stream);
+// dst[i] = bf16(src[i]), i < n.
+void launch_pack(const float* src, bf16* dst, int64_t n, hipStream_t stream);
 
 // Compute units of the current device (cached per device).
 int cu_count();

@@ -88,9 +88,8 @@ __device__ inline int64_t mapped_row(const RowGemmArgs& a, int64_t m) {
     return (b * a.n + j) * a.n + (bn - b * a.n);
   }
   if (a.tmap == kMapGridOut || a.tmap == kMapGridIn) {
-    const int64_t gg = (int64_t)a.npm * a.npm;
-    const int64_t b = m / gg, rem = m - b * gg;
-    const int i = min((int)(rem / a.npm), a.n - 1), k = min((int)(rem % a.npm), a.n - 1);
+    const int64_t bi = m / a.gk, b = bi / a.n;
+    const int i = (int)(bi - b * a.n), k = min((int)(m - bi * a.gk), a.n - 1);
     return a.tmap == kMapGridOut ? (b * a.n + i) * a.n + k : (b * a.n + k) * a.n + i;
   }
   return m;
@@ -153,10 +152,9 @@ __device__ inline const float* tile_weight_row(const RowGemmArgs& a, int ot, int
 template <int EPI>
 __device__ __forceinline__ float row_pre(const RowGemmArgs& a, const int64_t m) {
   if (EPI == kEpiTrimul) {
-    const int64_t gg = (int64_t)a.npm * a.npm;
-    const int64_t b = m / gg, rem = m - b * gg;
-    const int i = (int)(rem / a.npm), k = (int)(rem - (int64_t)i * a.npm);
-    return i < a.n && k < a.n && a.mask[b * a.n + i] && a.mask[b * a.n + k] ? 1.f : 0.f;
+    const int64_t bi = m / a.gk, b = bi / a.n;
+    const int i = (int)(bi - b * a.n), k = (int)(m - bi * a.gk);
+    return k < a.n && a.mask[b * a.n + i] && a.mask[b * a.n + k] ? 1.f : 0.f;
   }
   return 0.f;
 }
@@ -257,7 +255,8 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
   } else if (EPI == kEpiTrimul) {
     const int hid = a.O / 4;
     const int64_t gg = (int64_t)a.npm * a.npm;
-    const int64_t b = m / gg, rem = m - b * gg;
+    const int64_t bi = m / a.gk, b = bi / a.n;
+    const int64_t rem = (bi - b * a.n) * a.npm + (m - bi * a.gk);
     const float keep = pre;  // the pair mask factor (row_pre)
     bf16* plane = (seg == 0 ? a.pa : a.pb) + b * hid * gg + rem;
 #pragma unroll
@@ -546,11 +545,11 @@ struct TileRun {
 };
 template <int EPI>
 __device__ __forceinline__ void run_radix(const RowGemmArgs& a, uint32_t& L, uint32_t& R) {
-  L = EPI == kEpiTrimul ? a.npm
+  L = EPI == kEpiTrimul ? a.gk
       : EPI == kEpiOpm  ? a.sp
       : EPI == kEpiPwa || EPI == kEpiApbFlash ? a.np
                                               : a.n;
-  R = EPI == kEpiTrimul ? a.npm : EPI == kEpiPwa ? a.depth : a.n;
+  R = EPI == kEpiPwa ? a.depth : a.n;
   L = L ? L : 1;  // (the epilogues without a row map leave n unset)
   R = R ? R : 1;
 }
@@ -589,7 +588,7 @@ __device__ __forceinline__ int64_t run_row(const RowGemmArgs& a, const TileRun& 
     return (int64_t)t.b * a.depth * n + t.r + (int64_t)s * n;
   }
   if (EPI == kEpiTrimul) {
-    const int i = min((int)t.r, n - 1), k = min((int)t.rem + li, n - 1);
+    const int i = (int)t.r, k = min((int)t.rem + li, n - 1);
     return a.tmap == kMapGridOut ? ((int64_t)t.b * n + i) * n + k
                                  : (int64_t)t.b * n * n + i + (int64_t)k * n;
   }
@@ -619,11 +618,6 @@ __device__ __forceinline__ int64_t run_row(const RowGemmArgs& a, const TileRun& 
     return ((int64_t)b * n + j) * n + r;
   }
   return m0 + l;
-}
-
-// Mask bits of a tile's 32 rows at row 8 v + 4 g + e: bit set -> x, clear -> 0.
-__device__ __forceinline__ float keep_bit(float x, uint32_t bits_g, int v, int e) {
-  return __uint_as_float(__float_as_uint(x) & (uint32_t)((int32_t)(bits_g << (31 - 8 * v - e)) >> 31));
 }
 
 template <int EPI, int XSRC, int K>
@@ -723,7 +717,7 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
     keep = 0;
     if (EPI == kEpiTrimul) {
       const uint8_t* mb = a.mask + (int64_t)tr.b * a.n;
-      const int i = min((int)tr.r, a.n - 1), k = min((int)tr.rem + li, a.n - 1);
+      const int i = (int)tr.r, k = min((int)tr.rem + li, a.n - 1);
       keep = (uint32_t)mb[k] | ((uint32_t)mb[i] << 8);
     } else if (EPI == kEpiOpm) {
       keep = a.rows_mask[row];
@@ -734,7 +728,7 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
     // rows kept by the mask, bit = row of the tile
     uint32_t bits = ~0u;
     if constexpr (EPI == kEpiTrimul) {
-      const bool on = (int)tr.r < a.n && (int)tr.rem + li < a.n && (keep & 0xff) && (keep >> 8);
+      const bool on = (int)tr.rem + li < a.n && (keep & 0xff) && (keep >> 8);
       bits = (uint32_t)__ballot(on);
       if (bits == 0) {
         // every pair of the tile is masked or padding: zeros, without the products

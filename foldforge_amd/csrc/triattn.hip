@@ -57,8 +57,12 @@ constexpr float kSumRescale = 1.8446744073709552e19f; // 2^64: a tile's partial 
 
 constexpr int kPT = 64;        // positions per projection / output tile
 
-// Persistent, weight-stationary, one barrier per tile. Tiles are (batch, row r of the padded
-// grid, 64 positions along the attention row). Waves 0-3 hold the query and key rows of
+// Persistent, weight-stationary, one barrier per tile. Tiles are (batch, attention row r, 64
+// positions along it), r < n padded to 32: the flash core takes 4 rows at once and reads the
+// bias (whose queries or keys the rows are) in tiles of 32; positions past n are zero rows. The fp32 parameters are rounded to bf16 once per workgroup,
+// behind the first tiles' transfers (the query rows carry q_scale, the bias rows log2(e)). The
+// first workgroups also pack the output kernel's weights and count the flash core's key stages:
+// a launch of their own in front of every call took 4 to 5 us. Waves 0-3 hold the query and key rows of
 // head w, waves 4-7 the value rows of head w - 4; waves 4 and 5 also project the pair bias
 // of the tile's first and second 32 positions (4 heads padded to 32 rows). The z tiles
 // arrive by LDS DMA two tiles ahead in a three-slot ring and are normalised in place one
@@ -66,15 +70,19 @@ constexpr int kPT = 64;        // positions per projection / output tile
 // Each wave stages its outputs in LDS of its own and writes 16 bytes per lane: q and k as
 // 64-byte position rows, v^T as 128-byte runs of the 64 positions of one channel.
 __global__ __launch_bounds__(512, 2) void triattn_project(
-    const bf16* __restrict__ z, const float* __restrict__ maskf, const float* __restrict__ ln_w,
-    const float* __restrict__ ln_b, const bf16* __restrict__ wqkv, const bf16* __restrict__ wb,
-    bf16* __restrict__ qo, bf16* __restrict__ ko, bf16* __restrict__ vto, float* __restrict__ bo,
+    const bf16* __restrict__ z, const uint8_t* __restrict__ mask, const float* __restrict__ ln_w,
+    const float* __restrict__ ln_b, const float* __restrict__ w_query,
+    const float* __restrict__ w_key, const float* __restrict__ w_value,
+    const float* __restrict__ w_bias, float q_scale, const float* __restrict__ w_gate,
+    const float* __restrict__ w_out, const float* __restrict__ w_out_t, bf16* __restrict__ w_next,
+    int* __restrict__ kstages, bf16* __restrict__ qo, bf16* __restrict__ ko, bf16* __restrict__ vto, float* __restrict__ bo,
     int batch, int n, int np, int starting, int transposed_bias, float eps) {
   constexpr int NB = 3, H = 4;
   __shared__ __attribute__((aligned(16))) bf16 zt[NB][kPT * 128];  // raw z, then LN(z) (off128)
-  __shared__ __attribute__((aligned(16))) bf16 sqk[4][32 * 32];    // [position][d], q then k
-  __shared__ __attribute__((aligned(16))) bf16 svt[4][32 * kPT];   // [d][key slot]
-  __shared__ __attribute__((aligned(16))) float keep[NB][kPT];     // key mask per position
+  // per wave: the output stage (waves 0-3: q then k [position][d]; 4-7: v^T [d][key slot]), first
+  // the tile its weights are turned in
+  __shared__ __attribute__((aligned(16))) bf16 stage[8][32 * 128];
+  __shared__ __attribute__((aligned(16))) uint32_t keep[NB][kPT];  // key mask per position
   __shared__ __attribute__((aligned(16))) bf16 wbl[H * 128];       // the pair-bias rows
   __shared__ __attribute__((aligned(16))) float lnp[2][128];        // LayerNorm affine
   const int tid = threadIdx.x;
@@ -82,27 +90,18 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool qk = wave < 4;
   const int head = wave & 3;
-  if (tid < 256) lnp[tid >> 7][tid & 127] = (tid < 128 ? ln_w : ln_b)[tid & 127];
-  for (int e = tid; e < H * 128; e += 512) wbl[e] = wb[e];  // published by the first barrier
-  WFrag w0, w1;
-  load_wfrag(w0, wqkv, qk ? 32 * head : 256 + 32 * head, li, g);
-  settle(w0);
-  if (qk) {
-    load_wfrag(w1, wqkv, 128 + 32 * head, li, g);
-    settle(w1);
-  }
   // The bias entry at tile position t is (query r, key s0 + t), except for the AF3 ending
   // node (bias from the un-transposed pair), where it is (query s0 + t, key r).
   const bool key_major = !starting && !transposed_bias;
-  const int nsb = np / kPT;
+  const int nsb = (n + kPT - 1) / kPT, rows = (n + 31) & ~31;
   const int64_t nb = np / 32;
-  const int ntiles = batch * np * nsb;
+  const int ntiles = batch * rows * nsb;
   auto where = [&](int tile, int& b, int& r, int& s0, int& valid) {
     const int sb = tile % nsb;
-    r = (tile / nsb) % np;
-    b = tile / (nsb * np);
+    r = (tile / nsb) % rows;
+    b = tile / (nsb * rows);
     s0 = sb * kPT;
-    valid = (r < n) ? max(0, min(kPT, n - s0)) : 0;
+    valid = (r < n) ? min(kPT, n - s0) : 0;
   };
   // This wave's 2 one-KB pieces (positions 8 wave .. 8 wave + 7) of a tile's z rows into ring
   // slot buf (positions past the end re-read a real row, zeroed by the LayerNorm); wave 7
@@ -130,18 +129,35 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
       dma16_stream(base, pe * stride + 16 * ((lane & 15) ^ (pos & 15)), dst + 1024 * piece);
     }
     if (wave == 7) {
-      const float* mrow = maskf + (int64_t)b * np + (key_major ? r : s0);
-      dma4(mrow, key_major ? 0u : 4u * lane, lds_addr(&keep[buf][0]));
+      dma1(mask + (int64_t)b * n, (uint32_t)min(key_major ? r : s0 + lane, n - 1), lds_addr(&keep[buf][0]));
     }
   };
   const int step = gridDim.x;
   if ((int)blockIdx.x >= ntiles) return;
   z_dma(blockIdx.x, 0);
   z_dma(blockIdx.x + step, 1);
-  if (wave == 7)
-    wait_vm_lds<3>();  // this wave's transfers of the first tile landed
-  else
-    wait_vm_lds<2>();
+  // published by the first barrier
+  if (tid < 256) lnp[tid >> 7][tid & 127] = (tid < 128 ? ln_w : ln_b)[tid & 127];
+  wbl[tid] = (bf16)(w_bias[tid] * kLog2e);  // H * 128 = the workgroup's threads
+  WFrag w0, w1;
+  {
+    WRows r0, r1;
+    fetch_wrows(r0, qk ? w_query : w_value, 32 * head, lane);
+    if (qk) fetch_wrows(r1, w_key, 32 * head, lane);
+    // the output kernel's weights (gate, output projection, the dual form's second one)
+    const int pieces = w_next ? (w_out_t ? 3 : 2) * 2048 : 0;
+    for (int idx = blockIdx.x * 512 + tid; idx < pieces; idx += gridDim.x * 512) {
+      const int m = idx >> 11;
+      pack_wfrag(m == 0 ? w_gate : m == 1 ? w_out : w_out_t, m == 0 ? -kLog2e : 1.f, w_next + m * 16384,
+                 idx & 2047);
+    }
+    turn_wrows(w0, r0, qk ? q_scale : 1.f, stage[wave], lane);
+    if (qk) turn_wrows(w1, r1, 1.f, stage[wave], lane);
+  }
+  if (wave == 0) count_stages(mask, n, batch, blockIdx.x, gridDim.x, lane, kstages);
+  settle(w0);
+  if (qk) settle(w1);
+  wait_vm_lds<0>();  // this wave's transfers of the first tiles landed
   __syncthreads();
   {
     int b, r, s0, valid;
@@ -170,7 +186,7 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
     const bf16* xh = zt[buf];
     const int64_t bh = (int64_t)b * H + head;
     if (qk) {
-      bf16* st = sqk[head];
+      bf16* st = stage[wave];
       bf16* qd = qo + ((bh * np + r) * np + s0) * 32;
       bf16* kd = ko + ((bh * np + r) * np + s0) * 32;
 #pragma unroll
@@ -206,7 +222,7 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
         }
       }
     } else {
-      bf16* st = svt[head];
+      bf16* st = stage[wave];
 #pragma unroll
       for (int pt = 0; pt < kPT / 32; ++pt) {
         f32x16 av = zero16();
@@ -232,14 +248,14 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
             ab = mfma32(wrow, ld8(&xh[off128(pt * 32 + li, 2 * kk + g)]), ab);
           }
           // D[head][position]: heads are rows 0..3 = registers 0..3 of lane group 0
-          const float kp = keep[buf][pt * 32 + li];
           const int64_t s = s0 + pt * 32 + li;
           const int64_t query = key_major ? s : r;
           const int64_t key = key_major ? r : s;
+          const bool kp = key < n && keep[buf][pt * 32 + li] != 0;
           if (g == 0) {
 #pragma unroll
             for (int q = 0; q < H; ++q)
-              bo[bias_index((int64_t)b * H + q, nb, query, key)] = kp != 0.f ? ab[q] : -INFINITY;
+              bo[bias_index((int64_t)b * H + q, nb, query, key)] = kp ? ab[q] : -INFINITY;
           }
         }
       }
@@ -347,7 +363,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_bias(FlashArgs a) {
   const int dl = DQ == 1 ? li & 15 : li;  // V^T row (of each half) of this lane (16-wide heads: rows repeat)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t jw = j0 + 32 * wave;  // first query of this wave
-  const bool active = jw < np;        // the last query block may be partial
+  const bool active = jw < a.n_valid;  // the last query block may be partial
   const int64_t j = jw + li;
   const int64_t nb = np / 32;
   const int64_t nstage = np / kFK;
@@ -598,7 +614,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_bias(FlashArgs a) {
       return st;
     };
     float mx = -INFINITY;
-    for (int64_t kb = 0; kb < nb; ++kb) {
+    for (int64_t kb = 0; kb < nrun; ++kb) {
       const f32x16 st = logits(kb);
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[i]);
@@ -609,7 +625,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_bias(FlashArgs a) {
 #pragma unroll
     for (int h = 0; h < DH; ++h) o[h] = zero16();
     float ls = 0.f;
-    for (int64_t kb = 0; kb < nb; ++kb) {
+    for (int64_t kb = 0; kb < nrun; ++kb) {
       f32x16 st = logits(kb);
 #pragma unroll
       for (int i = 0; i < 16; ++i) st[i] -= off;
@@ -690,16 +706,6 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
   const int lane = tid & 63, g = lane >> 5, li = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cb = wave & 3, pt = wave >> 2;
-  if (tid < 256) lnp[tid >> 7][tid & 127] = (tid < 128 ? ln_w : ln_b)[tid & 127];
-  if (tid >= 256) {  // published by the first barrier; absent biases are zeros
-    const int c = tid & 127;
-    pbias[(tid >> 7) & 1][c] = tid < 384 ? (bg ? -kLog2e * bg[c] : 0.f) : (bo ? bo[c] : 0.f);
-  }
-  WFrag fg, fo;
-  load_wfrag(fg, wg, 32 * cb, li, g);
-  load_wfrag(fo, wo, 32 * cb, li, g);
-  settle(fg);
-  settle(fo);
   const int njb = (n + kPT - 1) / kPT;
   const int ntiles = batch * n * njb;
   auto where = [&](int tile, int& valid) -> int64_t {
@@ -730,7 +736,20 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
   if ((int)blockIdx.x >= ntiles) return;
   dma(blockIdx.x, 0);
   dma(blockIdx.x + step, 1);
-  wait_vm_lds<4>();  // this wave's transfers of the first tile landed
+  // behind the transfers: affine and biases (published by the first barrier; absent biases are
+  // zeros) and the weights
+  if (tid < 256) {
+    lnp[tid >> 7][tid & 127] = (tid < 128 ? ln_w : ln_b)[tid & 127];
+  } else {
+    const int c = tid & 127;
+    pbias[(tid >> 7) & 1][c] = tid < 384 ? (bg ? -kLog2e * bg[c] : 0.f) : (bo ? bo[c] : 0.f);
+  }
+  WFrag fg, fo;
+  load_wfrag(fg, wg, cb, lane);
+  load_wfrag(fo, wo, cb, lane);
+  settle(fg);
+  settle(fo);
+  wait_vm_lds<0>();  // this wave's transfers of the first tiles landed
   __syncthreads();
   {
     int valid;
@@ -844,10 +863,10 @@ void launch_flash(const FlashArgs& a, hipStream_t stream) {
 
 void launch_triattn(const TriattnArgs& a, hipStream_t stream) {
   const int np = a.np;
-  const int tiles_p = a.batch * np * (np / kPT);
+  const int tiles_p = a.batch * ((a.n + 31) & ~31) * ((a.n + kPT - 1) / kPT);
   triattn_project<<<persistent_grid(tiles_p, 1), 512, 0, stream>>>(
-      a.z, a.maskf, a.ln_w, a.ln_b, a.wqkv, a.wb, a.q, a.k, a.vt, a.bias, a.batch, a.n, np,
-      a.starting, a.transposed_bias, a.eps);
+      a.z, a.mask, a.ln_w, a.ln_b, a.w_query, a.w_key, a.w_value, a.w_bias, a.q_scale,
+      a.w_gate, a.w_out, a.w_out_t, a.project_only ? nullptr : a.wgo, a.kstages, a.q, a.k, a.vt, a.bias, a.batch, a.n, np, a.starting, a.transposed_bias, a.eps);
   FlashArgs f{};
   f.q = a.q;
   f.k = a.k;
@@ -877,18 +896,18 @@ void launch_triattn(const TriattnArgs& a, hipStream_t stream) {
   const int tiles_o = a.batch * a.n * ((a.n + kPT - 1) / kPT);
   auto output = [&](const bf16* wo, const float* bo, bf16* dst, int residual) {
     triattn_output<<<persistent_grid(tiles_o, 1), 512, 0, stream>>>(
-        a.z, a.o, a.ln_w, a.ln_b, a.wg, wo, a.bg, bo, dst, a.batch, a.n, residual, a.eps);
+        a.z, a.o, a.ln_w, a.ln_b, a.wgo, wo, a.bg, bo, dst, a.batch, a.n, residual, a.eps);
   };
   if (a.form == kTriattnUntransposed) {
     // the update in the attention's orientation: the z-frame update, transposed
-    output(a.wo, a.bo, a.tbuf, 0);
+    output(a.wgo + 16384, a.bo, a.tbuf, 0);
     launch_pair_add_transposed(a.residual ? a.z : nullptr, a.tbuf, a.out, a.batch, a.n, 128, stream);
   } else if (a.form == kTriattnDual) {
-    output(a.wo_t, a.bo_t, a.tbuf, 0);
-    output(a.wo, a.bo, a.out, a.residual);
+    output(a.wgo + 2 * 16384, a.bo_t, a.tbuf, 0);
+    output(a.wgo + 16384, a.bo, a.out, a.residual);
     launch_pair_add_transposed(a.out, a.tbuf, a.out, a.batch, a.n, 128, stream);
   } else {
-    output(a.wo, a.bo, a.out, a.residual);
+    output(a.wgo + 16384, a.bo, a.out, a.residual);
   }
 }
 

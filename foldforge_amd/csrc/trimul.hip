@@ -28,37 +28,37 @@ constexpr int kCT = 128;      // contraction output tile
 constexpr int kCK = 32;       // contraction k step
 constexpr int kCKP = kCK + 8; // LDS row stride of a contraction operand tile
 
-// Persistent: tiles are (batch, row r of the padded grid, 64 positions along s); one
-// workgroup of 8 waves per CU. wp rows: [0,h) to_left, [h,2h) to_left_gate, [2h,3h)
-// to_right, [3h,4h) to_right_gate. Wave w computes output o = w / 4 (0: A, 1: B) for hidden
-// channels 32 (w % 4) .. + 31, holding that slice of the projection and of its gate in
-// registers.
+// Persistent: tiles are (batch, row r < n, 64 positions along s); one workgroup of 8 waves per
+// CU. Wave w computes output o = w / 4 (0: A, 1: B) for hidden channels 32 (w % 4) .. + 31,
+// holding that slice of the projection and of its gate in registers, rounded from the fp32
+// parameters once per workgroup, behind the first tiles' transfers (the gate rows carry
+// -log2(e)). The first workgroups also pack the output kernel's weights and count the key stages
+// of the contraction: a launch of their own in front of every call took 4 to 5 us.
 // Memory stays busy through the compute: the z tiles stream through a ring of three LDS
 // buffers by LDS DMA, two tiles ahead, and the stores of a tile are left in flight (a wave
 // only waits for its own DMA pieces, never for its stores).
 __global__ __launch_bounds__(512, 2) void trimul_project(
-    const bf16* __restrict__ z, const float* __restrict__ maskf, const float* __restrict__ ln_w,
-    const float* __restrict__ ln_b, const bf16* __restrict__ wp, bf16* __restrict__ a_out,
-    bf16* __restrict__ b_out, int batch, int n, int np, int outgoing, float eps) {
+    const bf16* __restrict__ z, const uint8_t* __restrict__ mask, const float* __restrict__ ln_w,
+    const float* __restrict__ ln_b, const float* __restrict__ w_left,
+    const float* __restrict__ w_right, const float* __restrict__ w_left_gate,
+    const float* __restrict__ w_right_gate, bf16* __restrict__ a_out, bf16* __restrict__ b_out,
+    const float* __restrict__ w_gate, const float* __restrict__ w_out, bf16* __restrict__ w_next,
+    int* __restrict__ kstages, int batch, int n, int np, int outgoing, float eps) {
   constexpr int H = 128, NB = 3;
   __shared__ __attribute__((aligned(16))) bf16 zt[NB][kPT * 128];  // raw z, then LN(z) (off128)
-  __shared__ __attribute__((aligned(16))) bf16 stage[8][32 * kPS];  // [channel][position]
-  __shared__ __attribute__((aligned(16))) float msk[NB][8][kPT];    // token mask m[s0 + t], per wave
-  __shared__ float mrw[NB][8];                                      // token mask m[r], per wave
+  // per wave: the output stage [channel][position], first the tile its weights are turned in
+  __shared__ __attribute__((aligned(16))) bf16 stage[8][32 * 128];
+  static_assert(32 * kPS <= 32 * 128, "stage size");
+  __shared__ __attribute__((aligned(16))) uint32_t msk[NB][8][kPT];  // token mask m[s0 + t], per wave
+  __shared__ uint32_t mrw[NB][8];                                    // token mask m[r], per wave
   __shared__ __attribute__((aligned(16))) float lnp[2][H];  // LayerNorm affine
   const int tid = threadIdx.x;
   const int lane = tid & 63, g = lane >> 5, li = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int o = wave >> 2, cb = wave & 3;  // output (A / B), channel block
-  if (tid < 2 * H) lnp[tid / H][tid % H] = (tid < H ? ln_w : ln_b)[tid % H];  // published by the first barrier
-  WFrag wv, wgt;
-  load_wfrag(wv, wp, 2 * H * o + 32 * cb, li, g);
-  load_wfrag(wgt, wp, 2 * H * o + H + 32 * cb, li, g);
-  settle(wv);
-  settle(wgt);
-  const int nsb = np / kPT;
+  const int nsb = (n + kPT - 1) / kPT;
   const int64_t plane = (int64_t)np * np;
-  auto valid_of = [&](const TileAt& t) { return t.r < n ? max(0, min(kPT, n - t.blk * kPT)) : 0; };
+  auto valid_of = [&](const TileAt& t) { return min(kPT, n - t.blk * kPT); };
   // This wave's 2 one-KB pieces (positions 8 wave .. 8 wave + 7) of a tile's z rows and its
   // own copies of the tile's token-mask values m[s0 + t] (one float per lane) and m[r] (lane
   // 0) into ring slot buf; positions past the end re-read a real row (zeroed by the
@@ -69,17 +69,15 @@ __global__ __launch_bounds__(512, 2) void trimul_project(
   auto z_dma = [&](TileAt t, int buf) {
     if (t.b >= batch) t = TileAt{0, 0, 0};
     const int s0 = t.blk * kPT, valid = valid_of(t);
-    const bf16* base = z;
+    const bf16* base;
     uint32_t stride = 256;  // bytes between consecutive positions
-    if (valid > 0) {
-      if (outgoing) {
-        base = z + (((int64_t)t.b * n + t.r) * n + s0) * 128;
-      } else {
-        base = z + (((int64_t)t.b * n + s0) * n + t.r) * 128;
-        stride = (uint32_t)n * 256;
-      }
+    if (outgoing) {
+      base = z + (((int64_t)t.b * n + t.r) * n + s0) * 128;
+    } else {
+      base = z + (((int64_t)t.b * n + s0) * n + t.r) * 128;
+      stride = (uint32_t)n * 256;
     }
-    const int last = valid > 0 ? valid - 1 : 0;
+    const int last = valid - 1;
     const uint32_t dst = lds_addr(&zt[buf][0]);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -87,22 +85,37 @@ __global__ __launch_bounds__(512, 2) void trimul_project(
       const int pe = pos < last ? pos : last;
       dma16_stream(base, pe * stride + 16 * ((lane & 15) ^ (pos & 15)), dst + 1024 * piece);
     }
-    const float* mb = maskf + (int64_t)t.b * np;
-    dma4(mb + s0, 4u * lane, lds_addr(&msk[buf][wave][0]));
-    if (lane == 0) dma4(mb + t.r, 0u, lds_addr(&mrw[buf][wave]));
+    const uint8_t* mb = mask + (int64_t)t.b * n;
+    dma1(mb, (uint32_t)min(s0 + lane, n - 1), lds_addr(&msk[buf][wave][0]));
+    if (lane == 0) dma1(mb, (uint32_t)t.r, lds_addr(&mrw[buf][wave]));
   };
-  if ((int)blockIdx.x >= batch * np * nsb) return;
-  const TileAt stride = tile_at(gridDim.x, nsb, np);
-  TileAt cur = tile_at(blockIdx.x, nsb, np);
-  TileAt nxt = tile_add(cur, stride, nsb, np);
-  TileAt far = tile_add(nxt, stride, nsb, np);
+  if ((int)blockIdx.x >= batch * n * nsb) return;
+  const TileAt stride = tile_at(gridDim.x, nsb, n);
+  TileAt cur = tile_at(blockIdx.x, nsb, n);
+  TileAt nxt = tile_add(cur, stride, nsb, n);
+  TileAt far = tile_add(nxt, stride, nsb, n);
   // Software pipeline, one barrier per tile: after the barrier of tile k a wave issues the
   // fetch of tile k + 2, projects and stores tile k (normalised in the previous step), then
   // normalises tile k + 1 (fetched one step earlier) in its own ring slot, so LayerNorm work
   // overlaps the other waves' MFMAs.
   z_dma(cur, 0);
   z_dma(nxt, 1);
-  wait_vm_lds<4>();  // this wave's transfers of the first tile landed
+  if (tid < 2 * H) lnp[tid / H][tid % H] = (tid < H ? ln_w : ln_b)[tid % H];  // published by the first barrier
+  WFrag wv, wgt;
+  {
+    WRows rv, rg;
+    fetch_wrows(rv, o == 0 ? w_left : w_right, 32 * cb, lane);
+    fetch_wrows(rg, o == 0 ? w_left_gate : w_right_gate, 32 * cb, lane);
+    // the output kernel's weights (gate, then output projection), a piece per thread
+    for (int idx = blockIdx.x * 512 + tid; idx < 4096; idx += gridDim.x * 512)
+      pack_wfrag(idx < 2048 ? w_gate : w_out, idx < 2048 ? -kLog2e : 1.f, w_next + (idx & 2048) * 8, idx & 2047);
+    turn_wrows(wv, rv, 1.f, stage[wave], lane);
+    turn_wrows(wgt, rg, -kLog2e, stage[wave], lane);
+  }
+  if (wave == 0) count_stages(mask, n, batch, blockIdx.x, gridDim.x, lane, kstages);
+  settle(wv);
+  settle(wgt);
+  wait_vm_lds<0>();  // this wave's transfers of the first tiles landed
   __syncthreads();
   ln_inplace_swz<kPT, 512>(zt[0], valid_of(cur), lnp[0], lnp[1], eps);
   int buf = 0, k = 0;
@@ -120,13 +133,11 @@ __global__ __launch_bounds__(512, 2) void trimul_project(
     __syncthreads();
     z_dma(far, fbuf);
     const bf16* xh = zt[buf];
-    // pair mask m[r] m[s]: lane t holds m[s0 + t]; a tile whose 64 pairs are all real takes
-    // the unmasked epilogue, a tile whose pairs are all masked (a padded row, or every
-    // position past the real length) is zero without any product
-    const float mr = mrw[buf][wave];
-    const float ms = msk[buf][wave][lane];
-    const bool full = mr == 1.f && __builtin_amdgcn_ballot_w64(ms != 1.f) == 0;
-    const bool none = mr == 0.f || __builtin_amdgcn_ballot_w64(ms != 0.f) == 0;
+    // pair mask m[r] m[s], bit t of pos s0 + t; a tile whose 64 pairs are all real takes the
+    // unmasked epilogue, a tile whose pairs are all masked is zero without any product
+    const uint64_t bits = __ballot(mrw[buf][wave] != 0 && msk[buf][wave][lane] != 0 && s0 + lane < n);
+    const bool full = bits == ~(uint64_t)0;
+    const bool none = bits == 0;
     bf16* st = stage[wave];
     if (none) {
       const bf16x4 zero4 = {};
@@ -157,15 +168,11 @@ __global__ __launch_bounds__(512, 2) void trimul_project(
       } else {
 #pragma unroll
         for (int m4 = 0; m4 < 4; ++m4) {
+          const uint32_t bits_g = (uint32_t)(bits >> (32 * pt)) >> (4 * g);
           bf16x4 v;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int pa = pt * 32 + 8 * m4 + e;  // uniform; lane group 1 takes pa + 4
-            const float m0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ms), pa));
-            const float m1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ms), pa + 4));
-            const float mk = mr * (g ? m1 : m0);
-            v[e] = (bf16)(av[4 * m4 + e] * mk * sigmoid_scaled(ag[4 * m4 + e]));
-          }
+          for (int e = 0; e < 4; ++e)
+            v[e] = (bf16)(keep_bit(av[4 * m4 + e], bits_g, m4, e) * sigmoid_scaled(ag[4 * m4 + e]));
           *reinterpret_cast<bf16x4*>(&st[li * kPS + pt * 32 + 8 * m4 + 4 * g]) = v;
         }
       }
@@ -183,18 +190,19 @@ __global__ __launch_bounds__(512, 2) void trimul_project(
     if (nxt.b < batch) ln_inplace_swz<kPT, 512>(zt[nbuf], valid_of(nxt), lnp[0], lnp[1], eps);
     cur = nxt;
     nxt = far;
-    far = tile_add(far, stride, nsb, np);
+    far = tile_add(far, stride, nsb, n);
   }
   wait_vm_lds<0>();  // no LDS write may land after exit
 }
 
-// P[bh][i][j] = sum_k X[bh][i][k] * Y[bh][j][k]; all planes [np][np] bf16, np % 128 == 0.
+// P[bh][i][j] = sum_k X[bh][i][k] * Y[bh][j][k], i, j, k < n; all planes [np][np] bf16,
+// np % 128 == 0, n > np - 128.
 // grid: (np / 128)^2 * batch * h workgroups in one dimension, renumbered so that the tiles
 // of a channel plane (which share its X rows and Y rows) run on one XCD and hit one L2;
 // block 256 = 2 x 2 waves of 64 x 64.
 __global__ __launch_bounds__(256) void trimul_contract(const bf16* __restrict__ X,
                                                        const bf16* __restrict__ Y,
-                                                       bf16* __restrict__ P, int np,
+                                                       bf16* __restrict__ P, int n, int np,
                                                        const int* __restrict__ kstages,
                                                        int planes_per_batch) {
   // operand tiles during the k loop, then the output tile [128][kCT + 8] for the stores
@@ -210,17 +218,25 @@ __global__ __launch_bounds__(256) void trimul_contract(const bf16* __restrict__ 
   const bf16* Xb = X + bh * plane + (int64_t)i0 * np;
   const bf16* Yb = Y + bh * plane + (int64_t)j0 * np;
   // k past the batch element's last real key: zero operands, left out
-  const int kend = kstages ? min(np, kstages[bh / planes_per_batch] * kCK) : np;
+  const int k32 = (n + kCK - 1) / kCK;
+  const int kend = (kstages ? min(k32, kstages[bh / planes_per_batch]) : k32) * kCK;
   const int tid = threadIdx.x;
   // global -> LDS: a 128 x 32 tile is 512 chunks of 8 bf16; 2 per thread per operand.
   bf16x8 rx[2], ry[2];
+  const bf16* xsrc[2];
+  const bf16* ysrc[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int c = tid + 256 * u, row = c >> 2, kc = (c & 3) * 8;
+    // rows past n re-read the last one (never written, and their products are dropped)
+    xsrc[u] = Xb + (int64_t)min(row, n - 1 - i0) * np + kc;
+    ysrc[u] = Yb + (int64_t)min(row, n - 1 - j0) * np + kc;
+  }
   auto gload = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int c = tid + 256 * u;
-      const int row = c >> 2, kc = (c & 3) * 8;
-      rx[u] = ld8(Xb + (int64_t)row * np + k0 + kc);
-      ry[u] = ld8(Yb + (int64_t)row * np + k0 + kc);
+      rx[u] = ld8(xsrc[u] + k0);
+      ry[u] = ld8(ysrc[u] + k0);
     }
   };
   auto sstore = [&](int buf) {
@@ -289,7 +305,7 @@ __global__ __launch_bounds__(256) void trimul_contract(const bf16* __restrict__ 
   for (int u = 0; u < kCT * kCT / 8 / 256; ++u) {
     const int chunk = tid + 256 * u;
     const int row = chunk >> 4, c = chunk & 15;
-    st16<kNtContract>(Pb + (int64_t)row * np + 8 * c, ld8(&smem[row * kOS + 8 * c]));
+    if (i0 + row < n) st16<kNtContract>(Pb + (int64_t)row * np + 8 * c, ld8(&smem[row * kOS + 8 * c]));
   }
 }
 
@@ -306,7 +322,7 @@ constexpr int kBStages = 2;
 constexpr int kBStage = 2 * kBT * kBK;      // bf16 per stage (X then Y)
 __global__ __launch_bounds__(512, 2) void trimul_contract256(const bf16* __restrict__ X,
                                                              const bf16* __restrict__ Y,
-                                                             bf16* __restrict__ P, int np,
+                                                             bf16* __restrict__ P, int n, int np,
                                                              const int* __restrict__ kstages,
                                                              int planes_per_batch) {
   __shared__ __attribute__((aligned(16))) bf16 smem[kBStages * kBStage];  // 128 KB
@@ -332,8 +348,10 @@ __global__ __launch_bounds__(512, 2) void trimul_contract256(const bf16* __restr
       const int piece = 8 * wave + u, half = piece >> 5;
       const int row = 8 * (piece & 31) + (lane >> 3);
       const int c = (lane & 7) ^ ((row >> 1) & 7);
+      // (rows past n re-read the last one: never written, and their products are dropped)
+      const int rr = min(row, n - 1 - (half ? j0 : i0));
       const bf16* src = (half ? Yb : Xb) + s * kBK;
-      dma16(src, (uint32_t)(row * np * 2 + 16 * c), base + 1024 * piece);
+      dma16(src, (uint32_t)(rr * np * 2 + 16 * c), base + 1024 * piece);
     }
   };
   f32x16 acc[4][2];
@@ -343,7 +361,8 @@ __global__ __launch_bounds__(512, 2) void trimul_contract256(const bf16* __restr
     for (int c = 0; c < 2; ++c) acc[a][c] = zero16();
   // 32-key stages past the batch element's last real key: zero operands, left out (a 64-wide
   // stage may end with one of them)
-  const int nk32 = kstages ? min(np / kCK, kstages[bh / planes_per_batch]) : np / kCK;
+  const int k32 = (n + kCK - 1) / kCK;
+  const int nk32 = kstages ? min(k32, kstages[bh / planes_per_batch]) : k32;
   const int nk = (nk32 + 1) / 2;
   if (nk > 0) stage_dma(0);
 #pragma unroll 1
@@ -394,7 +413,7 @@ __global__ __launch_bounds__(512, 2) void trimul_contract256(const bf16* __restr
   for (int u = 0; u < kBT * kBT / 8 / 512; ++u) {
     const int chunk = tid + 512 * u;
     const int row = chunk >> 5, c = chunk & 31;
-    st16<kNtContract>(Pb + (int64_t)row * np + 8 * c, ld8(&smem[row * kBT + 8 * (c ^ (row & 15))]));
+    if (i0 + row < n) st16<kNtContract>(Pb + (int64_t)row * np + 8 * c, ld8(&smem[row * kBT + 8 * (c ^ (row & 15))]));
   }
 }
 
@@ -409,8 +428,8 @@ __global__ __launch_bounds__(512, 2) void trimul_contract256(const bf16* __restr
 __global__ __launch_bounds__(512, 2) void trimul_output(
     const bf16* __restrict__ z, const bf16* __restrict__ P, const float* __restrict__ ln_w,
     const float* __restrict__ ln_b, const float* __restrict__ lno_w,
-    const float* __restrict__ lno_b, const bf16* __restrict__ wg, const bf16* __restrict__ wo,
-    bf16* __restrict__ out, int batch, int n, int np, int residual, float eps,
+    const float* __restrict__ lno_b, const bf16* __restrict__ wgo, bf16* __restrict__ out,
+    int batch, int n, int np, int residual, float eps,
     const float* __restrict__ eps_out_dev) {
   constexpr int H = 128, NB = 3;
   __shared__ __attribute__((aligned(16))) bf16 zs[NB][kPT * 128];  // raw z, then out (off128)
@@ -423,15 +442,8 @@ __global__ __launch_bounds__(512, 2) void trimul_output(
   const int lane = tid & 63, g = lane >> 5, li = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cb = wave & 3, pt = wave >> 2;
-  const float* const lsrc[4] = {ln_w, ln_b, lno_w, lno_b};
-  lnp[tid >> 7][tid & 127] = lsrc[tid >> 7][tid & 127];  // published by the first barrier
-  // the centre norm's epsilon: a device value when the contraction is length-divided
-  const float eps_out = eps_out_dev ? *eps_out_dev : eps;
   WFrag fg, fo;
-  load_wfrag(fg, wg, 32 * cb, li, g);
-  load_wfrag(fo, wo, 32 * cb, li, g);
-  settle(fg);
-  settle(fo);
+  float eps_out;
   const int njb = (n + kPT - 1) / kPT;
   const int64_t plane = (int64_t)np * np;
   const int ntiles = batch * n * njb;
@@ -526,7 +538,16 @@ __global__ __launch_bounds__(512, 2) void trimul_output(
   if ((int)blockIdx.x >= ntiles) return;
   dma(blockIdx.x, 0);
   dma(blockIdx.x + step, 1);
-  wait_vm_lds<4>();  // this wave's transfers of the first tile landed
+  // behind the transfers: the affines (published by the first barrier) and the weights
+  const float* const lsrc[4] = {ln_w, ln_b, lno_w, lno_b};
+  lnp[tid >> 7][tid & 127] = lsrc[tid >> 7][tid & 127];
+  // the centre norm's epsilon: a device value when the contraction is length-divided
+  eps_out = eps_out_dev ? *eps_out_dev : eps;
+  load_wfrag(fg, wgo, cb, lane);
+  load_wfrag(fo, wgo, 4 + cb, lane);
+  settle(fg);
+  settle(fo);
+  wait_vm_lds<0>();  // this wave's transfers of the first tiles landed
   __syncthreads();
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
@@ -606,13 +627,13 @@ static int persistent_grid(int ntiles, int per_cu) {
 
 void launch_trimul(const TrimulArgs& a, hipStream_t stream) {
   const int np = a.np;
-  const int tiles_p = a.batch * np * (np / kPT);
-  trimul_project<<<persistent_grid(tiles_p, 1), 512, 0, stream>>>(
-      a.z, a.maskf, a.ln_w, a.ln_b, a.wp, a.A, a.B, a.batch, a.n, np, a.outgoing, a.eps);
-  launch_trimul_contract(a.A, a.B, a.P, (int64_t)a.batch * 128, np, stream, a.kstages, 128);
-  const int tiles_o = a.batch * a.n * ((a.n + kPT - 1) / kPT);
-  trimul_output<<<persistent_grid(tiles_o, 1), 512, 0, stream>>>(
-      a.z, a.P, a.ln_w, a.ln_b, a.lno_w, a.lno_b, a.wg, a.wo, a.out, a.batch, a.n, np,
+  const int tiles = a.batch * a.n * ((a.n + kPT - 1) / kPT);
+  trimul_project<<<persistent_grid(tiles, 1), 512, 0, stream>>>(
+      a.z, a.mask, a.ln_w, a.ln_b, a.w_left, a.w_right, a.w_left_gate, a.w_right_gate, a.A, a.B,
+      a.w_gate, a.w_out, a.wgo, a.kstages, a.batch, a.n, np, a.outgoing, a.eps);
+  launch_trimul_contract(a.A, a.B, a.P, (int64_t)a.batch * 128, a.n, np, stream, a.kstages, 128);
+  trimul_output<<<persistent_grid(tiles, 1), 512, 0, stream>>>(
+      a.z, a.P, a.ln_w, a.ln_b, a.lno_w, a.lno_b, a.wgo, a.out, a.batch, a.n, np,
       a.residual, a.eps, a.eps_out);
 }
 
@@ -645,16 +666,16 @@ void launch_length_eps(const uint8_t* mask, int batch, int n, float eps, float* 
   length_eps<<<1, 256, 0, stream>>>(mask, batch, n, eps, eps_out);
 }
 
-void launch_trimul_contract(const bf16* A, const bf16* B, bf16* P, int64_t planes, int np,
+void launch_trimul_contract(const bf16* A, const bf16* B, bf16* P, int64_t planes, int n, int np,
                             hipStream_t stream, const int* kstages, int planes_per_batch) {
   if (np % kBT == 0) {
     const int64_t nt = np / kBT;
     trimul_contract256<<<dim3((unsigned)(nt * nt * planes)), 512, 0, stream>>>(
-        A, B, P, np, kstages, planes_per_batch);
+        A, B, P, n, np, kstages, planes_per_batch);
     return;
   }
   const int64_t nt = np / kCT;
-  trimul_contract<<<dim3((unsigned)(nt * nt * planes)), 256, 0, stream>>>(A, B, P, np, kstages,
+  trimul_contract<<<dim3((unsigned)(nt * nt * planes)), 256, 0, stream>>>(A, B, P, n, np, kstages,
                                                                         planes_per_batch);
 }
 

@@ -228,11 +228,12 @@ def test_transition_of_64_channels(rows, factor):
     assert torch.equal(inplace, got)
 
 
-@pytest.mark.parametrize("c,h", [(64, 64), (256, 256)])
-@pytest.mark.parametrize("n,lengths", [(1, [1]), (31, [31, 7]), (97, [97, 20])])
-def test_streaming_projections_at_row_and_mask_edges(c, h, n, lengths):
-    """The projections' tile walk where it can go wrong: rows shorter than a 32-row tile, rows that
-    end inside one, and a batch element whose mask leaves whole tiles without a pair."""
+@pytest.mark.parametrize("c,h", [(64, 64), (128, 128), (256, 256)])
+@pytest.mark.parametrize("n,lengths", [(1, [1]), (31, [31, 7]), (97, [97, 20]), (129, [65, 129, 1])])
+def test_projections_at_row_and_mask_edges(c, h, n, lengths):
+    """The projections' tile walk where it can go wrong: rows shorter than a tile, rows that end
+    inside one (pair 128: the fused kernels' padding to 64 and 128), and batch elements whose mask
+    leaves whole tiles or key stages without a pair."""
     z, mask = _pair(n, c, lengths, seed=n + c)
     for outgoing in (True, False):
         m = randomise(factories.triangle_multiplication(c, outgoing=outgoing, d_hidden=h), seed=n + h).cuda()
@@ -244,3 +245,18 @@ def test_streaming_projections_at_row_and_mask_edges(c, h, n, lengths):
         m.set_backend("hip")
         want = ps.triangle_attention(z, mask, m.state_dict(), n_head=4, starting=starting, dtype=torch.float64) - z.double()
         _check(hip_delta(m, z.cuda(), mask.cuda()).cpu(), want, _pairs(mask), f"triattn c={c} n={n} starting={starting}")
+
+
+def test_fused_ops_take_parameters_of_any_fp32_alignment():
+    """Parameters that are slices of a flat buffer (4-byte aligned only), as a loader may hand out."""
+    z, mask = _pair(40, 128, [33], seed=3)
+    for m in (factories.triangle_multiplication(128, outgoing=True),
+              factories.triangle_attention(128, 4, starting=False, model="af3")):
+        m = randomise(m, seed=5).cuda()
+        m.set_backend("hip")
+        want = m(z.cuda(), mask.cuda())
+        for p in m.parameters():
+            flat = torch.empty(p.numel() + 1, device="cuda", dtype=p.dtype)
+            flat[1:].copy_(p.detach().reshape(-1))
+            p.data = flat[1:].view_as(p)
+        assert torch.equal(m(z.cuda(), mask.cuda()), want)
