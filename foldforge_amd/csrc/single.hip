@@ -46,10 +46,14 @@ __device__ __forceinline__ int vkey_pos(int key) {
 // D[o][m] = sum_k W[o][k] X[m][k] over 32 rows of X per workgroup: A = W rows (fp32 parameters,
 // converted in registers), B = X rows. The workgroup's 8 waves cover NO output tiles of 32
 // with KS waves each (NO * KS = 8): the KS waves of a tile split k in groups of 64 (part p
-// takes groups p, p + KS, ...), keep the next group's global loads in flight while
-// multiplying the current one, and add their partial tiles through LDS; part 0 runs the
-// epilogue. For MFMA step t of a group, lane half g supplies k = 64 kg + 32 g + 8 t + (0..7)
-// of both operands.
+// takes groups p, p + KS, ...), keep two groups of global loads in flight, and add their
+// partial tiles through LDS; part 0 runs the epilogue. Weight rows and fp32 x rows are loaded 128
+// bytes of 8 rows at a time and turned into operands in a wave-private LDS tile: loaded in operand
+// order (a row per lane), an instruction touches 64 cache lines. q / k / v / gate of 201 tokens x
+// 384: 15.4 -> 13.3 us; squeeze (k 1536) and expand of 97 tokens 14.8 -> 10.0 and 17.2 -> 13.9;
+// transition of 2000 rows x 384 87 -> 73. Three groups in flight (96 VGPRs) ran one workgroup per
+// CU and 2-5% slower than two. Bound by its dependent chain at these sizes: launch, LayerNorm,
+// one L2 latency per pair of groups, reduction, epilogue.
 // Precision: activations enter as fp32 and are split into bf16 hi + lo (two MFMAs); the weights
 // are rounded to bf16, or with w_split also split into hi + lo (a third MFMA, lo x hi: the
 // products then carry about fp32 accuracy, the lo x lo term below it dropped). The single-track
@@ -63,10 +67,13 @@ __device__ __forceinline__ int vkey_pos(int key) {
 // (acc[4 v + e]).
 
 constexpr int kGemmWaves = 8;
+constexpr int kTurnTile = 2 * 32 * 32;  // a wave's LDS tile: 32 rows x 32 k, hi then lo
+__device__ __forceinline__ int turn_off(int r, int p) { return r * 32 + 8 * (p ^ ((r >> 2) & 3)); }
 
 size_t row_gemm_lds(int xsrc, int K, int no) {
+  const size_t tiles = (size_t)kGemmWaves * (xsrc == kXLn ? 1 : 2) * kTurnTile * sizeof(bf16);
   const size_t red = (size_t)(kGemmWaves - no) * 64 * 16 * sizeof(float);
-  return xsrc == kXLn ? red + (size_t)2 * 32 * (K + 8) * sizeof(bf16) : red;
+  return tiles + red + (xsrc == kXLn ? (size_t)2 * 32 * (K + 8) * sizeof(bf16) : 0);
 }
 
 // The input row of logical row m under the row map a.tmap (see kMap* in ffk_kernels.h).
@@ -375,9 +382,12 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
 template <int EPI, int XSRC, int NO>
 __global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
   constexpr int KS = kGemmWaves / NO;
+  constexpr int kTurns = XSRC == kXLn ? 1 : 2;  // tiles per wave: weights, fp32 x rows
+  constexpr int kAhead = 2;                     // groups in flight
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* red = reinterpret_cast<float*>(smem);  // [NO][KS - 1][64][16]
-  bf16* xs_hi = reinterpret_cast<bf16*>(smem + (kGemmWaves - NO) * 64 * 16 * sizeof(float));
+  bf16* turns = reinterpret_cast<bf16*>(smem);  // [kGemmWaves][kTurns][kTurnTile]
+  float* red = reinterpret_cast<float*>(turns + kGemmWaves * kTurns * kTurnTile);  // [NO][KS - 1][64][16]
+  bf16* xs_hi = reinterpret_cast<bf16*>(red + (kGemmWaves - NO) * 64 * 16);
   const int xstride = a.K + 8;  // [32][K + 8]: rows 16 bytes apart modulo 256, conflict-free
   bf16* xs_lo = xs_hi + 32 * xstride;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, g = lane >> 5;
@@ -385,24 +395,52 @@ __global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
   const int ot = blockIdx.y * NO + osub;
   const bool active = ot * 32 < a.O;
   const int64_t m0 = (int64_t)blockIdx.x * 32;
-  const int G = a.K / 64;
+  const int G = a.K / 64, ng = active && part < G ? (G - part + KS - 1) / KS : 0;
 
+  // this lane's loads: k 4 (lane % 8) .. of each 32, of rows 8 u + lane / 8, u = 0 .. 3 (packed
+  // tiles take rows 16-31 from a second matrix: a pointer per 16 rows)
   int seg, cbase;
-  const float* wr = tile_weight_row<EPI>(a, ot, li, seg, cbase);
-  wr += 32 * g;
-  const float* x32 = a.x32 + mapped_row(a, m0 + li) * a.K + 32 * g;
+  const int kq = 4 * (lane & 7), row8 = lane >> 3;
+  const float* wr[2];
+  const float* xr4[4];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) wr[u] = tile_weight_row<EPI>(a, ot, 16 * u + row8, seg, cbase) + kq;
+  if (XSRC == kXF32) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) xr4[u] = a.x32 + mapped_row(a, m0 + 8 * u + row8) * a.K + kq;
+  }
+  bf16* wt = turns + wave * kTurns * kTurnTile;
+  bf16* xt = wt + kTurnTile;
 
   f32x16 acc = zero16();
-  f32x4 wc[8], wn[8], xc[8], xn[8];
-  auto fetch = [&](int kg, f32x4* w, f32x4* x) {
+  f32x4 wv[kAhead][8], xv4[kAhead][XSRC == kXF32 ? 8 : 1];
+  auto fetch = [&](int i, f32x4* w, f32x4* x) __attribute__((always_inline)) {
+    const int k = 64 * (part + KS * i);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) w[q] = *reinterpret_cast<const f32x4*>(wr + 64 * kg + 4 * q);
-    if (XSRC == kXF32) {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) x[q] = *reinterpret_cast<const f32x4*>(x32 + 64 * kg + 4 * q);
+    for (int q = 0; q < 8; ++q) {
+      const int h = q >> 2, u = q & 3;
+      w[q] = *reinterpret_cast<const f32x4*>(wr[u >> 1] + (int64_t)(8 * (u & 1)) * a.K + k + 32 * h);
+      if (XSRC == kXF32) x[q] = *reinterpret_cast<const f32x4*>(xr4[u] + k + 32 * h);
     }
   };
-  if (active && part < G) fetch(part, wc, xc);
+  // rows 8 u + lane / 8 of one 32-k half into a tile, hi and (lo_on) lo
+  auto turn = [&](const f32x4* v, bf16* tile, bool lo_on) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      bf16x4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        hi[e] = (bf16)v[u][e];
+        lo[e] = (bf16)(v[u][e] - (float)hi[e]);
+      }
+      const int at = turn_off(8 * u + row8, kq >> 3) + (kq & 4);
+      *reinterpret_cast<bf16x4*>(tile + at) = hi;
+      if (lo_on) *reinterpret_cast<bf16x4*>(tile + 32 * 32 + at) = lo;
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s)
+    if (s < ng) fetch(s, wv[s], xv4[s]);
 
   if (XSRC == kXLn) {
     // thread t normalises row t / 16, chunks (t % 16) + 16 i of 8 channels, held in registers;
@@ -458,33 +496,41 @@ __global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
     __syncthreads();
   }
 
-  if (active) {
-    for (int kg = part; kg < G; kg += KS) {
-      const bool more = kg + KS < G;
-      if (more) fetch(kg + KS, wn, xn);
+  // (LDS operations of a wave complete in order: a tile is rewritten behind its reads)
+  auto consume = [&](int i, const f32x4* w, const f32x4* x) __attribute__((always_inline)) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        bf16x8 whi, wlo, xhi, xlo;
-        split8(wc[2 * t], wc[2 * t + 1], whi, wlo);
+    for (int h = 0; h < 2; ++h) {
+      turn(w + 4 * h, wt, a.w_split != 0);
+      if (XSRC == kXF32) turn(x + 4 * h, xt, true);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int at = turn_off(li, 2 * t + g);
+        bf16x8 xhi, xlo;
         if (XSRC == kXLn) {
-          const int k = 64 * kg + 32 * g + 8 * t;
-          xhi = *reinterpret_cast<const bf16x8*>(xs_hi + li * xstride + k);
-          xlo = *reinterpret_cast<const bf16x8*>(xs_lo + li * xstride + k);
+          const int k = 64 * (part + KS * i) + 32 * h + 16 * t + 8 * g;
+          xhi = ld8(xs_hi + li * xstride + k);
+          xlo = ld8(xs_lo + li * xstride + k);
         } else {
-          split8(xc[2 * t], xc[2 * t + 1], xhi, xlo);
+          xhi = ld8(xt + at);
+          xlo = ld8(xt + 32 * 32 + at);
         }
+        const bf16x8 whi = ld8(wt + at);
         acc = mfma32(whi, xlo, acc);
         acc = mfma32(whi, xhi, acc);
-        if (a.w_split) acc = mfma32(wlo, xhi, acc);
+        if (a.w_split) acc = mfma32(ld8(wt + 32 * 32 + at), xhi, acc);
       }
-      if (more) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          wc[q] = wn[q];
-          xc[q] = xn[q];
-        }
-      }
+      __builtin_amdgcn_wave_barrier();
     }
+  };
+#pragma unroll 1
+  for (int i = 0; i < ng; i += kAhead) {
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s)
+      if (i + s < ng) {
+        consume(i + s, wv[s], xv4[s]);
+        if (i + s + kAhead < ng) fetch(i + s + kAhead, wv[s], xv4[s]);
+      }
   }
   if (KS > 1) {
     if (part > 0) {
