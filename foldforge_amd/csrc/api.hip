@@ -259,15 +259,29 @@ int64_t pad32(int64_t n) { return (n + 31) / 32 * 32; }
 int64_t pad64(int64_t n) { return (n + 63) / 64 * 64; }
 
 struct PwaWs {
-  bf16 *vt, *gate, *w, *og;
+  bf16 *vt, *gate, *w, *og, *wo;
   float* logits;
   size_t bytes;
 };
-PwaWs pwa_ws(void* ws, int64_t batch, int64_t depth, int64_t n, int heads, int dh) {
+// The shapes of pwa_fused (8 waves, a head each; whole heads in a 32-row operand tile).
+bool pwa_fused_shape(int cm, int heads, int dh) {
+  return cm == 64 && heads == 8 && (dh == 8 || dh == 16 || dh == 32);
+}
+PwaWs pwa_ws(void* ws, int64_t batch, int64_t depth, int64_t n, int cm, int heads, int dh) {
   Carver cv{static_cast<char*>(ws)};
   const int64_t np = pad64(n);
   const size_t tok = (size_t)batch * depth * n * heads * dh;
-  PwaWs w;
+  PwaWs w{};
+  if (pwa_fused_shape(cm, heads, dh)) {
+    const int64_t s = 32 / dh;  // MSA rows of an operand tile
+    w.vt = cv.take<bf16>((size_t)batch * heads * ((depth + s - 1) / s) * 32 * np);
+    w.gate = cv.take<bf16>(tok);
+    w.logits = cv.take<float>((size_t)batch * heads * n * np);
+    w.w = cv.take<bf16>((size_t)batch * heads * pad32(n) * np);
+    w.wo = cv.take<bf16>((size_t)64 * heads * dh);
+    w.bytes = cv.used;
+    return w;
+  }
   w.vt = cv.take<bf16>((size_t)batch * heads * depth * dh * np);
   w.gate = cv.take<bf16>(tok);
   w.logits = cv.take<float>((size_t)batch * heads * n * np);
@@ -1190,7 +1204,7 @@ size_t ffk_msa_pair_weighted_averaging_workspace(int64_t batch, int64_t depth, i
                                                   int32_t d_head) {
   if (batch <= 0 || depth <= 0 || n <= 0 || d_msa <= 0 || d_pair <= 0 || n_head <= 0 || d_head <= 0)
     return 0;
-  return pwa_ws(nullptr, batch, depth, n, n_head, d_head).bytes;
+  return pwa_ws(nullptr, batch, depth, n, d_msa, n_head, d_head).bytes;
 }
 
 int32_t ffk_msa_pair_weighted_averaging(
@@ -1216,10 +1230,10 @@ int32_t ffk_msa_pair_weighted_averaging(
   if (!aligned16(m) || !aligned16(z) || !aligned16(out) || !aligned16(w_value) ||
       !aligned16(w_gate) || !aligned16(w_out))
     return fail(FFK_ERR_INVALID, "msa_pair_weighted_averaging: m/z/out and the projection weights must be 16-byte aligned");
-  const PwaWs need = pwa_ws(nullptr, batch, depth, n, n_head, d_head);
+  const PwaWs need = pwa_ws(nullptr, batch, depth, n, d_msa, n_head, d_head);
   if (!workspace || workspace_bytes < need.bytes || !aligned16(workspace))
     return fail(FFK_ERR_WORKSPACE, "msa_pair_weighted_averaging: workspace %zu bytes < %zu", workspace_bytes, need.bytes);
-  const PwaWs w = pwa_ws(workspace, batch, depth, n, n_head, d_head);
+  const PwaWs w = pwa_ws(workspace, batch, depth, n, d_msa, n_head, d_head);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t rows = batch * depth * n;
   const int64_t np = pad64(n);
@@ -1242,6 +1256,8 @@ int32_t ffk_msa_pair_weighted_averaging(
   p.heads = n_head;
   p.dh = d_head;
   p.depth = (int)depth;
+  const bool fused = pwa_fused_shape(d_msa, n_head, d_head);
+  p.v_frag = fused ? 1 : 0;
   launch_row_gemm(p, kEpiPwa, kXLn, st);
 
   PairBiasArgs pb{};
@@ -1259,12 +1275,33 @@ int32_t ffk_msa_pair_weighted_averaging(
   pb.transposed = 0;
   launch_apb_pair_bias(pb, st);
 
-  PwaSoftmaxArgs sm;
+  PwaSoftmaxArgs sm{};
   sm.logits = w.logits;
   sm.w = w.w;
   sm.rows = batch * n_head * n;
   sm.np = (int)np;
+  sm.n = (int)n;
+  sm.frag = fused ? 1 : 0;
+  sm.hd = (int)hd;
+  sm.w_out = w_out;
+  sm.wo = w.wo;
   launch_pwa_softmax(sm, st);
+  if (fused) {
+    PwaFusedArgs f;
+    f.vt = w.vt;
+    f.w = w.w;
+    f.wo = w.wo;
+    f.gate = w.gate;
+    f.res = residual ? static_cast<const bf16*>(m) : nullptr;
+    f.out = static_cast<bf16*>(out);
+    f.batch = (int)batch;
+    f.depth = (int)depth;
+    f.n = (int)n;
+    f.np = (int)np;
+    f.dh = d_head;
+    launch_pwa_fused(f, st);
+    return check_launch("msa_pair_weighted_averaging");
+  }
 
   PwaAverageArgs av;
   av.vt = w.vt;

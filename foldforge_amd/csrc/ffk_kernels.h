@@ -183,6 +183,8 @@ struct RowGemmArgs {
   // kEpiPwa: w0 = to_value, w1 = to_gate ([hd][K] each, O = 2 hd); tokens m = (b S + s) n + j;
   // v^T [batch][heads][S][dh][np] (bf16, keys contiguous), gate = sigmoid(x W_g^T) [M][hd]
   int depth;
+  // row_stream with v_frag = 1 (dh 8, 16 or 32): v^T in pwa_fused's fragment order instead
+  int v_frag;
   // kEpiOpm: w0 = to_left, w1 = to_right ([32][K] each, O = 64), bias0 / bias1 their biases
   // (NULL: none). Logical rows m = (b n + j) sp + s (s < sp, sp % 32 == 0) read MSA row
   // (b depth + s) n + j; rows with s >= depth, or masked in rows_mask [batch][depth][n],
@@ -299,6 +301,11 @@ struct PwaSoftmaxArgs {
   bf16* w;              // [batch][heads][n][np] softmax weights, 0 at masked / padding keys
   int64_t rows;         // batch * heads * n
   int np;
+  // frag = 1: the weights in pwa_fused's fragment order instead (queries padded to 32), and
+  // w_out [64][hd] packed behind them into wo (see pwa_fused)
+  int frag, n, hd;
+  const float* w_out;
+  bf16* wo;
 };
 void launch_pwa_softmax(const PwaSoftmaxArgs& a, hipStream_t stream);
 
@@ -310,6 +317,18 @@ struct PwaAverageArgs {
   int batch, heads, depth, n, np, dh;
 };
 void launch_pwa_average(const PwaAverageArgs& a, hipStream_t stream);
+// The average of 8 heads of 8, 16 or 32 channels, gated, projected to 64 channels and added to the
+// residual, in one kernel.
+struct PwaFusedArgs {
+  const bf16* vt;    // values in fragment order (RowGemmArgs::v_frag)
+  const bf16* w;     // softmax weights in fragment order (PwaSoftmaxArgs::frag)
+  const bf16* wo;    // packed output projection
+  const bf16* gate;  // [batch][S][n][8 dh]
+  const bf16* res;   // [batch][S][n][64] or NULL
+  bf16* out;         // [batch][S][n][64]; may alias res
+  int batch, depth, n, np, dh;
+};
+void launch_pwa_fused(const PwaFusedArgs& a, hipStream_t stream);
 
 // Outer product mean (opm.hip). For every pair (i, j): o[(c, e)] = sum_s l[s][i][c] r[s][j][e]
 // over the MSA rows, out = (o W^T scale1 + bias) scale2 with the count n_ij = sum_s

@@ -10,8 +10,9 @@
 //   row_gemm<kEpiPwa, kXLn> (single.hip): LN_msa + value / gate projections -> v^T, gate
 //   apb_pair_bias (single.hip): pair logits in log2 units, masked keys very negative
 //   pwa_softmax: the softmax of every (batch, head, query) row -> bf16 weights
-//   pwa_average: the per-head GEMM, gated -> fp32 (gate * o)
-//   row_gemm<kEpiResid, kXF32>: the output projection and the residual.
+//   8 heads of 8, 16 or 32 channels on 64 MSA channels: pwa_fused, everything behind the softmax
+//   in one kernel; other shapes: pwa_average, the per-head GEMM, gated -> bf16 (gate * o), and
+//   row_gemm<kEpiResid, kXLn>, the output projection and the residual.
 #include "ffk_device.h"
 #include "ffk_kernels.h"
 
@@ -26,9 +27,24 @@ constexpr float kNoKey = -1e29f;
 __global__ __launch_bounds__(256) void pwa_softmax(PwaSoftmaxArgs a) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + wave;
-  if (row >= a.rows) return;
+  if (row >= a.rows) {
+    // frag: the workgroups behind the rows pack the output projection, a 16-byte piece per thread
+    const int64_t idx = ((int64_t)blockIdx.x - (a.rows + 3) / 4) * 256 + threadIdx.x;
+    if (a.frag && idx >= 0 && idx < 8 * a.hd) {
+      const int l = (int)idx & 63, t = (int)(idx >> 6), kt = t % (a.hd / 16), ot = t / (a.hd / 16);
+      const float* src = a.w_out + (32 * ot + (l & 31)) * a.hd + 16 * kt + 8 * (l >> 5);
+      bf16x8 v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = (bf16)src[e];
+      *reinterpret_cast<bf16x8*>(a.wo + idx * 8) = v;
+    }
+    return;
+  }
   const float* x = a.logits + row * a.np;
   bf16* w = a.w + row * a.np;
+  const int64_t bh = row / a.n;
+  const int q = (int)(row - bh * a.n);
+  if (a.frag) w = a.w + ((bh * ((a.n + 31) / 32) + q / 32) * (a.np / 16)) * 512 + (q & 31) * 8;
   float mx = -INFINITY;
   for (int j = 4 * lane; j < a.np; j += 256) {
     const f32x4 v = *reinterpret_cast<const f32x4*>(x + j);
@@ -49,7 +65,136 @@ __global__ __launch_bounds__(256) void pwa_softmax(PwaSoftmaxArgs a) {
     bf16x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = (bf16)(fast_exp2(v[e] - mx) * inv);
-    *reinterpret_cast<bf16x4*>(w + j) = o;
+    *reinterpret_cast<bf16x4*>(w + (a.frag ? (j >> 4) * 512 + ((j >> 3) & 1) * 256 + (j & 7) : j)) = o;
+  }
+}
+
+// The weighted average, gate, output projection and residual for 8 heads of DH = 8, 16 or 32
+// channels and 64 MSA channels. A workgroup of 8 waves takes S = 32 / DH MSA rows x 128 queries:
+//   wave h: O_h[(s, d)][q] = sum_j v^T_h[(s, d)][j] w_h[q][j], one 32-row A tile (the head's S
+//   rows) x 4 query tiles, both operands straight from memory in fragment order (a 16-key step of
+//   a tile is one contiguous KB: [tile][k / 16][lane][8]), two steps fetched ahead;
+//   the averages go to LDS as bf16 token rows [(s, q)][8 DH] (64 KB for every DH, 16-byte pieces
+//   XOR-swizzled by row);
+//   then each wave projects its share of the (token tile, 32-channel output tile) pairs: gate
+//   times the LDS rows as the B operand, W_out fragments as A; residual and 16-byte stores.
+// Rows past the depth and queries past n hold whatever the operands held: they are not stored
+// and no product mixes rows or queries. This replaces a 128 x 128-tile GEMM per head, its gated
+// output in memory and a token-row GEMM: 512 x 256 tokens, 8 x 8: 50 -> 18 us. Bound by the
+// fragment traffic from L2 (640 KB a workgroup at 256 keys).
+template <int DH>
+__global__ __launch_bounds__(512) void pwa_fused(PwaFusedArgs a) {
+  constexpr int S = 32 / DH, HD = 8 * DH, KT = HD / 16, PC = HD / 8;
+  constexpr int kTiles = 4 * S;                 // token tiles of 32
+  constexpr int kPer = 2 * kTiles / 8;          // (token tile, output tile) pairs per wave
+  __shared__ __attribute__((aligned(16))) bf16 os[S * 128 * HD];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = a.n, nqt = (n + 127) / 128, sbn = (a.depth + S - 1) / S, nk = a.np / 16;
+  const uint32_t wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int qt = (int)(wg % nqt);
+  const int64_t bs = wg / nqt;
+  const int64_t b = bs / sbn;
+  const int s0 = (int)(bs - b * sbn) * S, q0 = qt * 128;
+  auto piece = [](int row, int p) { return row * HD + 8 * (p ^ (HD == 64 ? (row >> 1) & 7 : row & (PC - 1) & 15)); };
+
+  const bf16* A = a.vt + (((b * 8 + wave) * sbn + s0 / S) * nk) * 512 + lane * 8;
+  const bf16* B[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)  // query tiles past n re-read the last one
+    B[t] = a.w + (((b * 8 + wave) * ((n + 31) / 32) + min(q0 / 32 + t, (n - 1) / 32)) * nk) * 512 + lane * 8;
+  f32x16 acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = zero16();
+  bf16x8 fa[2][2], fb[2][2][4];
+  auto fetch = [&](int k, bf16x8 (&x)[2], bf16x8 (&y)[2][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      x[u] = ld8(A + (k + u) * 512);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) y[u][t] = ld8(B[t] + (k + u) * 512);
+    }
+  };
+  auto multiply = [&](const bf16x8 (&x)[2], const bf16x8 (&y)[2][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[t] = mfma32(x[u], y[u][t], acc[t]);
+  };
+  // np is a multiple of 64: steps in whole groups of 4
+  fetch(0, fa[0], fb[0]);
+#pragma unroll 1
+  for (int k = 0; k < nk; k += 4) {
+    fetch(k + 2, fa[1], fb[1]);
+    multiply(fa[0], fb[0]);
+    if (k + 4 < nk) fetch(k + 4, fa[0], fb[0]);
+    multiply(fa[1], fb[1]);
+  }
+
+  // this wave's token tiles and output tiles: pairs kPer wave .. + kPer - 1 of (tile, half); the
+  // gate of its token rows travels while the averages are published
+  constexpr int kRt = kPer >= 2 ? kPer / 2 : 1;  // token tiles of this wave
+  const int rt0 = kPer >= 2 ? wave * kRt : wave >> 1;
+  bf16x8 gv[kRt][KT];
+  int64_t tok[kRt];
+  bool real[kRt];
+#pragma unroll
+  for (int i = 0; i < kRt; ++i) {
+    const int row = 32 * (rt0 + i) + li, s = s0 + row / 128, q = q0 + row % 128;
+    real[i] = s < a.depth && q < n;
+    tok[i] = (b * a.depth + min(s, a.depth - 1)) * n + min(q, n - 1);
+#pragma unroll
+    for (int t = 0; t < KT; ++t) gv[i][t] = ld8(a.gate + tok[i] * HD + 16 * t + 8 * g);
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    float y[2][8];
+    acc_pieces(acc[t], y);  // y[k]: rows (s, d) 8 (2 k + g) .. + 7 of query li
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int r = 8 * (2 * k + g), s = r / DH, d = r % DH;
+      bf16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (bf16)y[k][e];
+      *reinterpret_cast<bf16x8*>(&os[piece(s * 128 + 32 * t + li, (wave * DH + d) / 8)]) = o;
+    }
+  }
+  __syncthreads();
+
+#pragma unroll
+  for (int i = 0; i < kRt; ++i) {
+    const int row = 32 * (rt0 + i) + li;
+    bf16x8 x[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      const bf16x8 o = ld8(&os[piece(row, 2 * t + g)]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[t][e] = (bf16)((float)o[e] * (float)gv[i][t][e]);
+    }
+#pragma unroll
+    for (int u = 0; u < (kPer >= 2 ? 2 : 1); ++u) {
+      const int ot = kPer >= 2 ? u : wave & 1;
+      f32x16 y = zero16();
+#pragma unroll
+      for (int t = 0; t < KT; ++t) y = mfma32(ld8(a.wo + ((ot * KT + t) * 64 + lane) * 8), x[t], y);
+      float p[2][8];
+      acc_pieces(y, p);
+      if (!real[i]) continue;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int64_t at = tok[i] * 64 + 32 * ot + 8 * (2 * k + g);
+        bf16x8 o;
+        if (a.res) {
+          const bf16x8 r = ld8(a.res + at);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) o[e] = (bf16)(p[k][e] + (float)r[e]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) o[e] = (bf16)p[k][e];
+        }
+        *reinterpret_cast<bf16x8*>(a.out + at) = o;
+      }
+    }
   }
 }
 
@@ -223,7 +368,19 @@ __global__ __launch_bounds__(256) void pwa_average(PwaAverageArgs a) {
 }  // namespace
 
 void launch_pwa_softmax(const PwaSoftmaxArgs& a, hipStream_t stream) {
-  pwa_softmax<<<dim3((unsigned)((a.rows + 3) / 4)), 256, 0, stream>>>(a);
+  const int64_t packs = a.frag ? (8 * a.hd + 255) / 256 : 0;
+  pwa_softmax<<<dim3((unsigned)((a.rows + 3) / 4 + packs)), 256, 0, stream>>>(a);
+}
+
+void launch_pwa_fused(const PwaFusedArgs& a, hipStream_t stream) {
+  const int S = 32 / a.dh;
+  const int64_t blocks = (int64_t)((a.n + 127) / 128) * ((a.depth + S - 1) / S) * a.batch;
+  if (a.dh == 8)
+    pwa_fused<8><<<dim3((unsigned)blocks), 512, 0, stream>>>(a);
+  else if (a.dh == 16)
+    pwa_fused<16><<<dim3((unsigned)blocks), 512, 0, stream>>>(a);
+  else
+    pwa_fused<32><<<dim3((unsigned)blocks), 512, 0, stream>>>(a);
 }
 
 void launch_pwa_average(const PwaAverageArgs& a, hipStream_t stream) {

@@ -974,6 +974,23 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
         if (ot * 32 < hd) {
           const f32x16 y = product(ot - ot0, true);
           const int c = ot * 32 + li, hh = (int)(((uint32_t)c * inv) >> 24), d = c - hh * a.dh;
+          if (a.v_frag) {
+            // row (s % S) dh + d of the head's S MSA rows, S = 32 / dh: 16-byte pieces of 8 keys
+            const int sh = 5 - __builtin_ctz(a.dh), sb = (a.depth + (1 << sh) - 1) >> sh;
+            bf16* dst = a.vt +
+                        ((((int64_t)tr.b * a.heads + hh) * sb + (tr.r >> sh)) * (a.np >> 4) + (tr.rem >> 4)) * 512 +
+                        (32 * g + (int)(tr.r & ((1u << sh) - 1)) * a.dh + d) * 8;
+            float p[2][8];
+            acc_pieces(y, p);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              bf16x8 o;
+#pragma unroll
+              for (int e = 0; e < 8; ++e) o[e] = (bf16)p[k][e];
+              *reinterpret_cast<bf16x8*>(dst + 512 * k) = o;
+            }
+            continue;
+          }
           store_rows(a.vt + ((((int64_t)tr.b * a.heads + hh) * a.depth + tr.r) * a.dh + d) * a.np + tr.rem, y);
         } else {
           const f32x16 acc = product(ot - ot0, false);

@@ -74,6 +74,19 @@ def test_msa_pair_weighted_averaging_matches_oracle(cm, heads, dh, depth, n, len
     _check(full, want + msa.double(), "msa_pwa residual")
 
 
+@pytest.mark.parametrize("dh", [8, 16, 32])
+@pytest.mark.parametrize("depth,n,lengths", [(1, 1, [1]), (5, 33, [20]), (2, 129, [129, 77]), (9, 200, [200])])
+def test_msa_pair_weighted_averaging_of_eight_heads_at_tile_edges(dh, depth, n, lengths):
+    """The one-kernel form: MSA rows that do not fill an operand tile (4, 2 or 1 rows), queries past
+    the last 32- and 128-query tile."""
+    msa, z, mask = _inputs(depth, n, 64, lengths, seed=n + dh)
+    mod = _pwa(64, 8, dh, seed=dh + depth)
+    want = ps.msa_pair_weighted_averaging(msa, z, mask, mod.state_dict(), n_head=8,
+                                          dtype=torch.float64) - msa.double()
+    _check(hip_delta(mod, msa.cuda(), z.cuda(), mask.cuda()).cpu(), want, f"msa_pwa 8x{dh} S={depth} n={n}")
+    _check(hip_forward(mod, msa.cuda(), z.cuda(), mask.cuda()).cpu(), want + msa.double(), "msa_pwa residual")
+
+
 @pytest.mark.parametrize("heads,dh", [(1, 256), (3, 64)])
 @pytest.mark.parametrize("n", [1, 31, 65])
 def test_msa_pair_weighted_averaging_wide_heads_and_broken_key_runs(heads, dh, n):
