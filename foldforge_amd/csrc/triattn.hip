@@ -95,21 +95,14 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
   const bool key_major = !starting && !transposed_bias;
   const int nsb = (n + kPT - 1) / kPT, rows = (n + 31) & ~31;
   const int64_t nb = np / 32;
-  const int ntiles = batch * rows * nsb;
-  auto where = [&](int tile, int& b, int& r, int& s0, int& valid) {
-    const int sb = tile % nsb;
-    r = (tile / nsb) % rows;
-    b = tile / (nsb * rows);
-    s0 = sb * kPT;
-    valid = (r < n) ? min(kPT, n - s0) : 0;
-  };
+  auto valid_of = [&](const TileAt& t) { return t.r < n ? min(kPT, n - t.blk * kPT) : 0; };
   // This wave's 2 one-KB pieces (positions 8 wave .. 8 wave + 7) of a tile's z rows into ring
   // slot buf (positions past the end re-read a real row, zeroed by the LayerNorm); wave 7
-  // also fetches the tile's 64 key-mask values. A tile index past the end fetches tile 0
-  // again, so that every wave always has the same number of transfers in flight.
-  auto z_dma = [&](int tile, int buf) {
-    int b, r, s0, valid;
-    where(tile < ntiles ? tile : 0, b, r, s0, valid);
+  // also fetches the tile's 64 key-mask values. A tile past the end fetches tile 0 again, so
+  // that every wave always has the same number of transfers in flight.
+  auto z_dma = [&](TileAt t, int buf) {
+    if (t.b >= batch) t = TileAt{0, 0, 0};
+    const int b = t.b, r = t.r, s0 = t.blk * kPT, valid = valid_of(t);
     const bf16* base = z;
     uint32_t stride = 256;  // bytes between consecutive positions
     if (valid > 0) {
@@ -132,10 +125,14 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
       dma1(mask + (int64_t)b * n, (uint32_t)min(key_major ? r : s0 + lane, n - 1), lds_addr(&keep[buf][0]));
     }
   };
-  const int step = gridDim.x;
-  if ((int)blockIdx.x >= ntiles) return;
-  z_dma(blockIdx.x, 0);
-  z_dma(blockIdx.x + step, 1);
+  if ((int)blockIdx.x >= batch * rows * nsb) return;
+  // the walk advances by the grid stride with adds and carries (see TileAt)
+  const TileAt step = tile_at(gridDim.x, nsb, rows);
+  TileAt cur = tile_at(blockIdx.x, nsb, rows);
+  TileAt nxt = tile_add(cur, step, nsb, rows);
+  TileAt far = tile_add(nxt, step, nsb, rows);
+  z_dma(cur, 0);
+  z_dma(nxt, 1);
   // published by the first barrier
   if (tid < 256) lnp[tid >> 7][tid & 127] = (tid < 128 ? ln_w : ln_b)[tid & 127];
   wbl[tid] = (bf16)(w_bias[tid] * kLog2e);  // H * 128 = the workgroup's threads
@@ -159,18 +156,13 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
   if (qk) settle(w1);
   wait_vm_lds<0>();  // this wave's transfers of the first tiles landed
   __syncthreads();
-  {
-    int b, r, s0, valid;
-    where(blockIdx.x, b, r, s0, valid);
-    ln_inplace_swz<kPT, 512>(zt[0], valid, lnp[0], lnp[1], eps);
-  }
+  ln_inplace_swz<kPT, 512>(zt[0], valid_of(cur), lnp[0], lnp[1], eps);
   const int sw = (li >> 2) & 3;  // 16-byte column swizzle of a staged q / k row
   const int swv = (li >> 1) & 7;  // of a staged v^T row
   int buf = 0, k = 0;
 #pragma unroll 1
-  for (int tile = blockIdx.x; tile < ntiles; tile += step, ++k, buf = buf == NB - 1 ? 0 : buf + 1) {
-    int b, r, s0, valid;
-    where(tile, b, r, s0, valid);
+  for (; cur.b < batch; ++k, buf = buf == NB - 1 ? 0 : buf + 1) {
+    const int b = cur.b, r = cur.r, s0 = cur.blk * kPT;
     const int nbuf = buf == NB - 1 ? 0 : buf + 1, fbuf = nbuf == NB - 1 ? 0 : nbuf + 1;
     // this wave's transfers of tile + step have landed (issued after them: only the previous
     // tile's stores, 8 on waves 0-5 and 4 on waves 6-7); the barrier publishes everyone's
@@ -182,7 +174,7 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
     else
       wait_vm_lds<4>();
     __syncthreads();
-    z_dma(tile + 2 * step, fbuf);
+    z_dma(far, fbuf);
     const bf16* xh = zt[buf];
     const int64_t bh = (int64_t)b * H + head;
     if (qk) {
@@ -271,11 +263,10 @@ __global__ __launch_bounds__(512, 2) void triattn_project(
                          ld8(&st[d * kPT + 8 * (c ^ ((d >> 1) & 7))]));
       }
     }
-    if (tile + step < ntiles) {
-      int nb2, nr, ns0, nvalid;
-      where(tile + step, nb2, nr, ns0, nvalid);
-      ln_inplace_swz<kPT, 512>(zt[nbuf], nvalid, lnp[0], lnp[1], eps);
-    }
+    if (nxt.b < batch) ln_inplace_swz<kPT, 512>(zt[nbuf], valid_of(nxt), lnp[0], lnp[1], eps);
+    cur = nxt;
+    nxt = far;
+    far = tile_add(far, step, nsb, rows);
   }
   wait_vm_lds<0>();  // no LDS write may land after exit
 }
@@ -707,21 +698,15 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cb = wave & 3, pt = wave >> 2;
   const int njb = (n + kPT - 1) / kPT;
-  const int ntiles = batch * n * njb;
-  auto where = [&](int tile, int& valid) -> int64_t {
-    const int jb = tile % njb;
-    const int i = (tile / njb) % n;
-    const int b = tile / (njb * n);
-    const int j0 = jb * kPT;
-    valid = min(kPT, n - j0);
-    return (((int64_t)b * n + i) * n + j0) * 128;
-  };
+  auto valid_of = [&](const TileAt& t) { return min(kPT, n - t.blk * kPT); };
+  auto offset_of = [&](const TileAt& t) { return (((int64_t)t.b * n + t.r) * n + t.blk * kPT) * 128; };
   // This wave's 2 one-KB pieces of the tile's z and of its o into ring slot buf (positions
-  // past the end re-read the last real one); a tile index past the end fetches tile 0 again,
-  // so every wave always has the same number of transfers in flight.
-  auto dma = [&](int tile, int buf) {
-    int valid;
-    const int64_t off = where(tile < ntiles ? tile : 0, valid);
+  // past the end re-read the last real one); a tile past the end fetches tile 0 again, so every
+  // wave always has the same number of transfers in flight.
+  auto dma = [&](TileAt t, int buf) {
+    if (t.b >= batch) t = TileAt{0, 0, 0};
+    const int valid = valid_of(t);
+    const int64_t off = offset_of(t);
     const uint32_t dz = lds_addr(&zs[buf][0]), dov = lds_addr(&os[buf][0]);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -732,10 +717,13 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
       dma16_stream(o + off, voff, dov + 1024 * piece);
     }
   };
-  const int step = gridDim.x;
-  if ((int)blockIdx.x >= ntiles) return;
-  dma(blockIdx.x, 0);
-  dma(blockIdx.x + step, 1);
+  if ((int)blockIdx.x >= batch * n * njb) return;
+  const TileAt step = tile_at(gridDim.x, njb, n);
+  TileAt cur = tile_at(blockIdx.x, njb, n);
+  TileAt nxt = tile_add(cur, step, njb, n);
+  TileAt far = tile_add(nxt, step, njb, n);
+  dma(cur, 0);
+  dma(nxt, 1);
   // behind the transfers: affine and biases (published by the first barrier; absent biases are
   // zeros) and the weights
   if (tid < 256) {
@@ -751,11 +739,7 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
   settle(fo);
   wait_vm_lds<0>();  // this wave's transfers of the first tiles landed
   __syncthreads();
-  {
-    int valid;
-    where(blockIdx.x, valid);
-    ln_swz<kPT, 512>(zs[0], xh[0], valid, lnp[0], lnp[1], eps);
-  }
+  ln_swz<kPT, 512>(zs[0], xh[0], valid_of(cur), lnp[0], lnp[1], eps);
   const int p0 = 32 * pt + li;  // this lane's position in both products
   int buf = 0, k = 0, prev_valid = kPT, last_buf = 0;
   int64_t prev_off = 0;
@@ -769,9 +753,9 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
     }
   };
 #pragma unroll 1
-  for (int tile = blockIdx.x; tile < ntiles; tile += step, ++k, buf = buf == NB - 1 ? 0 : buf + 1) {
-    int valid;
-    const int64_t off = where(tile, valid);
+  for (; cur.b < batch; ++k, buf = buf == NB - 1 ? 0 : buf + 1) {
+    const int valid = valid_of(cur);
+    const int64_t off = offset_of(cur);
     const int nbuf = buf == NB - 1 ? 0 : buf + 1, fbuf = nbuf == NB - 1 ? 0 : nbuf + 1;
     // this wave's transfers of tile + step have landed (nothing was issued after them); the
     // barrier publishes everyone's pieces, LN(z) and the previous tile's output rows, and
@@ -782,7 +766,7 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
       store_rows(zs[fbuf], prev_off, prev_valid);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the rows are read before the slot is refilled
     }
-    dma(tile + 2 * step, fbuf);
+    dma(far, fbuf);
     // gate: D[channel][position], lane position p0, registers channels 32 cb + 8 j + 4 g + e
     {
       const bf16* xr = xh[k & 1];
@@ -801,11 +785,7 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
         *po = v;
       }
     }
-    if (tile + step < ntiles) {
-      int nvalid;
-      where(tile + step, nvalid);
-      ln_swz<kPT, 512>(zs[nbuf], xh[(k + 1) & 1], nvalid, lnp[0], lnp[1], eps);
-    }
+    if (nxt.b < batch) ln_swz<kPT, 512>(zs[nbuf], xh[(k + 1) & 1], valid_of(nxt), lnp[0], lnp[1], eps);
     __syncthreads();
     // output projection: D[channel][position] over the gated o of all 128 channels
     {
@@ -828,6 +808,9 @@ __global__ __launch_bounds__(512, 2) void triattn_output(
     prev_valid = valid;
     prev_off = off;
     last_buf = buf;
+    cur = nxt;
+    nxt = far;
+    far = tile_add(far, step, njb, n);
   }
   __syncthreads();  // every wave's part of the last tile's output rows
   store_rows(zs[last_buf], prev_off, prev_valid);

@@ -446,21 +446,14 @@ __global__ __launch_bounds__(512, 2) void trimul_output(
   float eps_out;
   const int njb = (n + kPT - 1) / kPT;
   const int64_t plane = (int64_t)np * np;
-  const int ntiles = batch * n * njb;
-  auto where = [&](int tile, int& b, int& i, int& j0, int& valid) {
-    const int jb = tile % njb;
-    i = (tile / njb) % n;
-    b = tile / (njb * n);
-    j0 = jb * kPT;
-    valid = min(kPT, n - j0);
-  };
+  auto valid_of = [&](const TileAt& t) { return min(kPT, n - t.blk * kPT); };
   // This wave's 2 one-KB pieces of the tile's z (positions past the end re-read the last
   // real one) and 2 of its P (8 channel rows each; j0 + 63 < np) into ring slot buf; a tile
-  // index past the end fetches tile 0 again, so every wave always has the same number of
-  // transfers in flight.
-  auto dma = [&](int tile, int buf) {
-    int b, i, j0, valid;
-    where(tile < ntiles ? tile : 0, b, i, j0, valid);
+  // past the end fetches tile 0 again, so every wave always has the same number of transfers in
+  // flight.
+  auto dma = [&](TileAt t, int buf) {
+    if (t.b >= batch) t = TileAt{0, 0, 0};
+    const int b = t.b, i = t.r, j0 = t.blk * kPT, valid = valid_of(t);
     const bf16* zb = z + (((int64_t)b * n + i) * n + j0) * 128;
     const uint32_t dz = lds_addr(&zs[buf][0]), dp = lds_addr(&ps[buf][0]);
 #pragma unroll
@@ -534,10 +527,14 @@ __global__ __launch_bounds__(512, 2) void trimul_output(
     for (int r = 0; r < 16; ++r) ag[r] = sigmoid_scaled(ag[r]);
     return ag;
   };
-  const int step = gridDim.x;
-  if ((int)blockIdx.x >= ntiles) return;
-  dma(blockIdx.x, 0);
-  dma(blockIdx.x + step, 1);
+  if ((int)blockIdx.x >= batch * n * njb) return;
+  // the walk advances by the grid stride with adds and carries (see TileAt)
+  const TileAt step = tile_at(gridDim.x, njb, n);
+  TileAt cur = tile_at(blockIdx.x, njb, n);
+  TileAt nxt = tile_add(cur, step, njb, n);
+  TileAt far = tile_add(nxt, step, njb, n);
+  dma(cur, 0);
+  dma(nxt, 1);
   // behind the transfers: the affines (published by the first barrier) and the weights
   const float* const lsrc[4] = {ln_w, ln_b, lno_w, lno_b};
   lnp[tid >> 7][tid & 127] = lsrc[tid >> 7][tid & 127];
@@ -554,22 +551,17 @@ __global__ __launch_bounds__(512, 2) void trimul_output(
     cn_w[e] = lnp[2][16 * wave + e];
     cn_b[e] = lnp[3][16 * wave + e];
   }
-  {
-    int b, i, j0, valid;
-    where(blockIdx.x, b, i, j0, valid);
-    ln_swz<kPT, 512>(zs[0], xh, valid, lnp[0], lnp[1], eps);
-    p_sum(0, 0);
-  }
+  ln_swz<kPT, 512>(zs[0], xh, valid_of(cur), lnp[0], lnp[1], eps);
+  p_sum(0, 0);
   __syncthreads();
   f32x16 sg = gate();
   p_centred(0, 0);
   int buf = 0, k = 0, prev_valid = kPT;
 #pragma unroll 1
-  for (int tile = blockIdx.x; tile < ntiles; tile += step, ++k, buf = buf == NB - 1 ? 0 : buf + 1) {
-    int b, i, j0, valid;
-    where(tile, b, i, j0, valid);
+  for (; cur.b < batch; ++k, buf = buf == NB - 1 ? 0 : buf + 1) {
+    const int b = cur.b, i = cur.r, j0 = cur.blk * kPT, valid = valid_of(cur);
     const int nbuf = buf == NB - 1 ? 0 : buf + 1, fbuf = nbuf == NB - 1 ? 0 : nbuf + 1;
-    const bool has_next = tile + step < ntiles;
+    const bool has_next = nxt.b < batch;
     // this wave's transfers of tile + step have landed (issued after them: the previous
     // tile's 2 stores, fewer for a partial tile); the barrier publishes everyone's pieces,
     // LN(z) and statistics, and retires the previous tile's accesses to ring slot fbuf
@@ -578,12 +570,10 @@ __global__ __launch_bounds__(512, 2) void trimul_output(
     else
       wait_vm_lds<2>();
     __syncthreads();
-    dma(tile + 2 * step, fbuf);
+    dma(far, fbuf);
     p_normalise(buf, k & 1);
     if (has_next) {
-      int nb, ni, nj0, nvalid;
-      where(tile + step, nb, ni, nj0, nvalid);
-      ln_swz<kPT, 512>(zs[nbuf], xh, nvalid, lnp[0], lnp[1], eps);
+      ln_swz<kPT, 512>(zs[nbuf], xh, valid_of(nxt), lnp[0], lnp[1], eps);
       p_sum(nbuf, (k + 1) & 1);
     }
     __syncthreads();
@@ -617,6 +607,9 @@ __global__ __launch_bounds__(512, 2) void trimul_output(
       p_centred(nbuf, (k + 1) & 1);
     }
     prev_valid = valid;
+    cur = nxt;
+    nxt = far;
+    far = tile_add(far, step, njb, n);
   }
   wait_vm_lds<0>();  // no LDS write may land after exit
 }
