@@ -1147,8 +1147,6 @@ int32_t ffk_attention_pair_bias(
   p.np = (int)np;
   p.heads = n_head;
   p.dh = dh;
-  launch_row_gemm(p, kEpiApb, kXLn, st);
-
   PairBiasArgs pb{};
   pb.z = static_cast<const bf16*>(z);
   pb.mask = key_mask;
@@ -1167,7 +1165,7 @@ int32_t ffk_attention_pair_bias(
   pb.extra_sb = extra_stride_b;
   pb.extra_sh = extra_stride_h;
   pb.extra_si = extra_stride_i;
-  launch_apb_pair_bias(pb, st);
+  launch_apb_project_bias(p, pb, st);
 
   ApbAttnArgs at;
   at.q = w.q;

@@ -234,6 +234,8 @@ struct PairBiasArgs {
   int64_t extra_sb, extra_sh, extra_si;
 };
 void launch_apb_pair_bias(const PairBiasArgs& a, hipStream_t stream);
+// Both of the single track's first kernels (kEpiApb from kXLn rows, and the bias).
+void launch_apb_project_bias(const RowGemmArgs& a, const PairBiasArgs& p, hipStream_t stream);
 
 struct ApbAttnArgs {
   const bf16 *q, *k, *vt, *gate;

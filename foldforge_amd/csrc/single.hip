@@ -8,7 +8,8 @@
 //   bias[h, i, j] = LN_pair(z[i, j]) . W_b[h]   (the pair norm has no offset)
 //   o = softmax_j(q_i . k_j / sqrt(dh) + bias[h, i, j]) over valid keys j, 0 for an empty row
 //   out = s + (g * o) W_out^T
-// is run as: row_gemm<kEpiApb, kXLn> (LayerNorm prologue; q, k, v^T, gate) -> apb_pair_bias
+// is run as: row_gemm<kEpiApb, kXLn> (LayerNorm prologue; q, k, v^T, gate) and apb_pair_bias (few
+// tokens: one launch, apb_project_bias)
 // -> apb_attention (gate applied) -> row_gemm<kEpiResid>.
 // The wide transition is row_gemm<kEpiSwiglu, kXLn> -> row_gemm<kEpiResid>.
 // The same file holds row_stream, the streaming LayerNorm-fed token-row GEMM that the
@@ -380,7 +381,7 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
 }
 
 template <int EPI, int XSRC, int NO>
-__global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
+__device__ __forceinline__ void row_gemm_body(const RowGemmArgs& a, const int bx, const int by) {
   constexpr int KS = kGemmWaves / NO;
   constexpr int kTurns = XSRC == kXLn ? 1 : 2;  // tiles per wave: weights, fp32 x rows
   constexpr int kAhead = 2;                     // groups in flight
@@ -392,9 +393,9 @@ __global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
   bf16* xs_lo = xs_hi + 32 * xstride;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, g = lane >> 5;
   const int osub = wave / KS, part = wave % KS;
-  const int ot = blockIdx.y * NO + osub;
+  const int ot = by * NO + osub;
   const bool active = ot * 32 < a.O;
-  const int64_t m0 = (int64_t)blockIdx.x * 32;
+  const int64_t m0 = (int64_t)bx * 32;
   const int G = a.K / 64, ng = active && part < G ? (G - part + KS - 1) / KS : 0;
 
   // this lane's loads: k 4 (lane % 8) .. of each 32, of rows 8 u + lane / 8, u = 0 .. 3 (packed
@@ -548,6 +549,11 @@ __global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
   const int64_t m = m0 + li;
   if (!active || m >= a.M) return;
   row_epilogue<EPI>(a, acc, m, ot, seg, cbase, g, nullptr, row_pre<EPI>(a, m));
+}
+
+template <int EPI, int XSRC, int NO>
+__global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
+  row_gemm_body<EPI, XSRC, NO>(a, blockIdx.x, blockIdx.y);
 }
 
 // ---------------------------------------------------------------------------- streaming row GEMM
@@ -1163,14 +1169,15 @@ __global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a
 // 32 contiguous bytes per row (lanes l and l ^ 32 together), the statistics come from those
 // registers (two passes, halves joined across lane l ^ 32), and the heads x keys block is
 // one 32 x 32 MFMA tile (A = W' rows, B = the z rows; channels 16 t .. 16 t + 15 feed step t).
-template <int C>
-__global__ __launch_bounds__(256) void apb_pair_bias(PairBiasArgs a) {
+// W waves per workgroup, workgroup bx of gx.
+template <int C, int W>
+__device__ __forceinline__ void pair_bias_body(const PairBiasArgs& a, const int bx, const int gx) {
   constexpr int kU = C / 16;  // 8-channel chunks per lane (each lane half holds C / 2)
-  __shared__ float wsum_s[4][32];
+  __shared__ float wsum_s[W][32];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 31, g = lane >> 5;
   const int n = a.n;
   const int njt = a.np / 32;
-  const int64_t stride = (int64_t)gridDim.x * 4;
+  const int64_t stride = (int64_t)gx * W;
 
   // Tiles are fetched one ahead (two register buffers used alternately); a fetch past the
   // last tile re-reads the last tile, so every load stays inside z.
@@ -1188,7 +1195,7 @@ __global__ __launch_bounds__(256) void apb_pair_bias(PairBiasArgs a) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) zf[u] = ld8(zr + 16 * u);
   };
-  int64_t t = (int64_t)blockIdx.x * 4 + wave;
+  int64_t t = (int64_t)bx * W + wave;
   bf16x8 z0[kU], z1[kU];
   fetch(z0, t);
 
@@ -1272,6 +1279,24 @@ __global__ __launch_bounds__(256) void apb_pair_bias(PairBiasArgs a) {
     process(z1, t);
     t += stride;
   }
+}
+
+template <int C>
+__global__ __launch_bounds__(256) void apb_pair_bias(PairBiasArgs a) {
+  pair_bias_body<C, 4>(a, blockIdx.x, gridDim.x);
+}
+
+// The single track's projections and its pair bias, which do not depend on each other, in one
+// launch: workgroups below gx * gy run the GEMM, the rest the bias. Up to 320 tokens the GEMM
+// has at most half the CUs' workgroups and either kernel alone is one chain of latencies; together
+// they take the longer one. 201 tokens: 13.3 + 10.1 -> 15.6 us.
+template <int NO>
+__global__ __launch_bounds__(512) void apb_project_bias(RowGemmArgs a, PairBiasArgs p, int gx, int gy) {
+  const int id = blockIdx.x, gemm = gx * gy;
+  if (id < gemm)
+    row_gemm_body<kEpiApb, kXLn, NO>(a, id % gx, id / gx);
+  else
+    pair_bias_body<128, kGemmWaves>(p, id - gemm, gridDim.x - gemm);
 }
 
 // The same bias at pair width 128 with the z rows staged through LDS: each wave owns two 8 KB
@@ -1709,6 +1734,26 @@ void launch_apb_pair_bias(const PairBiasArgs& a, hipStream_t stream) {
     apb_pair_bias<256><<<dim3((unsigned)blocks), 256, 0, stream>>>(a);
   else
     apb_pair_bias<128><<<dim3((unsigned)blocks), 256, 0, stream>>>(a);
+}
+
+void launch_apb_project_bias(const RowGemmArgs& a, const PairBiasArgs& p, hipStream_t stream) {
+  constexpr int NO = 4;
+  const int64_t gx = (a.M + 31) / 32, gy = (a.O / 32 + NO - 1) / NO;
+  const bool stream_case = a.K == 64 || a.K == 128 || a.K == 256;  // (row_stream's widths)
+  if (stream_case || p.c != 128 || gx * gy > cu_count() / 2) {
+    launch_row_gemm(a, kEpiApb, kXLn, stream);
+    launch_apb_pair_bias(p, stream);
+    return;
+  }
+  const size_t lds = row_gemm_lds(kXLn, a.K, NO);
+  auto kernel = apb_project_bias<NO>;
+  if (lds > 65536 - 8192)  // (with the bias's static LDS)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  // one workgroup per CU (registers): the bias takes the CUs that the GEMM leaves
+  const int64_t bias = std::max<int64_t>(1, std::min<int64_t>((p.tiles + kGemmWaves - 1) / kGemmWaves,
+                                                              cu_count() - gx * gy));
+  kernel<<<dim3((unsigned)(gx * gy + bias)), 64 * kGemmWaves, lds, stream>>>(a, p, (int)gx, (int)gy);
 }
 
 void launch_apb_attention(const ApbAttnArgs& a, int batch, hipStream_t stream) {
