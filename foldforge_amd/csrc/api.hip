@@ -9,8 +9,10 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <map>
 #include <mutex>
 #include <string>
+#include <utility>
 
 #include "foldforge_amd.h"
 #include "ffk_device.h"
@@ -80,6 +82,21 @@ int cu_count() {
     g_cu_count[dev] = cus;
   }
   return g_cu_count[dev];
+}
+
+int resident_blocks(const void* kernel, int threads, size_t dynamic_lds) {
+  static std::mutex mutex;
+  static std::map<std::pair<const void*, size_t>, int> known;  // (one architecture: gfx950)
+  std::lock_guard<std::mutex> lock(mutex);
+  int& n = known[{kernel, dynamic_lds}];
+  if (n == 0) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, dynamic_lds) != hipSuccess) {
+      (void)hipGetLastError();
+      n = 0;
+    }
+    n = n < 1 ? 1 : n;
+  }
+  return n;
 }
 
 namespace {

@@ -682,24 +682,20 @@ void launch_planes_to_rows(const bf16* planes, bf16* rows, int batch, int hid, i
 
 void launch_trimul_out_planes(const TrimulPlanesArgs& a, hipStream_t stream) {
   const int64_t tiles = (int64_t)a.batch * a.n * ((a.n + 31) / 32);
-  const int64_t blocks = std::min<int64_t>((tiles + kTmoWaves - 1) / kTmoWaves, (int64_t)cu_count() * 6);
-  const dim3 grid((unsigned)std::max<int64_t>(1, blocks));
-  if (a.hid == 128)
-    trimul_out_planes<128><<<grid, 64 * kTmoWaves, 0, stream>>>(a);
-  else
-    trimul_out_planes<64><<<grid, 64 * kTmoWaves, 0, stream>>>(a);
+  auto kernel = a.hid == 128 ? trimul_out_planes<128> : trimul_out_planes<64>;
+  const int64_t cap =
+      (int64_t)cu_count() * resident_blocks(reinterpret_cast<const void*>(kernel), 64 * kTmoWaves, 0);
+  const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((tiles + kTmoWaves - 1) / kTmoWaves, cap));
+  kernel<<<dim3((unsigned)blocks), 64 * kTmoWaves, 0, stream>>>(a);
 }
 
 void launch_triattn_out_rows(const TriattnRowsArgs& a, hipStream_t stream) {
   const int64_t tiles = ((int64_t)a.batch * a.n * a.n + 31) / 32;
-  const int64_t blocks = std::min<int64_t>((tiles + kTmoWaves - 1) / kTmoWaves, (int64_t)cu_count() * 6);
-  const dim3 grid((unsigned)std::max<int64_t>(1, blocks));
-  if (a.hd == 256)
-    triattn_out_rows<256><<<grid, 64 * kTmoWaves, 0, stream>>>(a);
-  else if (a.hd == 128)
-    triattn_out_rows<128><<<grid, 64 * kTmoWaves, 0, stream>>>(a);
-  else
-    triattn_out_rows<64><<<grid, 64 * kTmoWaves, 0, stream>>>(a);
+  auto kernel = a.hd == 256 ? triattn_out_rows<256> : a.hd == 128 ? triattn_out_rows<128> : triattn_out_rows<64>;
+  const int64_t cap =
+      (int64_t)cu_count() * resident_blocks(reinterpret_cast<const void*>(kernel), 64 * kTmoWaves, 0);
+  const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((tiles + kTmoWaves - 1) / kTmoWaves, cap));
+  kernel<<<dim3((unsigned)blocks), 64 * kTmoWaves, 0, stream>>>(a);
 }
 
 void launch_transition_rows(const TransitionRowsArgs& a, hipStream_t stream) {

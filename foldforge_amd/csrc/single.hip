@@ -672,8 +672,15 @@ __device__ __forceinline__ int64_t run_row(const RowGemmArgs& a, const TileRun& 
   return m0 + l;
 }
 
+// Waves per SIMD the registers are held to at K = 64: 128 registers for four workgroups per CU
+// where little or nothing spills (unbounded, q / k / v of the template stacks took 137 + 16 and
+// three workgroups: 88 -> 75 us), else 168 for three.
+__host__ __device__ constexpr int stream_simd_waves(int epi, int K) {
+  return K != 64 ? 2 : epi == kEpiTrimul || epi == kEpiOpm || epi == kEpiResid ? 3 : 4;
+}
+
 template <int EPI, int XSRC, int K>
-__global__ __launch_bounds__(64 * stream_waves(K)) void row_stream(RowGemmArgs a) {
+__global__ __launch_bounds__(64 * stream_waves(K), stream_simd_waves(EPI, K)) void row_stream(RowGemmArgs a) {
   constexpr int kStreamWaves = stream_waves(K);
   constexpr int KS = K / 16;  // MFMA steps
   constexpr int KH = K / 2;   // channels per lane
@@ -1613,7 +1620,8 @@ void launch_row_stream_t(const RowGemmArgs& a, hipStream_t stream) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   const int64_t tiles = (a.M + 31) / 32;
-  const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(4, (160 * 1024) / (int64_t)lds));
+  const int64_t per_cu =
+      resident_blocks(reinterpret_cast<const void*>(kernel), 64 * kStreamWaves, lds);
   const int64_t blocks = std::min<int64_t>((tiles + kStreamWaves - 1) / kStreamWaves,
                                            std::max<int64_t>(1, cu_count() * per_cu / parts));
   kernel<<<dim3((unsigned)std::max<int64_t>(1, blocks), (unsigned)parts), 64 * kStreamWaves, lds, stream>>>(a);
@@ -1724,16 +1732,10 @@ void launch_apb_pair_bias(const PairBiasArgs& a, hipStream_t stream) {
     apb_pair_bias_lds<<<dim3((unsigned)blocks), 256, 0, stream>>>(a);
     return;
   }
-  int64_t blocks = (a.tiles + 7) / 8;  // about two tiles per wave
-  const int64_t cap = (int64_t)cu_count() * 8;
-  if (blocks > cap) blocks = cap;
-  if (blocks < 1) blocks = 1;
-  if (a.c == 64)
-    apb_pair_bias<64><<<dim3((unsigned)blocks), 256, 0, stream>>>(a);
-  else if (a.c == 256)
-    apb_pair_bias<256><<<dim3((unsigned)blocks), 256, 0, stream>>>(a);
-  else
-    apb_pair_bias<128><<<dim3((unsigned)blocks), 256, 0, stream>>>(a);
+  auto kernel = a.c == 64 ? apb_pair_bias<64> : a.c == 256 ? apb_pair_bias<256> : apb_pair_bias<128>;
+  const int64_t cap = (int64_t)cu_count() * resident_blocks(reinterpret_cast<const void*>(kernel), 256, 0);
+  const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((a.tiles + 3) / 4, cap));
+  kernel<<<dim3((unsigned)blocks), 256, 0, stream>>>(a);
 }
 
 void launch_apb_project_bias(const RowGemmArgs& a, const PairBiasArgs& p, hipStream_t stream) {
