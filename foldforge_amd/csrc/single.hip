@@ -1587,7 +1587,7 @@ void launch_row_gemm_t(const RowGemmArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)((a.M + 31) / 32), (unsigned)((otiles + NO - 1) / NO));
   const size_t lds = row_gemm_lds(XSRC, a.K, NO);
   auto kernel = row_gemm<EPI, XSRC, NO>;
-  if (lds > 65536)  // beyond the default dynamic LDS size (K > 480 with the LayerNorm tile)
+  if (lds > 65536)  // beyond the default dynamic LDS size
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   kernel<<<grid, 64 * kGemmWaves, lds, stream>>>(a);
