@@ -1294,9 +1294,11 @@ __global__ __launch_bounds__(256) void apb_pair_bias(PairBiasArgs a) {
 }
 
 // The single track's projections and its pair bias, which do not depend on each other, in one
-// launch: workgroups below gx * gy run the GEMM, the rest the bias. Up to 320 tokens the GEMM
-// has at most half the CUs' workgroups and either kernel alone is one chain of latencies; together
-// they take the longer one. 201 tokens: 13.3 + 10.1 -> 15.6 us.
+// launch: workgroups below gx * gy run the GEMM, the rest the bias. Up to 384 tokens the GEMM
+// has at most 9/16 of the CUs in workgroups and either kernel alone is one chain of latencies; together
+// they take the longer one. 201 tokens: 13.3 + 10.1 -> 15.6 us; the call at 384 tokens 42.7 -> 40.4,
+// but at 448 46.8 -> 50.0 and at 512
+// (three quarters of the CUs) 50.7 -> 69.8.
 template <int NO>
 __global__ __launch_bounds__(512) void apb_project_bias(RowGemmArgs a, PairBiasArgs p, int gx, int gy) {
   const int id = blockIdx.x, gemm = gx * gy;
@@ -1742,7 +1744,7 @@ void launch_apb_project_bias(const RowGemmArgs& a, const PairBiasArgs& p, hipStr
   constexpr int NO = 4;
   const int64_t gx = (a.M + 31) / 32, gy = (a.O / 32 + NO - 1) / NO;
   const bool stream_case = a.K == 64 || a.K == 128 || a.K == 256;  // (row_stream's widths)
-  if (stream_case || p.c != 128 || gx * gy > cu_count() / 2) {
+  if (stream_case || p.c != 128 || gx * gy > cu_count() * 9 / 16) {
     launch_row_gemm(a, kEpiApb, kXLn, stream);
     launch_apb_pair_bias(p, stream);
     return;
