@@ -48,8 +48,10 @@ __device__ __forceinline__ int vkey_pos(int key) {
 // converted in registers), B = X rows. The workgroup's 8 waves cover NO output tiles of 32
 // with KS waves each (NO * KS = 8): the KS waves of a tile split k in groups of 64 (part p
 // takes groups p, p + KS, ...), keep two groups of global loads in flight, and add their
-// partial tiles through LDS; part 0 runs the epilogue. Weight rows and fp32 x rows are loaded 128
-// bytes of 8 rows at a time and turned into operands in a wave-private LDS tile: loaded in operand
+// partial tiles through LDS; part 0 runs the epilogue. For MFMA step t of a group, lane half g
+// supplies k = 32 g + 8 t .. + 7 of both operands (the order of the sums, and with it every output
+// bit, is part of the kernel). Weight rows and fp32 x rows are loaded 64 bytes of each half of 8 rows at
+// a time, two steps' worth, and turned into operands in a wave-private LDS tile: loaded in operand
 // order (a row per lane), an instruction touches 64 cache lines. q / k / v / gate of 201 tokens x
 // 384: 15.4 -> 13.3 us; squeeze (k 1536) and expand of 97 tokens 14.8 -> 10.0 and 17.2 -> 13.9;
 // transition of 2000 rows x 384 87 -> 73. Three groups in flight (96 VGPRs) ran one workgroup per
@@ -68,7 +70,7 @@ __device__ __forceinline__ int vkey_pos(int key) {
 // (acc[4 v + e]).
 
 constexpr int kGemmWaves = 8;
-constexpr int kTurnTile = 2 * 32 * 32;  // a wave's LDS tile: 32 rows x 32 k, hi then lo
+constexpr int kTurnTile = 2 * 32 * 32;  // a wave's LDS tile: 32 rows x (2 halves x 16 k), hi then lo
 __device__ __forceinline__ int turn_off(int r, int p) { return r * 32 + 8 * (p ^ ((r >> 2) & 3)); }
 
 size_t row_gemm_lds(int xsrc, int K, int no) {
@@ -398,10 +400,11 @@ __device__ __forceinline__ void row_gemm_body(const RowGemmArgs& a, const int bx
   const int64_t m0 = (int64_t)bx * 32;
   const int G = a.K / 64, ng = active && part < G ? (G - part + KS - 1) / KS : 0;
 
-  // this lane's loads: k 4 (lane % 8) .. of each 32, of rows 8 u + lane / 8, u = 0 .. 3 (packed
-  // tiles take rows 16-31 from a second matrix: a pointer per 16 rows)
+  // this lane's loads: column kc = 4 (lane % 8) of the tile, i.e. k 32 (kc / 16) + 16 h + kc % 16 of the
+  // group in its half h, of rows 8 u + lane / 8, u = 0 .. 3 (packed tiles take rows 16-31 from a
+  // second matrix: a pointer per 16 rows)
   int seg, cbase;
-  const int kq = 4 * (lane & 7), row8 = lane >> 3;
+  const int kc = 4 * (lane & 7), kq = 32 * (kc >> 4) + (kc & 15), row8 = lane >> 3;
   const float* wr[2];
   const float* xr4[4];
 #pragma unroll
@@ -420,11 +423,11 @@ __device__ __forceinline__ void row_gemm_body(const RowGemmArgs& a, const int bx
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       const int h = q >> 2, u = q & 3;
-      w[q] = *reinterpret_cast<const f32x4*>(wr[u >> 1] + (int64_t)(8 * (u & 1)) * a.K + k + 32 * h);
-      if (XSRC == kXF32) x[q] = *reinterpret_cast<const f32x4*>(xr4[u] + k + 32 * h);
+      w[q] = *reinterpret_cast<const f32x4*>(wr[u >> 1] + (int64_t)(8 * (u & 1)) * a.K + k + 16 * h);
+      if (XSRC == kXF32) x[q] = *reinterpret_cast<const f32x4*>(xr4[u] + k + 16 * h);
     }
   };
-  // rows 8 u + lane / 8 of one 32-k half into a tile, hi and (lo_on) lo
+  // rows 8 u + lane / 8 of steps 2 h and 2 h + 1 into a tile, hi and (lo_on) lo
   auto turn = [&](const f32x4* v, bf16* tile, bool lo_on) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -434,7 +437,7 @@ __device__ __forceinline__ void row_gemm_body(const RowGemmArgs& a, const int bx
         hi[e] = (bf16)v[u][e];
         lo[e] = (bf16)(v[u][e] - (float)hi[e]);
       }
-      const int at = turn_off(8 * u + row8, kq >> 3) + (kq & 4);
+      const int at = turn_off(8 * u + row8, kc >> 3) + (kc & 4);
       *reinterpret_cast<bf16x4*>(tile + at) = hi;
       if (lo_on) *reinterpret_cast<bf16x4*>(tile + 32 * 32 + at) = lo;
     }
@@ -506,10 +509,10 @@ __device__ __forceinline__ void row_gemm_body(const RowGemmArgs& a, const int bx
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const int at = turn_off(li, 2 * t + g);
+        const int at = turn_off(li, 2 * g + t);
         bf16x8 xhi, xlo;
         if (XSRC == kXLn) {
-          const int k = 64 * (part + KS * i) + 32 * h + 16 * t + 8 * g;
+          const int k = 64 * (part + KS * i) + 32 * g + 16 * h + 8 * t;
           xhi = ld8(xs_hi + li * xstride + k);
           xlo = ld8(xs_lo + li * xstride + k);
         } else {

@@ -79,3 +79,19 @@ def test_swiglu_ffn_matches_oracle(rows, d, hidden):
     assert inplace.data_ptr() == xc.data_ptr()
     assert torch.equal(inplace.cpu(), kernels.swiglu_ffn(x.cuda(), wa.cuda(), wb.cuda(), wo.cuda(),
                                                          residual=x.cuda()).cpu())
+
+
+@pytest.mark.parametrize("d_in", [64, 192, 384, 768])
+def test_row_gemm_adds_the_channels_in_steps_of_both_halves_of_a_group(d_in):
+    """Channels k and k + 32 of a 64-channel group enter the sum in one step, before those of k + 8:
+    2^25 - 2^25 + 1 is 1 in fp32 that way and 0 in the order of the channels. (The norm's weight is
+    zero and its offset one, so the rows are exactly one; the sums are exact in any split of the
+    groups.)"""
+    w = torch.zeros(64, d_in)
+    for o in range(64):
+        k = 64 * (o % (d_in // 64)) + o % 8
+        w[o, k], w[o, k + 32], w[o, k + 8] = 2.0 ** 25, -2.0 ** 25, 1.0
+    x = torch.randn(70, d_in, generator=torch.Generator().manual_seed(d_in)).bfloat16()
+    got = kernels.layer_norm_linear(x.cuda(), torch.zeros(d_in).cuda(), torch.ones(d_in).cuda(), w.cuda(),
+                                    out_dtype=torch.float32).cpu()
+    assert torch.equal(got, torch.ones(70, 64))
