@@ -478,18 +478,19 @@ __global__ __launch_bounds__(64 * kTmoWaves) void triattn_out_rows(TriattnRowsAr
 // wave needs 190 VGPRs, and three waves per SIMD spilled: 96 instead of 73 us for F = 2). Every
 // wave walks tiles of 32 rows on its own, the next tile's rows loaded while it works: lane
 // (li, g) holds channels 32 g .. 32 g + 31 of row li, normalised to bf16 hi + lo as in the row
-// GEMMs. Per 32 hidden channels the two expand products leave the lane with 16 of its row's
-// hidden values, which in accumulator order are the squeeze's operand as they stand (its
-// weight columns are stored in that order); the squeeze rows are permuted so that a lane's
-// accumulators hold its own channels of x. expand_a is held times -log2(e) and the squeeze times
-// -ln(2), so that the accumulator is the exponent of the sigmoid (as in transition.hip). Bound
+// GEMMs. The expand rows are permuted so that per product a lane half g is left with the 16 hidden
+// values (H / 2) g + 16 hb .. + 15 of its row, the squeeze's operand as they stand and in the order of
+// the row GEMM's steps; the squeeze rows are permuted so that a lane's accumulators hold its own
+// channels of x. The weights are the parameters rounded to bf16 and nothing else (a checkpoint in bf16
+// loses nothing on them: the update is 2.3e-3 from the exact one, and was 3.3e-3 with the weights held
+// times log2(e) for the sigmoid's exponent, a multiply per hidden value less and 2% faster). Bound
 // by instruction issue: per tile 160 / 80 MFMAs (5.1 / 2.6 k cycles) and about as long again of
 // SwiGLU, normalisation and rounding.
 template <int F>
 struct __attribute__((aligned(16))) TransitionRowsLds {
-  bf16 wa[64 * F * kTmoWs];        // expand_a rows, k = 64
-  bf16 wb[64 * F * kTmoWs];        // expand_b rows
-  bf16 ws[64 * (64 * F + 8)];      // squeeze rows (permuted), hidden in accumulator order
+  bf16 wa[64 * F * kTmoWs];        // expand_a rows (permuted), k = 64
+  bf16 wb[64 * F * kTmoWs];        // expand_b rows alike
+  bf16 ws[64 * (64 * F + 8)];      // squeeze rows (permuted)
   float lnw[64], lnb[64];
 };
 constexpr int transition_rows_waves(int F) { return F == 4 ? 8 : 4; }
@@ -503,24 +504,15 @@ __global__ __launch_bounds__(64 * transition_rows_waves(F), 2) void transition_r
   const int lane = tid & 63, g = lane >> 5, li = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int idx = tid; idx < H * 8; idx += 64 * W) {
+    // row 8 v + 4 g + e of block hb: hidden (H / 2) g + 16 hb + 4 v + e
     const int row = idx >> 3, ch = 8 * (idx & 7);
-    bf16x8 w;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) w[e] = (bf16)(-kLog2e * a.w_a[row * 64 + ch + e]);
-    *reinterpret_cast<bf16x8*>(lds.wa + row * kTmoWs + ch) = w;
-    *reinterpret_cast<bf16x8*>(lds.wb + row * kTmoWs + ch) = cvt8(a.w_b + row * 64 + ch);
+    const int hid = (H / 2) * ((row >> 2) & 1) + 16 * (row >> 5) + 4 * ((row >> 3) & 3) + (row & 3);
+    *reinterpret_cast<bf16x8*>(lds.wa + row * kTmoWs + ch) = cvt8(a.w_a + hid * 64 + ch);
+    *reinterpret_cast<bf16x8*>(lds.wb + row * kTmoWs + ch) = cvt8(a.w_b + hid * 64 + ch);
   }
   for (int idx = tid; idx < 64 * (H / 8); idx += 64 * W) {
-    // piece q of a 16-block: hidden 4 q .. 4 q + 3 and 8 + 4 q .. 8 + 4 q + 3
-    const int row = idx / (H / 8), p = idx % (H / 8);
-    const float* src = a.w_s + tmo_perm(row) * H + 16 * (p >> 1) + 4 * (p & 1);
-    bf16x8 w;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      w[e] = (bf16)((-1.f / kLog2e) * src[e]);
-      w[4 + e] = (bf16)((-1.f / kLog2e) * src[8 + e]);
-    }
-    *reinterpret_cast<bf16x8*>(lds.ws + row * HS + 8 * p) = w;
+    const int row = idx / (H / 8), ch = 8 * (idx % (H / 8));
+    *reinterpret_cast<bf16x8*>(lds.ws + row * HS + ch) = cvt8(a.w_s + tmo_perm(row) * H + ch);
   }
   if (tid < 64) {
     lds.lnw[tid] = a.ln_w[tid];
@@ -592,11 +584,11 @@ __global__ __launch_bounds__(64 * transition_rows_waves(F), 2) void transition_r
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float v = av[8 * k + e];
-          h[e] = (bf16)(v * sigmoid_scaled(v) * bv[8 * k + e]);
+          h[e] = (bf16)(v * sigmoid_scaled(-kLog2e * v) * bv[8 * k + e]);
         }
 #pragma unroll
         for (int t2 = 0; t2 < 2; ++t2)
-          oy[t2] = mfma32(ld8(lds.ws + (32 * t2 + li) * HS + 32 * hb + 16 * k + 8 * g), h, oy[t2]);
+          oy[t2] = mfma32(ld8(lds.ws + (32 * t2 + li) * HS + (H / 2) * g + 16 * hb + 8 * k), h, oy[t2]);
       }
     }
     const int64_t m = tile * 32 + li;

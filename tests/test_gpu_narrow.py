@@ -228,6 +228,23 @@ def test_transition_of_64_channels(rows, factor):
     assert torch.equal(inplace, got)
 
 
+@pytest.mark.parametrize("factor", [2, 4])
+def test_transition_of_64_channels_takes_bf16_weights_as_they_are(factor):
+    """Parameters that bf16 holds exactly, as a bf16 checkpoint has them, lose nothing in the kernel.
+    A bf16 rounding of random values is 1.66e-3 of them (rms). The update has two: its own and the
+    hidden rows' (2.35e-3 together); a rounding of expand_a and of squeeze would make it four
+    (3.3e-3)."""
+    m = randomise(factories.transition(64, factor), seed=factor)
+    for p in m.parameters():
+        p.data = p.data.bfloat16().float()
+    m = m.cuda()
+    m.set_backend("hip")
+    x = torch.randn(2000, 64, generator=torch.Generator().manual_seed(factor)).bfloat16()
+    want = ps.transition(x, m.state_dict(), dtype=torch.float64) - x.double()
+    got = hip_delta(m, x.cuda()).cpu().double()
+    assert ((got - want).norm() / want.norm()).item() <= 2.8e-3
+
+
 @pytest.mark.parametrize("c,h", [(64, 64), (128, 128), (256, 256)])
 @pytest.mark.parametrize("n,lengths", [(1, [1]), (31, [31, 7]), (97, [97, 20]), (129, [65, 129, 1])])
 def test_projections_at_row_and_mask_edges(c, h, n, lengths):
