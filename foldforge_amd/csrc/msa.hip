@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void pwa_softmax(PwaSoftmaxArgs a) {
     const int64_t idx = ((int64_t)blockIdx.x - (a.rows + 3) / 4) * 256 + threadIdx.x;
     if (a.frag && idx >= 0 && idx < 8 * a.hd) {
       const int l = (int)idx & 63, t = (int)(idx >> 6), kt = t % (a.hd / 16), ot = t / (a.hd / 16);
-      const float* src = a.w_out + (32 * ot + (l & 31)) * a.hd + 16 * kt + 8 * (l >> 5);
+      const float* src = a.w_out + (32 * ot + (l & 31)) * a.hd + 8 * kt + (a.hd / 2) * (l >> 5);
       bf16x8 v;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = (bf16)src[e];
@@ -74,10 +74,12 @@ __global__ __launch_bounds__(256) void pwa_softmax(PwaSoftmaxArgs a) {
 //   wave h: O_h[(s, d)][q] = sum_j v^T_h[(s, d)][j] w_h[q][j], one 32-row A tile (the head's S
 //   rows) x 4 query tiles, both operands straight from memory in fragment order (a 16-key step of
 //   a tile is one contiguous KB: [tile][k / 16][lane][8]), two steps fetched ahead;
-//   the averages go to LDS as bf16 token rows [(s, q)][8 DH] (64 KB for every DH, 16-byte pieces
-//   XOR-swizzled by row);
-//   then each wave projects its share of the (token tile, 32-channel output tile) pairs: gate
-//   times the LDS rows as the B operand, W_out fragments as A; residual and 16-byte stores.
+//   the averages are gated in fp32 (a lane's gate values travel behind the key loop) and go to LDS as
+//   bf16 token rows [(s, q)][8 DH] (64 KB for every DH, 16-byte pieces XOR-swizzled by row), the
+//   one rounding between the average and the projection;
+//   then each wave projects its share of the (token tile, 32-channel output tile) pairs: the LDS rows
+//   as the B operand, W_out fragments as A (step t: channels 4 DH g + 8 t ..); residual and
+//   16-byte stores.
 // Rows past the depth and queries past n hold whatever the operands held: they are not stored
 // and no product mixes rows or queries. This replaces a 128 x 128-tile GEMM per head, its gated
 // output in memory and a token-row GEMM: 512 x 256 tokens, 8 x 8: 50 -> 18 us. Bound by the
@@ -121,6 +123,16 @@ __global__ __launch_bounds__(512) void pwa_fused(PwaFusedArgs a) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) acc[t] = mfma32(x[u], y[u][t], acc[t]);
   };
+  // the gate of this lane's averages, pieces 8 (2 k + g) .. of the tile's rows (s, d) at query li of
+  // tile t (as acc_pieces leaves them): loaded first, so that they are there when the keys are done
+  bf16x8 gv[4][2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int r = 8 * (2 * k + g), s = s0 + r / DH, q = q0 + 32 * t + li;
+      gv[t][k] = ld8(a.gate + ((b * a.depth + min(s, a.depth - 1)) * n + min(q, n - 1)) * HD + wave * DH + r % DH);
+    }
   // np is a multiple of 64: steps in whole groups of 4
   fetch(0, fa[0], fb[0]);
 #pragma unroll 1
@@ -131,21 +143,6 @@ __global__ __launch_bounds__(512) void pwa_fused(PwaFusedArgs a) {
     multiply(fa[1], fb[1]);
   }
 
-  // this wave's token tiles and output tiles: pairs kPer wave .. + kPer - 1 of (tile, half); the
-  // gate of its token rows travels while the averages are published
-  constexpr int kRt = kPer >= 2 ? kPer / 2 : 1;  // token tiles of this wave
-  const int rt0 = kPer >= 2 ? wave * kRt : wave >> 1;
-  bf16x8 gv[kRt][KT];
-  int64_t tok[kRt];
-  bool real[kRt];
-#pragma unroll
-  for (int i = 0; i < kRt; ++i) {
-    const int row = 32 * (rt0 + i) + li, s = s0 + row / 128, q = q0 + row % 128;
-    real[i] = s < a.depth && q < n;
-    tok[i] = (b * a.depth + min(s, a.depth - 1)) * n + min(q, n - 1);
-#pragma unroll
-    for (int t = 0; t < KT; ++t) gv[i][t] = ld8(a.gate + tok[i] * HD + 16 * t + 8 * g);
-  }
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     float y[2][8];
@@ -155,22 +152,23 @@ __global__ __launch_bounds__(512) void pwa_fused(PwaFusedArgs a) {
       const int r = 8 * (2 * k + g), s = r / DH, d = r % DH;
       bf16x8 o;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = (bf16)y[k][e];
+      for (int e = 0; e < 8; ++e) o[e] = (bf16)(y[k][e] * (float)gv[t][k][e]);
       *reinterpret_cast<bf16x8*>(&os[piece(s * 128 + 32 * t + li, (wave * DH + d) / 8)]) = o;
     }
   }
   __syncthreads();
 
+  // this wave's token tiles and output tiles: pairs kPer wave .. + kPer - 1 of (tile, half)
+  constexpr int kRt = kPer >= 2 ? kPer / 2 : 1;  // token tiles of this wave
+  const int rt0 = kPer >= 2 ? wave * kRt : wave >> 1;
 #pragma unroll
   for (int i = 0; i < kRt; ++i) {
-    const int row = 32 * (rt0 + i) + li;
+    const int row = 32 * (rt0 + i) + li, sr = s0 + row / 128, qr = q0 + row % 128;
+    const bool real = sr < a.depth && qr < n;
+    const int64_t tok = (b * a.depth + min(sr, a.depth - 1)) * n + min(qr, n - 1);
     bf16x8 x[KT];
 #pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      const bf16x8 o = ld8(&os[piece(row, 2 * t + g)]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[t][e] = (bf16)((float)o[e] * (float)gv[i][t][e]);
-    }
+    for (int t = 0; t < KT; ++t) x[t] = ld8(&os[piece(row, KT * g + t)]);
 #pragma unroll
     for (int u = 0; u < (kPer >= 2 ? 2 : 1); ++u) {
       const int ot = kPer >= 2 ? u : wave & 1;
@@ -179,10 +177,10 @@ __global__ __launch_bounds__(512) void pwa_fused(PwaFusedArgs a) {
       for (int t = 0; t < KT; ++t) y = mfma32(ld8(a.wo + ((ot * KT + t) * 64 + lane) * 8), x[t], y);
       float p[2][8];
       acc_pieces(y, p);
-      if (!real[i]) continue;
+      if (!real) continue;
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        const int64_t at = tok[i] * 64 + 32 * ot + 8 * (2 * k + g);
+        const int64_t at = tok * 64 + 32 * ot + 8 * (2 * k + g);
         bf16x8 o;
         if (a.res) {
           const bf16x8 r = ld8(a.res + at);

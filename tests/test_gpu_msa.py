@@ -87,6 +87,38 @@ def test_msa_pair_weighted_averaging_of_eight_heads_at_tile_edges(dh, depth, n, 
     _check(hip_forward(mod, msa.cuda(), z.cuda(), mask.cuda()).cpu(), want + msa.double(), "msa_pwa residual")
 
 
+@pytest.mark.parametrize("dh", [8, 16, 32])
+def test_msa_pair_weighted_averaging_of_eight_heads_rounds_the_gated_average_once(dh):
+    """The one-kernel form against its own roundings in 64 bits: values, weights, gate, gate times
+    average, the projections' weights and the update in bf16, nothing else. What is left are values
+    that fp32 and the hardware's exp2 and reciprocal put on the other side of a rounding, 1 to 2e-4 of
+    the update. The update's own rounding (steps u of 5.5e-3 of a value on average) moves a value of
+    error e by u with probability e / u, so e shows as sqrt(e u): 0.7 to 1.05e-3, and a second
+    rounding of the average (e = 1.66e-3) as 3e-3. The bound lies between the two."""
+    depth, n = 9, 200
+    msa, z, mask = _inputs(depth, n, 64, [180], seed=dh)
+    mod = _pwa(64, 8, dh, seed=dh)
+    p = {k: v.double().cpu() for k, v in mod.state_dict().items()}
+
+    def r(x):
+        return x.bfloat16().double()
+
+    def norm(x, name):
+        return torch.nn.functional.layer_norm(x, x.shape[-1:], p[name + ".weight"], p.get(name + ".bias"), 1e-5)
+
+    x = norm(msa.double(), "ln_msa")[0]  # [S, n, 64]
+    logits = (norm(z.double(), "ln_pair") @ p["to_bias.weight"].T)[0].permute(2, 0, 1)  # [8, i, j]
+    w = r(logits.masked_fill(~mask[0], float("-inf")).softmax(dim=-1))
+    v = r(x @ r(p["to_value.weight"]).T).unflatten(-1, (8, dh))  # [S, j, 8, dh]
+    gate = r(torch.sigmoid(x @ r(p["to_gate.weight"]).T))
+    average = torch.stack([w[h] @ v[:, :, h] for h in range(8)], dim=2).flatten(2)  # [S, i, 8 dh]
+    want = r(r(gate * average) @ r(p["to_out.weight"]).T)
+    got = hip_delta(mod, msa.cuda(), z.cuda(), mask.cuda()).cpu()[0].double()
+    err = ((got - want).norm() / want.norm()).item()
+    print(f"msa_pwa 8x{dh} against its own roundings: {err:.2e}", flush=True)
+    assert err <= 1.8e-3
+
+
 @pytest.mark.parametrize("heads,dh", [(1, 256), (3, 64)])
 @pytest.mark.parametrize("n", [1, 31, 65])
 def test_msa_pair_weighted_averaging_wide_heads_and_broken_key_runs(heads, dh, n):
