@@ -1260,8 +1260,7 @@ int32_t ffk_msa_pair_weighted_averaging(
   p.eps = eps_msa;
   p.w0 = w_value;
   p.w1 = w_gate;
-  p.tmap = kMapPadKeys;  // tokens padded to np: the key-contiguous values leave in whole pieces
-  p.M = batch * depth * np;
+  p.M = rows;
   p.K = d_msa;
   p.O = (int)(2 * hd);
   p.vt = w.vt;

@@ -181,7 +181,8 @@ struct RowGemmArgs {
   int flash_rows;
   int apb_no_gate;  // kEpiApb: 1 = q, k, v only (O = 3 cs; the gate is computed downstream)
   // kEpiPwa: w0 = to_value, w1 = to_gate ([hd][K] each, O = 2 hd); tokens m = (b S + s) n + j;
-  // v^T [batch][heads][S][dh][np] (bf16, keys contiguous), gate = sigmoid(x W_g^T) [M][hd]
+  // v^T [batch][heads][S][dh][np] (bf16, keys contiguous; keys n .. np - 1 are written, as copies of
+  // key n - 1, by row_stream only), gate = sigmoid(x W_g^T) [M][hd]
   int depth;
   // row_stream with v_frag = 1 (dh 8, 16 or 32): v^T in pwa_fused's fragment order instead
   int v_frag;

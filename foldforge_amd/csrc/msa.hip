@@ -206,7 +206,7 @@ static_assert(64 * kPOS * 4 <= 4 * kPT * kPKP * 2, "epilogue staging exceeds the
 // key-contiguous. grid: ceil(S dh / 128) * ceil(n / 128) * batch * heads workgroups (renumbered
 // so that neighbours share an XCD's L2), block 256 = 2 x 2 waves of 64 x 64; operands staged
 // through LDS 32 keys at a time (register prefetch two stages ahead, double buffer, one barrier per stage).
-// v^T is not written at keys >= n: those operand entries are zeroed as they are staged.
+// v^T may be unwritten at keys >= n (RowGemmArgs): those operand entries are zeroed as they are staged.
 // Epilogue: lane (li, g) holds query q0' + li and rows r = r0' + 8 v + 4 g + e, i.e.
 // (s, c) = (r / dh, r % dh): four consecutive channels of one MSA row (dh % 4 == 0).
 __global__ __launch_bounds__(256) void pwa_average(PwaAverageArgs a) {

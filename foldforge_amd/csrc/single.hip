@@ -227,8 +227,8 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
     }
   } else if (EPI == kEpiPwa) {
     const int hd = a.O / 2;
-    const int64_t bs = m / a.np;  // b S + s
-    const int j = (int)(m - bs * a.np);
+    const int64_t bs = m / a.n;  // b S + s
+    const int j = (int)(m - bs * a.n);
     const int64_t b = bs / a.depth, srow = bs - b * a.depth;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -239,10 +239,10 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
         bf16* dst = a.vt + (((b * a.heads + hh) * a.depth + srow) * a.dh + d0) * a.np + j;
 #pragma unroll
         for (int e = 0; e < 4; ++e) dst[(int64_t)e * a.np] = (bf16)y[e];
-      } else if (j < a.n) {
+      } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = sigmoid_scaled(-kLog2e * y[e]);
-        store4(a.gate + (bs * a.n + j) * hd + c, y[0], y[1], y[2], y[3]);
+        store4(a.gate + m * hd + c, y[0], y[1], y[2], y[3]);
       }
     }
   } else if (EPI == kEpiOpm) {
@@ -1668,7 +1668,15 @@ void launch_row_gemm(const RowGemmArgs& a, int epi, int xsrc, hipStream_t stream
     if (epi == kEpiResid && a.ln_plain && launch_row_stream<kEpiResid, kXBf16>(a, stream)) return;
     if (epi == kEpiResid && launch_row_stream<kEpiResid, kXLn>(a, stream)) return;
     if (epi == kEpiOpm && launch_row_stream<kEpiOpm, kXLn>(a, stream)) return;
-    if (epi == kEpiPwa && launch_row_stream<kEpiPwa, kXLn>(a, stream)) return;
+    if (epi == kEpiPwa) {
+      // tokens padded to np: the key-contiguous values leave the streaming kernel in whole 16-byte
+      // pieces (512 rows x 256 tokens of 64 channels: 22 -> 19 us). row_gemm stores them 2 bytes a lane either way and takes
+      // the rows as they are (192 channels, 128 x 129 tokens, 8 x 24: 83 us padded, 77 not)
+      RowGemmArgs padded = a;
+      padded.tmap = kMapPadKeys;
+      padded.M = a.M / a.n * a.np;
+      if (launch_row_stream<kEpiPwa, kXLn>(padded, stream)) return;
+    }
   } else if (epi == kEpiResid && launch_row_stream<kEpiResid, kXF32>(a, stream)) {
     return;
   }

@@ -11,7 +11,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from foldforge_amd import factories
+from foldforge_amd import _native, factories
 from foldforge_amd.trunk import randomise
 from oracle import pairstack as ps
 from tests.hip_calls import hip_delta, hip_forward
@@ -129,6 +129,35 @@ def test_msa_pair_weighted_averaging_wide_heads_and_broken_key_runs(heads, dh, n
     want = ps.msa_pair_weighted_averaging(msa, z, mask, mod.state_dict(), n_head=heads,
                                           dtype=torch.float64) - msa.double()
     _check(got, want, f"msa_pwa {heads}x{dh} n={n}")
+
+
+@pytest.mark.parametrize("cm,heads,dh", [(192, 8, 24), (384, 16, 12), (64, 8, 24)])
+@pytest.mark.parametrize("n", [1, 33, 65])
+def test_msa_pair_weighted_averaging_does_not_read_what_it_does_not_write(cm, heads, dh, n):
+    """On a workspace of NaN the update is that of any other workspace. The values are its first piece,
+    ``[heads][S][dh][n padded to 64]``: MSA widths outside the streaming projection's (64, 128, 256)
+    leave the padding keys alone instead of projecting copies of the last token."""
+    depth = 3
+    msa, z, mask = (t.cuda() for t in _inputs(depth, n, cm, [n], seed=n + dh))
+    mod = _pwa(cm, heads, dh, seed=dh)
+    want = hip_delta(mod, msa, z, mask)
+    lib, out = _native.lib(), torch.empty_like(msa)
+    size = lib.ffk_msa_pair_weighted_averaging_workspace(1, depth, n, cm, 128, heads, dh)
+    ws = torch.full((size,), 255, dtype=torch.uint8, device="cuda")
+    p = dict(mod.named_parameters())
+    names = ("ln_msa.weight", "ln_msa.bias", "ln_pair.weight", "to_bias.weight", "to_value.weight",
+             "to_gate.weight", "to_out.weight")
+    status = lib.ffk_msa_pair_weighted_averaging(
+        msa.data_ptr(), z.data_ptr(), mask.data_ptr(), *(p[k].data_ptr() for k in names), out.data_ptr(),
+        ws.data_ptr(), size, 1, depth, n, cm, 128, heads, dh, 0, mod.ln_msa.eps, mod.ln_pair.eps,
+        torch.cuda.current_stream().cuda_stream)
+    assert status == 0, lib.ffk_last_error().decode()
+    assert torch.equal(out, want)
+    np = (n + 63) // 64 * 64
+    vt = ws[:heads * depth * dh * np * 2].view(torch.bfloat16).view(heads, depth, dh, np)
+    assert torch.isfinite(vt[..., :n].float()).all()
+    if cm not in (64, 128, 256):
+        assert torch.isnan(vt[..., n:].float()).all()
 
 
 def test_msa_pair_weighted_averaging_masking_is_exact_and_empty_rows_are_zero():
