@@ -9,8 +9,7 @@
 //   o = softmax_j(q_i . k_j / sqrt(dh) + bias[h, i, j]) over valid keys j, 0 for an empty row
 //   out = s + (g * o) W_out^T
 // is run as: row_gemm<kEpiApb, kXLn> (LayerNorm prologue; q, k, v^T, gate) and apb_pair_bias (few
-// tokens: one launch, apb_project_bias)
-// -> apb_attention (gate applied) -> row_gemm<kEpiResid>.
+// tokens: one launch, apb_project_bias) -> apb_attention (gate applied) -> row_gemm<kEpiResid>.
 // The wide transition is row_gemm<kEpiSwiglu, kXLn> -> row_gemm<kEpiResid>.
 // The same file holds row_stream, the streaming LayerNorm-fed token-row GEMM that the
 // generic pair widths (template stacks, Chai-1's pair 256) run their projections on.
@@ -1297,11 +1296,9 @@ __global__ __launch_bounds__(256) void apb_pair_bias(PairBiasArgs a) {
 }
 
 // The single track's projections and its pair bias, which do not depend on each other, in one
-// launch: workgroups below gx * gy run the GEMM, the rest the bias. Up to 384 tokens the GEMM
-// has at most 9/16 of the CUs in workgroups and either kernel alone is one chain of latencies; together
-// they take the longer one. 201 tokens: 13.3 + 10.1 -> 15.6 us; the call at 384 tokens 42.7 -> 40.4,
-// but at 448 46.8 -> 50.0 and at 512
-// (three quarters of the CUs) 50.7 -> 69.8.
+// launch: workgroups below gx * gy run the GEMM, the rest the bias. Where the GEMM leaves CUs free,
+// either kernel alone is one chain of latencies; together they take the longer one. 201 tokens of 384
+// channels: 13.3 + 10.1 -> 15.6 us. launch_apb_project_bias has the rule.
 template <int NO>
 __global__ __launch_bounds__(512) void apb_project_bias(RowGemmArgs a, PairBiasArgs p, int gx, int gy) {
   const int id = blockIdx.x, gemm = gx * gy;
@@ -1751,11 +1748,20 @@ void launch_apb_pair_bias(const PairBiasArgs& a, hipStream_t stream) {
   kernel<<<dim3((unsigned)blocks), 256, 0, stream>>>(a);
 }
 
+// One launch while each CU that the GEMM leaves free gets at most 42 bias tiles of 32 keys, a few per wave
+// (more where more than 96 are free: the bias is then the longer kernel of the two either way): past that
+// its register-fed form (32-byte pieces of 32 rows a load) falls behind the LDS-DMA kernel on every CU.
+// The whole call, two launches -> one (free CUs, tiles on each): 384 channels, 201 tokens 36.3 -> 28.9 us
+// (172, 8), 320 42.1 -> 34.4 (136, 24), 384 43.7 -> 42.1 (112, 41), 448 48.6 -> 51.5 (88, 71), 512 52.3 -> 71.1 (64,
+// 128); 5 x 100 tokens 38.4 -> 34.3 (64, 31); 192 channels, 512 tokens 46.5 -> 45.4 (160, 51), 640 55.5 -> 59.3 (136, 94),
+// 768 66.9 -> 83.2 (112, 165); 512 channels, 320 44.8 -> 39.9 (96, 33), 384 47.0 -> 51.7 (64, 72); 768 channels,
+// 256 50.3 -> 41.5 (64, 32), 288 53.5 -> 56.9 (40, 65). Beside a trunk's pair track: 4 blocks of 201 / 256
+// tokens 1109 -> 1094 and 1221 -> 1202 us, 320 to 384 within 0.6%.
 void launch_apb_project_bias(const RowGemmArgs& a, const PairBiasArgs& p, hipStream_t stream) {
   constexpr int NO = 4;
-  const int64_t gx = (a.M + 31) / 32, gy = (a.O / 32 + NO - 1) / NO;
+  const int64_t gx = (a.M + 31) / 32, gy = (a.O / 32 + NO - 1) / NO, rest = cu_count() - gx * gy;
   const bool stream_case = a.K == 64 || a.K == 128 || a.K == 256;  // (row_stream's widths)
-  if (stream_case || p.c != 128 || gx * gy > cu_count() * 9 / 16) {
+  if (stream_case || p.c != 128 || rest <= 0 || p.tiles > rest * std::max<int64_t>(42, rest / 2 - 6)) {
     launch_row_gemm(a, kEpiApb, kXLn, stream);
     launch_apb_pair_bias(p, stream);
     return;
@@ -1766,8 +1772,7 @@ void launch_apb_project_bias(const RowGemmArgs& a, const PairBiasArgs& p, hipStr
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   // one workgroup per CU (registers): the bias takes the CUs that the GEMM leaves
-  const int64_t bias = std::max<int64_t>(1, std::min<int64_t>((p.tiles + kGemmWaves - 1) / kGemmWaves,
-                                                              cu_count() - gx * gy));
+  const int64_t bias = std::min<int64_t>((p.tiles + kGemmWaves - 1) / kGemmWaves, rest);
   kernel<<<dim3((unsigned)(gx * gy + bias)), 64 * kGemmWaves, lds, stream>>>(a, p, (int)gx, (int)gy);
 }
 

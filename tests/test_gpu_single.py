@@ -75,6 +75,25 @@ def test_attention_pair_bias_matches_oracle(cs, heads, n, lengths):
     _check(full, want + s.double(), "attention_pair_bias residual")
 
 
+# one launch for projections and bias, or two: on 256 CUs the first of each pair of sizes takes the one;
+# the second takes two because of its pair rows (192, 384 and 768 channels) or of its GEMM rows (320)
+@pytest.mark.parametrize("cs,heads,sizes", [(192, 8, [(4, 97), (3, 256)]), (384, 16, [(5, 64), (5, 130)]),
+                                            (768, 24, [(5, 64), (3, 100)]), (320, 10, [(2, 65), (5, 161)])])
+def test_attention_pair_bias_on_both_sides_of_the_one_launch_rule(cs, heads, sizes):
+    """Every batch element is the call on it alone, bit for bit, and that call (one launch) matches the
+    oracle."""
+    m = _apb(cs, heads, gate_bias=0.5, seed=cs)
+    for batch, n in sizes:
+        s, z, mask = _inputs(n, cs, [n - 3 * b for b in range(batch)], seed=n + cs)
+        got = hip_delta(m, s.cuda(), z.cuda(), mask.cuda()).cpu()
+        for b in (0, batch - 1):
+            alone = hip_delta(m, s[b:b + 1].cuda(), z[b:b + 1].cuda(), mask[b:b + 1].cuda()).cpu()
+            assert torch.equal(got[b], alone[0])
+        want = ps.attention_pair_bias(s[-1:], z[-1:], mask[-1:], m.state_dict(), n_head=heads, gate_bias=0.5,
+                                      dtype=torch.float64) - s[-1:].double()
+        _check(alone, want, f"attention_pair_bias cs={cs} n={n} batch {batch}")
+
+
 @pytest.mark.parametrize("form", ["nn_fp32", "bhnn_bf16"])
 def test_attention_pair_bias_extra_bias_matches_oracle(form):
     """The block's extra pair bias on hip: an fp32 [N, N] map (broadcast by zero strides, as
