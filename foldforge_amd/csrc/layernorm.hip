@@ -45,7 +45,7 @@ __device__ __forceinline__ float lanes_sum(float v) {
   return v;
 }
 
-// Rows of exactly L * P pieces; x, y, w, b 16-byte aligned. grid min(ceil(rows / (R 256 / L)),
+// Rows of exactly L * P pieces; x and y 16-byte aligned. grid min(ceil(rows / (R 256 / L)),
 // 32 per CU); block 256.
 template <typename T, int L, int P>
 __global__ __launch_bounds__(256) void layer_norm_vec(const T* __restrict__ x, const float* __restrict__ w,
@@ -170,10 +170,11 @@ template <typename T>
 void launch_typed(const T* x, const float* w, const float* b, T* y, int64_t rows, int cols, float eps,
                   hipStream_t stream) {
   // The vector kernel takes the widths whose pieces split evenly over 8 to 64 lanes with one or
-  // three pieces a lane (the stacks' 64 to 768 channels) and 16-byte aligned tensors; other
-  // widths, and views at odd offsets, keep the row kernel.
+  // three pieces a lane (the stacks' 64 to 768 channels) and 16-byte aligned tensors (the affine is
+  // read a value at a time: any alignment); other widths, and views at odd offsets, keep the row
+  // kernel.
   const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (cols % LnPiece<T>::kN == 0 && aligned(x) && aligned(y) && aligned(w) && aligned(b)) {
+  if (cols % LnPiece<T>::kN == 0 && aligned(x) && aligned(y)) {
     switch (cols / LnPiece<T>::kN) {
       case 8: return launch_vec<T, 8, 1>(x, w, b, y, rows, eps, stream);
       case 16: return launch_vec<T, 16, 1>(x, w, b, y, rows, eps, stream);

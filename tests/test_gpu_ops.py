@@ -106,6 +106,19 @@ def test_layer_norm_widths(cols, dtype):
         assert ((got.double() - want).abs() / (1 + want.abs())).max().item() <= ulp + 2e-6
 
 
+@pytest.mark.parametrize("cols", [64, 128, 384, 768])
+def test_layer_norm_takes_an_affine_of_any_fp32_alignment(cols):
+    """A weight and an offset that are slices of a flat buffer (4-byte aligned only) give the same bits
+    as aligned ones, i.e. run the same kernel (in fp32 the row kernel's sums differ)."""
+    g = torch.Generator().manual_seed(cols)
+    flat = torch.randn(2 * cols + 1, generator=g).cuda()
+    w, b = flat[1:cols + 1], flat[cols + 1:]
+    assert w.data_ptr() % 16 and b.data_ptr() % 16
+    for dtype in (torch.float32, torch.bfloat16):
+        x = torch.randn(2000, cols, generator=g).to(dtype).cuda()
+        assert torch.equal(kernels.layer_norm(x, w, b, 1e-5), kernels.layer_norm(x, w.clone(), b.clone(), 1e-5))
+
+
 @pytest.mark.parametrize("outgoing", [True, False])
 @pytest.mark.parametrize("n,lengths", [(64, None), (100, [77]), (130, [130, 41]), (256, [256, 203])])
 def test_trimul_matches_oracle(outgoing, n, lengths):
