@@ -245,6 +245,37 @@ def test_transition_of_64_channels_takes_bf16_weights_as_they_are(factor):
     assert ((got - want).norm() / want.norm()).item() <= 2.8e-3
 
 
+@pytest.mark.parametrize("d,factor", [(64, 3), (128, 2), (256, 2)])
+def test_transition_of_few_rows_is_that_of_many(d, factor):
+    """Few rows take more parts of the outputs (1 to 9409 rows: from one output tile a workgroup to the
+    parts that LDS asks for), which changes nothing in a row: the same bits as in a large call, and the
+    oracle's values."""
+    m = randomise(factories.transition(d, factor), seed=d).cuda()
+    m.set_backend("hip")
+    x = torch.randn(20000, d, generator=torch.Generator().manual_seed(d)).bfloat16()
+    many = m(x.cuda()).cpu()
+    for rows in (1, 33, 500, 2500, 9409):
+        assert torch.equal(m(x[:rows].cuda()).cpu(), many[:rows])
+    want = ps.transition(x[:500], m.state_dict(), dtype=torch.float64) - x[:500].double()
+    _check(hip_delta(m, x[:500].cuda()).cpu(), want, None, f"transition {d} x {factor}")
+
+
+@pytest.mark.parametrize("c,h", [(64, 128), (128, 64), (256, 256)])
+def test_generic_ops_of_few_tokens_work_in_place(c, h):
+    """``out`` is the pair itself: what still reads a row is done with it before it is written."""
+    z, mask = _pair(24, c, [24, 17], seed=c)
+    m = randomise(factories.triangle_multiplication(c, outgoing=False, d_hidden=h), seed=c).cuda()
+    names = ("ln_pair_weight", "ln_pair_bias", "to_left", "to_right", "to_left_gate", "to_right_gate",
+             "ln_out_weight", "ln_out_bias", "to_out", "to_gate")
+    p = {k: v for k, v in zip(names, (m.ln_pair.weight, m.ln_pair.bias, m.to_left.weight, m.to_right.weight,
+                                      m.to_left_gate.weight, m.to_right_gate.weight, m.ln_out.weight,
+                                      m.ln_out.bias, m.to_out.weight, m.to_gate.weight))}
+    inplace, mask = z.cuda(), mask.cuda()
+    want = kernels.triangle_multiplicative_update(z.cuda(), mask, outgoing=False, **p)
+    kernels.triangle_multiplicative_update(inplace, mask, outgoing=False, out=inplace, **p)
+    assert torch.equal(inplace, want)
+
+
 @pytest.mark.parametrize("c,h", [(64, 64), (128, 128), (256, 256)])
 @pytest.mark.parametrize("n,lengths", [(1, [1]), (31, [31, 7]), (97, [97, 20]), (129, [65, 129, 1])])
 def test_projections_at_row_and_mask_edges(c, h, n, lengths):
