@@ -758,9 +758,12 @@ __global__ __launch_bounds__(64 * stream_waves(K), stream_simd_waves(EPI, K)) vo
   uint32_t L = 1, R = 1;
   TileRun cur{}, step{};
   if constexpr (kRuns) {
-    run_radix<EPI>(a, L, R);
-    cur = run_at(t * 32, L, R);
-    step = run_at(stride * 32, L, R);
+    // (rows read as they are have no digits: the two divisions took 0.2 to 0.8 us of a small call)
+    if ((EPI != kEpiApb && EPI != kEpiResid) || a.tmap == kMapPairT) {
+      run_radix<EPI>(a, L, R);
+      cur = run_at(t * 32, L, R);
+      step = run_at(stride * 32, L, R);
+    }
   }
   const int apb_cs = EPI == kEpiApbFlash ? apb_width(a) : 1;
   const int dsh = EPI == kEpiApbFlash ? __builtin_ctz(a.dh) : 0;  // head widths 16, 32 or 64
