@@ -72,10 +72,9 @@ constexpr int kGemmWaves = 8;
 constexpr int kTurnTile = 2 * 32 * 32;  // a wave's LDS tile: 32 rows x (2 halves x 16 k), hi then lo
 __device__ __forceinline__ int turn_off(int r, int p) { return r * 32 + 8 * (p ^ ((r >> 2) & 3)); }
 
-size_t row_gemm_lds(int xsrc, int K, int no) {
+size_t row_gemm_lds(int xsrc, int K) {
   const size_t tiles = (size_t)kGemmWaves * (xsrc == kXLn ? 1 : 2) * kTurnTile * sizeof(bf16);
-  const size_t red = (size_t)(kGemmWaves - no) * 64 * 16 * sizeof(float);
-  return tiles + red + (xsrc == kXLn ? (size_t)2 * 32 * (K + 8) * sizeof(bf16) : 0);
+  return tiles + (xsrc == kXLn ? (size_t)2 * 32 * (K + 8) * sizeof(bf16) : 0);
 }
 
 // The input row of logical row m under the row map a.tmap (see kMap* in ffk_kernels.h).
@@ -381,15 +380,15 @@ __device__ __forceinline__ void row_epilogue(const RowGemmArgs& a, const f32x16&
   }
 }
 
-template <int EPI, int XSRC, int NO>
+template <int EPI, int XSRC, int NO, int kAhead>
 __device__ __forceinline__ void row_gemm_body(const RowGemmArgs& a, const int bx, const int by) {
   constexpr int KS = kGemmWaves / NO;
   constexpr int kTurns = XSRC == kXLn ? 1 : 2;  // tiles per wave: weights, fp32 x rows
-  constexpr int kAhead = 2;                     // groups in flight
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  bf16* turns = reinterpret_cast<bf16*>(smem);  // [kGemmWaves][kTurns][kTurnTile]
-  float* red = reinterpret_cast<float*>(turns + kGemmWaves * kTurns * kTurnTile);  // [NO][KS - 1][64][16]
-  bf16* xs_hi = reinterpret_cast<bf16*>(red + (kGemmWaves - NO) * 64 * 16);
+  // [kGemmWaves][kTurns][kTurnTile]; behind the products a wave's first tile takes its partial sums
+  bf16* turns = reinterpret_cast<bf16*>(smem);
+  static_assert(64 * 16 * sizeof(float) <= kTurnTile * sizeof(bf16), "partial sums exceed the turn tile");
+  bf16* xs_hi = turns + kGemmWaves * kTurns * kTurnTile;
   const int xstride = a.K + 8;  // [32][K + 8]: rows 16 bytes apart modulo 256, conflict-free
   bf16* xs_lo = xs_hi + 32 * xstride;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, g = lane >> 5;
@@ -537,15 +536,18 @@ __device__ __forceinline__ void row_gemm_body(const RowGemmArgs& a, const int bx
   }
   if (KS > 1) {
     if (part > 0) {
+      float* mine = reinterpret_cast<float*>(wt) + lane * 16;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) red[((osub * (KS - 1) + part - 1) * 64 + lane) * 16 + r] = acc[r];
+      for (int r = 0; r < 16; ++r) mine[r] = acc[r];
     }
     __syncthreads();
     if (part != 0) return;
 #pragma unroll
-    for (int w = 0; w < KS - 1; ++w)
+    for (int w = 1; w < KS; ++w) {
+      const float* theirs = reinterpret_cast<const float*>(turns + (wave + w) * kTurns * kTurnTile) + lane * 16;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] += red[((osub * (KS - 1) + w) * 64 + lane) * 16 + r];
+      for (int r = 0; r < 16; ++r) acc[r] += theirs[r];
+    }
   }
 
   const int64_t m = m0 + li;
@@ -553,9 +555,12 @@ __device__ __forceinline__ void row_gemm_body(const RowGemmArgs& a, const int bx
   row_epilogue<EPI>(a, acc, m, ot, seg, cbase, g, nullptr, row_pre<EPI>(a, m));
 }
 
-template <int EPI, int XSRC, int NO>
-__global__ __launch_bounds__(512) void row_gemm(RowGemmArgs a) {
-  row_gemm_body<EPI, XSRC, NO>(a, blockIdx.x, blockIdx.y);
+// kAhead: groups in flight, 2, or 1 where no wave has a second one (up to KS groups): 128 VGPRs then, and
+// two workgroups per CU (147 to 158 with two). Many rows need that: LayerNorm + linear of 100000 x 64 -> 128
+// 50.3 -> 33.9 us, 256 -> 64 70.6 -> 45.3; the grouped outer product of 192 channels, 512 x 200 tokens, 286 -> 221.
+template <int EPI, int XSRC, int NO, int kAhead>
+__global__ __launch_bounds__(64 * kGemmWaves, kAhead == 1 ? 4 : 2) void row_gemm(RowGemmArgs a) {
+  row_gemm_body<EPI, XSRC, NO, kAhead>(a, blockIdx.x, blockIdx.y);
 }
 
 // ---------------------------------------------------------------------------- streaming row GEMM
@@ -1307,7 +1312,7 @@ template <int NO>
 __global__ __launch_bounds__(512) void apb_project_bias(RowGemmArgs a, PairBiasArgs p, int gx, int gy) {
   const int id = blockIdx.x, gemm = gx * gy;
   if (id < gemm)
-    row_gemm_body<kEpiApb, kXLn, NO>(a, id % gx, id / gx);
+    row_gemm_body<kEpiApb, kXLn, NO, 2>(a, id % gx, id / gx);
   else
     pair_bias_body<128, kGemmWaves>(p, id - gemm, gridDim.x - gemm);
 }
@@ -1591,8 +1596,13 @@ template <int EPI, int XSRC, int NO>
 void launch_row_gemm_t(const RowGemmArgs& a, hipStream_t stream) {
   const int otiles = a.O / 32;
   const dim3 grid((unsigned)((a.M + 31) / 32), (unsigned)((otiles + NO - 1) / NO));
-  const size_t lds = row_gemm_lds(XSRC, a.K, NO);
-  auto kernel = row_gemm<EPI, XSRC, NO>;
+  const size_t lds = row_gemm_lds(XSRC, a.K);
+  // one group a wave, and workgroups to fill the second place on a CU (with fewer, the form held to 128
+  // VGPRs is up to 3% slower: the output projection of 201 tokens x 384). Eight output tiles a workgroup
+  // leave a wave all groups: one only at the 64 channels that just kEpiLinear brings here.
+  auto kernel = row_gemm<EPI, XSRC, NO, 2>;
+  if constexpr (NO < kGemmWaves || EPI == kEpiLinear)
+    if (a.K / 64 <= kGemmWaves / NO && (int64_t)grid.x * grid.y > cu_count()) kernel = row_gemm<EPI, XSRC, NO, 1>;
   if (lds > 65536)  // beyond the default dynamic LDS size
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1780,7 +1790,7 @@ void launch_apb_project_bias(const RowGemmArgs& a, const PairBiasArgs& p, hipStr
     launch_apb_pair_bias(p, stream);
     return;
   }
-  const size_t lds = row_gemm_lds(kXLn, a.K, NO);
+  const size_t lds = row_gemm_lds(kXLn, a.K);
   auto kernel = apb_project_bias<NO>;
   if (lds > 65536 - 8192)  // (with the bias's static LDS)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),

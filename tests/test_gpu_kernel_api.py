@@ -95,3 +95,28 @@ def test_row_gemm_adds_the_channels_in_steps_of_both_halves_of_a_group(d_in):
     got = kernels.layer_norm_linear(x.cuda(), torch.zeros(d_in).cuda(), torch.ones(d_in).cuda(), w.cuda(),
                                     out_dtype=torch.float32).cpu()
     assert torch.equal(got, torch.ones(70, 64))
+
+
+@pytest.mark.parametrize("d_in,d_out", [(64, 256), (64, 128), (128, 128), (256, 64), (192, 32)])
+def test_layer_norm_linear_of_many_rows_is_that_of_few(d_in, d_out):
+    """Widths whose waves have one group of channels each, on both sides of one workgroup per CU (the
+    form with one group in flight beyond): the same bits, and the oracle's values."""
+    g = torch.Generator().manual_seed(d_in + d_out)
+    x = torch.randn(9409, d_in, generator=g).bfloat16()
+    w, lw = 0.1 * torch.randn(d_out, d_in, generator=g), 1 + 0.1 * torch.randn(d_in, generator=g)
+    many = kernels.layer_norm_linear(x.cuda(), lw.cuda(), None, w.cuda(), out_dtype=torch.float32).cpu()
+    few = kernels.layer_norm_linear(x[-300:].contiguous().cuda(), lw.cuda(), None, w.cuda(),
+                                    out_dtype=torch.float32).cpu()
+    assert torch.equal(many[-300:], few)
+    want = ps.layer_norm_linear(x.double(), lw.double(), None, w.double(), dtype=torch.float64)
+    _check(many, want, f"layer_norm_linear 9409x{d_in}->{d_out}")
+
+
+@pytest.mark.parametrize("d,hidden", [(64, 256), (128, 512)])
+def test_swiglu_ffn_of_many_rows_is_that_of_few(d, hidden):
+    g = torch.Generator().manual_seed(hidden)
+    x = torch.randn(20000, d, generator=g).bfloat16().cuda()
+    wa, wb = (0.08 * torch.randn(hidden, d, generator=g).cuda() for _ in range(2))
+    wo = 0.08 * torch.randn(d, hidden, generator=g).cuda()
+    many = kernels.swiglu_ffn(x, wa, wb, wo)
+    assert torch.equal(many[:300], kernels.swiglu_ffn(x[:300].contiguous(), wa, wb, wo))
