@@ -434,8 +434,8 @@ __global__ __launch_bounds__(256, 2) void flash_attn_bias(FlashArgs a) {
   // branch the common case never takes). From then on the extra offset enters the row's S
   // accumulation through one more MFMA with constant operands (A: 1 at k = 0 of every key
   // row; B: minus the offset at k = 0 of the lane's query). Every offset depends on the row's
-  // and query's own logits, so no row of the workgroup (a padded one included) changes another
-  // row's rounding.
+  // and query's own logits, and the tile is recomputed for a query that is stored only: padded
+  // queries and rows, whose operands may never have been written, change nothing of the others.
   float msh = 0.f;
   if (active) {
     const float* bt = &lds.bias[wave][0][4 * lane];
@@ -506,7 +506,9 @@ __global__ __launch_bounds__(256, 2) void flash_attn_bias(FlashArgs a) {
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             const int rr = rp + u;
-            if (__builtin_amdgcn_ballot_w64(!(ts[u] < kSumRescale)) == 0) continue;
+            // (only a stored query's sum counts; asked here, where the common case never comes)
+            if (r0 + rr >= a.rows_valid || __builtin_amdgcn_ballot_w64(j < a.n_valid && !(ts[u] < kSumRescale)) == 0)
+              continue;
             // logits far above the offset: the row's extra offset rises to the tile's maximum
             // (rounded up to bf16), its sum and output so far are scaled by 2^-(increase), and
             // the tile is recomputed

@@ -308,3 +308,23 @@ def test_fused_ops_take_parameters_of_any_fp32_alignment():
             flat[1:].copy_(p.detach().reshape(-1))
             p.data = flat[1:].view_as(p)
         assert torch.equal(m(z.cuda(), mask.cuda()), want)
+
+
+@pytest.mark.parametrize("c,heads,d_hidden,model", [(64, 4, 64, "af3"), (64, 4, 256, "rf3"), (128, 4, 128, "af3"),
+                                                    (256, 4, 256, "chai1"), (128, 8, 192, "af3")])
+@pytest.mark.parametrize("n", [2, 33, 129])
+def test_triangle_attention_does_not_depend_on_what_the_workspace_held(monkeypatch, c, heads, d_hidden, model, n):
+    """Padded queries and attention rows are never written on the generic path: NaN there changes no bit
+    of the others (a NaN sum used to move the softmax offset of its whole tile)."""
+    z, mask = _pair(n, c, [n, max(1, n - 7)], seed=n + c)
+    z, mask = z.cuda(), mask.cuda()
+    got = []
+    for starting in (True, False):
+        m = randomise(factories.triangle_attention(c, heads, starting=starting, model=model, d_hidden=d_hidden),
+                      seed=n).cuda()
+        m.set_backend("hip")
+        for byte in (0, 255):
+            monkeypatch.setattr(kernels, "_workspace", lambda size, device, byte=byte: torch.full(
+                (max(int(size), 256),), byte, dtype=torch.uint8, device=device))
+            got.append(hip_delta(m, z, mask))
+        assert torch.equal(got[-1], got[-2])
