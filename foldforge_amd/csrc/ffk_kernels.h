@@ -377,7 +377,7 @@ void launch_pack(const float* src, bf16* dst, int64_t n, hipStream_t stream);
 int cu_count();
 // Workgroups of a kernel that a CU holds at once (registers and LDS; at least 1, cached): a
 // persistent grid larger than CUs x this runs a second, emptier round.
-int resident_blocks(const void* kernel, int threads, size_t dynamic_lds);
+int resident_blocks(const void* kernel, int threads, size_t dynamic_lds) noexcept;
 
 void launch_layer_norm(const void* x, const float* w, const float* b, void* y, int64_t rows,
                        int cols, float eps, int dtype, hipStream_t stream);

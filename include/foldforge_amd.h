@@ -200,8 +200,8 @@ int32_t ffk_flash_attention_bias(const void* q, const void* k, const void* v_t,
 
 /*
  * Pair (or single) transition: x + squeeze(silu(expand_a(LN(x))) * expand_b(LN(x))) over
- * `rows` token rows of width d. d = 128, factor = 4 runs one fused kernel (the 4x hidden
- * never reaches HBM); other widths (d and factor * d multiples of 64, e.g. the single
+ * `rows` token rows of width d. d = 128, factor = 4 and d = 64, factor = 2 or 4 run one fused
+ * kernel (the hidden rows never reach HBM); other widths (d and factor * d multiples of 64, e.g. the single
  * track's 384 x 4) run LayerNorm -> expand with SwiGLU epilogue -> squeeze + residual,
  * keeping the hidden rows in the workspace.
  * Replaces: engine Transition.forward / `transition`
