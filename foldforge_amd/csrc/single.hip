@@ -1598,7 +1598,7 @@ void launch_row_gemm_t(const RowGemmArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)((a.M + 31) / 32), (unsigned)((otiles + NO - 1) / NO));
   const size_t lds = row_gemm_lds(XSRC, a.K);
   // one group a wave, and workgroups to fill the second place on a CU (with fewer, the form held to 128
-  // VGPRs is up to 3% slower: the output projection of 201 tokens x 384). Eight output tiles a workgroup
+  // VGPRs is up to 2% slower: the output projection of 201 tokens x 384). Eight output tiles a workgroup
   // leave a wave all groups: one only at the 64 channels that just kEpiLinear brings here.
   auto kernel = row_gemm<EPI, XSRC, NO, 2>;
   if constexpr (NO < kGemmWaves || EPI == kEpiLinear)

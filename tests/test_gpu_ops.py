@@ -99,7 +99,7 @@ def test_layer_norm_widths(cols, dtype):
         ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23
         err = ((got.double() - want).abs() / (1 + want.abs())).max().item()
         assert err <= ulp + 2e-6, f"{rows}x{cols} {dtype}: {err:.2e}"
-    if not (cols == 128 and dtype == torch.bfloat16):  # that form refuses unaligned tensors
+    if not (cols == 128 and dtype == torch.bfloat16):  # refused at the C-ABI (FFK_ERR_INVALID), as ever
         flat = torch.randn(33 * cols + 1, generator=g).to(dtype).cuda()
         got = kernels.layer_norm(flat[1:].view(33, cols), w.cuda(), b.cuda(), 1e-5).cpu()
         want = ps.layer_norm(flat[1:].view(33, cols).cpu().double(), w.double(), b.double(), 1e-5)
@@ -131,29 +131,6 @@ def test_trimul_matches_oracle(outgoing, n, lengths):
     _check(got, want, _pairs(mask), f"trimul outgoing={outgoing} n={n}")
     full = hip_forward(m, z.cuda(), mask.cuda()).cpu()
     torch.testing.assert_close(full.float(), (z.float() + got.float()), atol=3e-2, rtol=1e-2)
-
-
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("cols", [32, 64, 128, 192, 256, 384, 512, 768, 1536, 72])
-def test_layer_norm_widths(cols, dtype):
-    # every lane split of the vector kernel and the row kernel's widths (72): one row, a row short
-    # of a workgroup, several passes of the workgroups, and a view 2 or 4 bytes off alignment.
-    # Tolerance: half an ulp of the output type on values up to about 6, and 1e-6 of arithmetic
-    g = torch.Generator().manual_seed(cols)
-    w, b = 1 + 0.1 * torch.randn(cols, generator=g), 0.05 * torch.randn(cols, generator=g)
-    most = 256 * 32 * 64 + 3 if cols <= 64 else 2049
-    for rows in (1, 31, 65, most):
-        x = (torch.randn(rows, cols, generator=g) * 2 + 0.5).to(dtype)
-        got = kernels.layer_norm(x.cuda(), w.cuda(), b.cuda(), 1e-5).cpu()
-        want = ps.layer_norm(x.double(), w.double(), b.double(), 1e-5)
-        ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23
-        err = ((got.double() - want).abs() / (1 + want.abs())).max().item()
-        assert err <= ulp + 2e-6, f"{rows}x{cols} {dtype}: {err:.2e}"
-    if not (cols == 128 and dtype == torch.bfloat16):  # that form refuses unaligned tensors
-        flat = torch.randn(33 * cols + 1, generator=g).to(dtype).cuda()
-        got = kernels.layer_norm(flat[1:].view(33, cols), w.cuda(), b.cuda(), 1e-5).cpu()
-        want = ps.layer_norm(flat[1:].view(33, cols).cpu().double(), w.double(), b.double(), 1e-5)
-        assert ((got.double() - want).abs() / (1 + want.abs())).max().item() <= ulp + 2e-6
 
 
 @pytest.mark.parametrize("outgoing", [True, False])
