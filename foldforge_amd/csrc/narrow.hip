@@ -472,8 +472,8 @@ __global__ __launch_bounds__(64 * kTmoWaves) void triattn_out_rows(TriattnRowsAr
 // stacks; F = 4: the Boltz-2 and RoseTTAFold3 ones and the MSA track):
 //   out = x + (silu(LN(x) W_a^T) * (LN(x) W_b^T)) W_s^T
 // as one streaming kernel, so the hidden rows never reach memory (two row GEMMs wrote and read
-// 128 F bytes of them per 128-byte row: 131072 rows, F = 4: 66 -> 31 us; 589824
-// rows, F = 2: 145 -> 71 us). All three weights sit in LDS
+// 128 F bytes of them per 128-byte row: 131072 rows, F = 4: 66 -> 28 us; 589824
+// rows, F = 2: 145 -> 68 us). All three weights sit in LDS
 // as bf16 (F = 4: 108 KiB, one workgroup of 8 waves per CU; F = 2: 54 KiB, two of 4: a
 // wave needs 190 VGPRs, and three waves per SIMD spilled: 96 instead of 73 us for F = 2). Every
 // wave walks tiles of 32 rows on its own, the next tile's rows loaded while it works: lane
@@ -484,8 +484,9 @@ __global__ __launch_bounds__(64 * kTmoWaves) void triattn_out_rows(TriattnRowsAr
 // channels of x. The weights are the parameters rounded to bf16 and nothing else (a checkpoint in bf16
 // loses nothing on them: the update is 2.3e-3 from the exact one, and was 3.3e-3 with the weights held
 // times log2(e) for the sigmoid's exponent, a multiply per hidden value less and 2% faster). Bound
-// by instruction issue: per tile 160 / 80 MFMAs (5.1 / 2.6 k cycles) and about as long again of
-// SwiGLU, normalisation and rounding.
+// by instruction issue and the waits between dependent ones: per tile 160 / 80 MFMAs (5.1 / 2.6 k cycles)
+// and longer than that of SwiGLU, normalisation and rounding (counters, F = 4 / 2: vector ALU busy 36 /
+// 52%, matrix cores 24 / 29%; of a wave's cycles 34 / 27% waiting for memory or LDS, 30 / 31% to issue).
 template <int F>
 struct __attribute__((aligned(16))) TransitionRowsLds {
   bf16 wa[64 * F * kTmoWs];        // expand_a rows (permuted), k = 64

@@ -111,10 +111,10 @@ __global__ __launch_bounds__(64 * kOpmSplit) void opm_prepare(OpmCountArgs a, co
 // all 64 pairs over half of k', so the weights come from L2 once per workgroup, fetched 8
 // fragments ahead (the first behind phase 1). Phase 3: the two halves are
 // joined through LDS in fp32 and leave as whole 256-byte rows.
-// Measured at 512 MSA rows x 384 tokens (193 GFLOP): 183 us, 1.05 PFLOP/s, against 314 us with
+// Measured at 512 MSA rows x 384 tokens (193 GFLOP): 183 to 186 us, 1.05 PFLOP/s, against 314 us with
 // register-staged 32-row stages (an L2 latency exposed per stage) and the weights read twice per
-// workgroup. Bound by the matrix cores, and by phases 2 and 3, which nothing overlaps: 128 KB
-// of LDS leave one workgroup per CU.
+// workgroup. Bound by the products (matrix cores busy 42% of the time) and by phases 2 and 3, which
+// nothing overlaps: 128 KB of LDS leave one workgroup per CU.
 __global__ __launch_bounds__(512, 2) void opm_contract(OpmContractArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 smem[2 * kOpmStage];  // 128 KB
   const int n = a.n;
